@@ -304,21 +304,22 @@ struct DpCollapser {
   }
 };
 
-// Renumbers the nodes so that those of the top PRT_TOP_LEVELS levels come
-// first, breadth first (the traversal kernels keep these in LDS); the other
-// nodes keep their depth-first order.  Internal child references (>= 0) are
-// remapped; leaf codes (< 0) are unchanged.
+// Renumbers the nodes so that those of the top PRT_WIDE_LEVELS levels (of
+// which the first PRT_TOP_LEVELS have their own count) come first, breadth
+// first (the traversal kernels keep them in LDS); the other nodes keep their
+// depth-first order.  Internal child references (>= 0) are remapped; leaf
+// codes (< 0) are unchanged.
 void number_top_levels(BvhOutput& out) {
   const size_t n = out.nodes.size();
   std::vector<int32_t> top;
   top.push_back(0);
-  for (size_t head = 0, level_end = 1, level = 1; head < top.size() && level < PRT_TOP_LEVELS;) {
+  for (size_t head = 0, level_end = 1, level = 1; head < top.size() && level < PRT_WIDE_LEVELS;) {
     const DevNode& d = out.nodes[(size_t)top[head]];
     for (int i = 0; i < 4; ++i)
       if (d.child[i] > 0 && d.lo_x[i] != std::numeric_limits<float>::infinity()) top.push_back(d.child[i]);
     if (++head == level_end) {
       level_end = top.size();
-      ++level;
+      if (++level == PRT_TOP_LEVELS) out.n_top = (int)top.size();
     }
   }
   std::vector<int32_t> perm(n, -1);  // old index -> new index
@@ -334,7 +335,8 @@ void number_top_levels(BvhOutput& out) {
     nodes[(size_t)perm[i]] = d;
   }
   out.nodes.swap(nodes);
-  out.n_top = (int)top.size();
+  out.n_wide = (int)top.size();
+  if (out.n_top == 0) out.n_top = out.n_wide;  // a tree of fewer levels
 }
 
 }  // namespace

@@ -23,6 +23,7 @@
 #include "prt_device.h"
 #include "prt_internal.h"
 #include "prt_kernels.h"
+#include "prt_stream.h"
 
 // 256-thread blocks per CU of the traversal grids
 #ifndef PRT_TRAV_BLOCKS_PER_CU
@@ -118,6 +119,7 @@ void Workspace::release() {
   counts.release();
   fetch.release();
   ctr.release();
+  pool.release();
   if (h_counts) (void)hipHostFree(h_counts);
   h_counts = nullptr;
   batch_samples = queue_cap = shadow_cap = 0;
@@ -375,6 +377,11 @@ static int scene_build(prt_scene* s, const prt_scene_desc* d) {
     }
   }
   s->n_tris = (int64_t)t_ent.size();
+  // spheres, then uvplanes (of equal hits the lowest entity index wins in any
+  // order, nearer_hit)
+  const size_t n_spheres = std::stable_partition(analytic.begin(), analytic.end(),
+                                                 [&](int32_t i) { return s->h_ents[i].type == PRT_ENTITY_SPHERE; }) -
+                           analytic.begin();
 
   // lights: light-material spheres and uvplanes, power-descending (stable)
   struct L { int32_t ent; double power; };
@@ -476,6 +483,7 @@ static int scene_build(prt_scene* s, const prt_scene_desc* d) {
   P.n_lights = (int32_t)s->h_lights.size();
   P.n_materials = (int32_t)s->h_mats.size();
   P.n_analytic = (int32_t)analytic.size();
+  P.n_spheres = (int32_t)n_spheres;
   P.n_nodes = (int32_t)bo.nodes.size();
   P.smp = 1.0 / smp.samples / (smp.supersamples * smp.supersamples);
   P.sensor_response = smp.sensor_response;
@@ -494,6 +502,7 @@ static int scene_build(prt_scene* s, const prt_scene_desc* d) {
   P.ovf_threads = (int32_t)ovf_threads;
   P.ovf_words = ovf_words;
   P.n_top = P.n_nodes > 0 ? std::min(bo.n_top, PRT_TOP_NODES) : 0;
+  P.n_wide = P.n_nodes > 0 ? std::min(bo.n_wide, PRT_WIDE_NODES) : 0;
   P.n_tris = (int32_t)s->n_tris;
   return PRT_OK;
 }
@@ -677,6 +686,15 @@ extern "C++" int prt::ensure_workspace(prt_scene* s, int64_t batch_samples, bool
   return PRT_OK;
 }
 
+// The part of the workspace a frame of the path kernel needs.
+static int ensure_path_workspace(prt_scene* s, int64_t samples) {
+  Workspace& w = s->pool->ws;
+  int rc;
+  if ((rc = dev_alloc(w.accum, (size_t)samples * 3 * sizeof(uint64_t)))) return rc;
+  if ((rc = dev_alloc(w.counts, 16 * sizeof(uint32_t)))) return rc;
+  return dev_alloc(w.ctr, CTR_COUNT * sizeof(uint64_t));
+}
+
 // Settings of one render call derived from the scene and the options.
 struct RenderSetup {
   Params P;
@@ -716,6 +734,76 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 #define PRT_DEPTHS_PER_SYNC 4
 #endif
 
+// Largest batches of scenes with next-event estimation that the path kernel
+// traces alone (camera samples), and the queue size at which it takes over a
+// batch's tail (rays).  A depth-synchronous depth or a tile-queue iteration
+// costs two traversal launches of 70 to 130 us each, however few its rays; the
+// path kernel pays no launch per depth, but its waves wait for their slowest
+// ray in every trip.  Measured (path kernel / queued engine, ms): mesh box, 0.6 M
+// samples 3.4 / 4.5, 0.8 M 4.4 / 5.2, 1.05 M 5.5 / 5.6 and 6.0 / 6.1 (5k and 82k
+// triangles); glass, where the tile queue drains through long tails, spheres 2.1 M
+// 4.0 / 7.7, spheres and 20k triangles 3.1 M 11.4 / 16.9, field of 400k triangles
+// 2.5 M 5.0 / 5.9.
+#ifndef PRT_PATH_SAMPLES
+#define PRT_PATH_SAMPLES (1 << 20)
+#endif
+#ifndef PRT_PATH_SAMPLES_GLASS
+#define PRT_PATH_SAMPLES_GLASS (3 << 20)
+#endif
+#ifndef PRT_PATH_TAIL
+#define PRT_PATH_TAIL (1 << 16)
+#endif
+
+extern "C++" PathGrid prt::path_grid(int cu_count, int waves, uint64_t n, bool whole_chunks) {
+  PathGrid g;
+  if (waves == 0) waves = n >= (uint64_t)std::max(1, cu_count) * 2 * 256 ? 3 : 2;
+  g.waves = waves;
+  g.blocks = std::max(1, cu_count) * waves;  // one 256-thread block per CU puts one wave on each SIMD
+  const uint64_t per_wave = (n + g.n_waves() - 1) / g.n_waves();
+  if (!whole_chunks && per_wave < 64) {
+    // fewer samples than lanes: every wave gets the same few, so that a wave's
+    // free lanes trace the light samples and glass branches of its own
+    g.unit = g.quota = (uint32_t)std::max<uint64_t>(1, per_wave);
+    g.blocks = (int)std::max<uint64_t>(1, ((n + g.unit - 1) / g.unit + 3) / 4);
+  }
+  if (per_wave >= 64 * 16) g.claim = 4;  // 256 samples per claim atomic
+  return g;
+}
+
+extern "C++" int prt::ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass) {
+  return dev_alloc(b, glass ? (size_t)g.n_waves() * PRT_PATH_POOL * sizeof(PoolRec) : 256);
+}
+
+static int64_t path_samples(const prt_scene* s) { return s->has_glass ? PRT_PATH_SAMPLES_GLASS : PRT_PATH_SAMPLES; }
+
+// One batch's samples (src PATH_FRAME), or the rays of q[k] (PATH_QUEUE),
+// through the path kernel.
+static int run_path(prt_scene* s, PathSource src, const Params& P, const Batch& B, int k, uint64_t* accum,
+                    const PathGrid& g) {
+  Workspace& w = s->pool->ws;
+  hipStream_t st = s->stream;
+  uint32_t* counts = (uint32_t*)w.counts.p;
+  const int64_t ns = B.n_pixels * P.spp;
+  Persist a{};
+  a.next = counts + 12;
+  a.accum = accum;
+  a.pool = (PoolRec*)w.pool.p;
+  a.ctr = (uint64_t*)w.ctr.p;
+  a.n_chunks = (uint32_t)((ns + g.unit - 1) / g.unit);
+  a.claim = g.claim;
+  a.n_scenes = 1;
+  a.quota = g.quota;
+  a.unit = g.unit;
+  a.n_samples = (uint32_t)ns;
+  a.nee = P.nee && P.n_lights > 0;
+  a.batch = B;
+  a.q = ray_queue(w.q[k], w.queue_cap);
+  a.cl = ChunkList{(const uint2*)w.desc[k].p, counts + k};
+  HIPCHK(launch_fill_u32(a.next, g.n_waves() * g.claim, 1, st));
+  HIPCHK(launch_path(src, a, P, g.waves, g.blocks, st));
+  return PRT_OK;
+}
+
 // One batch through the wavefront: generate, then extend / shade / NEE /
 // shadow per path depth until no ray is left.  Sample radiance accumulates
 // into `accum` (fixed point, 3 per camera sample of the batch).  Each
@@ -726,10 +814,24 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 // traced on the scene's second stream as PRT_OVERLAP_SHADOW selects; a NEE
 // that rewrites a shadow queue waits for the shadow launch that read it, and
 // the batch's end waits for every shadow launch.
-static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, Timer& tm,
-                        CallTotals& tot) {
+static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A,
+                        BatchForm form, Timer& tm, CallTotals& tot) {
   Workspace& w = s->pool->ws;
   hipStream_t st = s->stream;
+  const int64_t ns = B.n_pixels * P.spp;
+  if (form == FORM_PATH || (form == FORM_AUTO && ns <= path_samples(s))) {
+    const PathGrid g = path_grid(s->cu_count, 0, (uint64_t)ns, false);
+    int rc = ensure_path_pool(w.pool, g, s->has_glass);
+    if (rc) return rc;
+    HIPCHK(launch_fill_u64(accum, 0ull, 3 * ns, st));
+    if (P.mlt_u) HIPCHK(launch_mlt_gen(P, (uint32_t)ns, ray_queue(w.q[0], w.queue_cap), st));
+    if ((rc = tm.mark(T_OTHER))) return rc;
+    if ((rc = run_path(s, PATH_FRAME, P, B, 0, accum, g))) return rc;
+    if ((rc = tm.mark(T_EXTEND))) return rc;
+    tot.primary_rays += (uint64_t)ns;
+    tot.launches++;
+    return PRT_OK;
+  }
   const int overlap = A.on ? 0 : PRT_OVERLAP_SHADOW;
   hipStream_t st_sh = overlap ? s->stream2 : st;
   uint32_t* counts = (uint32_t*)w.counts.p;
@@ -840,7 +942,6 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
     }
     return PRT_OK;
   };
-  const int64_t ns = B.n_pixels * P.spp;
   const int64_t np = B.n_pixels * P.SS * P.SS;
   HIPCHK(launch_fill_u64(accum, 0ull, 3 * ns, st));
   HIPCHK(launch_fill_u32(counts, 0u, 16, st));
@@ -871,7 +972,17 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
     if ((depth - 1) % PRT_DEPTHS_PER_SYNC == 0) {
       HIPCHK(hipMemcpyAsync(w.h_counts, counts, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
-      if (w.h_counts[4 + cur] == 0) break;
+      const uint32_t rays = w.h_counts[4 + cur];
+      if (rays == 0) break;
+      if (form == FORM_AUTO && rays <= PRT_PATH_TAIL) {
+        // the rest of the batch in one launch
+        const PathGrid g = path_grid(s->cu_count, 2, rays, true);
+        if ((rc = ensure_path_pool(w.pool, g, s->has_glass))) return rc;
+        if ((rc = run_path(s, PATH_QUEUE, P, B, cur, accum, g))) return rc;
+        if ((rc = tm.mark(T_EXTEND))) return rc;
+        tot.launches++;
+        break;
+      }
     }
     const int nxt = cur ^ 1;
     if ((rc = next_fetch(&f))) return rc;
@@ -897,9 +1008,9 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
   return PRT_OK;
 }
 
-extern "C++" int prt::run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, Timer& tm,
-                   CallTotals& tot) {
-  const int rc = run_batch_on(s, P, B, accum, A, tm, tot);
+extern "C++" int prt::run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A,
+                                BatchForm form, Timer& tm, CallTotals& tot) {
+  const int rc = run_batch_on(s, P, B, accum, A, form, tm, tot);
   // a failed batch may have left shadow work queued on the second stream
   if (rc != PRT_OK) (void)hipStreamSynchronize(s->stream2);
   return rc;
@@ -1012,18 +1123,9 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
   if (engine == 3 && !persist_ok)
     return fail(PRT_E_INVALID, "the persistent engine writes float images of at most 2^28 samples, without "
                                "samples_override / batch_pixels");
-  if (engine == 3 || (engine == 0 && !nee_scene && persist_ok && !dumping)) {
-    prt_batch_opts b{};
-    b.seed = o ? o->seed : 0;
-    b.max_depth = o ? o->max_depth : 0;
-    b.persistent = 1;
-    b.trav_blocks_per_cu = 2;  // the compiler's own register budget (fastest without NEE)
-    prt_scene* const one[1] = {s};
-    float* const rgb[1] = {d_rgb};
-    float* const var[1] = {d_var};
-    return prt_render_batch_device(one, 1, &b, rgb, var, stats);
-  }
-  if (engine == 2 || (engine == 0 && s->has_glass && stream_ok && !dumping)) {
+  const int64_t frame = (int64_t)s->P.W * s->P.H * s->P.spp;
+  const bool path = engine == 3 || (engine == 0 && persist_ok && !dumping && (!nee_scene || frame <= path_samples(s)));
+  if (engine == 2 || (engine == 0 && !path && s->has_glass && stream_ok && !dumping)) {
     prt_batch_opts b{};
     b.seed = o ? o->seed : 0;
     b.max_depth = o ? o->max_depth : 0;
@@ -1032,7 +1134,6 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
     // samples in flight: a whole frame of up to 2^21, else the batched
     // renderer's automatic size (the most, up to 2^24, whose workspace fits
     // its share of the device memory)
-    const int64_t frame = (int64_t)s->P.W * s->P.H * s->P.spp;
     b.tile_samples = 4096;
     b.inflight_tiles = frame <= ((int64_t)1 << 21) ? (int32_t)std::max<int64_t>(1, (frame + 4095) / 4096) : 0;
     prt_scene* const one[1] = {s};
@@ -1043,13 +1144,21 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
   RenderSetup R;
   int rc;
   if ((rc = setup_render(s, o, R))) return rc;
-  if ((rc = ensure_workspace(s, R.bp * R.P.spp, false))) return rc;
+  if (path) {
+    R.bp = R.n_pix;  // one launch, which needs no queues
+    if ((rc = ensure_path_workspace(s, R.n_pix * R.P.spp))) return rc;
+  } else if ((rc = ensure_workspace(s, R.bp * R.P.spp, false))) {
+    return rc;
+  }
   hipStream_t st = s->stream;
   HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_COUNT, st));
   Timer tm;
-  if ((rc = tm.begin(o && o->timing != 0, st, &s->timer_events))) return rc;
+  if ((rc = tm.begin(path || (o && o->timing != 0), st, &s->timer_events))) return rc;
   CallTotals tot;
   Adjoint none{};
+  // engine 1 and renders with progress images or a batch size are asked to be
+  // depth-synchronous
+  const BatchForm form = path ? FORM_PATH : engine == 1 || dumping || (o && o->batch_pixels > 0) ? FORM_WAVEFRONT : FORM_AUTO;
   const int f64 = o && o->image_f64;
   if (dumping) {
     // pixels not yet rendered read as 0 in the progress images
@@ -1062,7 +1171,7 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
   }
   for (int64_t pb = 0; pb < R.n_pix; pb += R.bp) {
     Batch B{pb, std::min(R.bp, R.n_pix - pb)};
-    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum.p, none, tm, tot))) return rc;
+    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum.p, none, form, tm, tot))) return rc;
     HIPCHK(launch_resolve(R.P, B, (const uint64_t*)s->pool->ws.accum.p, d_rgb, d_var, f64, st));
     if ((rc = tm.mark(T_OTHER))) return rc;
     const int64_t done = pb + B.n_pixels;
@@ -1224,8 +1333,8 @@ int prt_adjoint_device(prt_scene* s, const prt_render_opts* o, const float* d_di
   A.scale = R.P.sensor_response * R.P.smp;
   for (int64_t pb = 0; pb < R.n_pix; pb += R.bp) {
     Batch B{pb, std::min(R.bp, R.n_pix - pb)};
-    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum2.p, none, tm, tot))) return rc;
-    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum.p, A, tm, tot))) return rc;
+    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum2.p, none, FORM_AUTO, tm, tot))) return rc;
+    if ((rc = run_batch(s, R.P, B, (uint64_t*)s->pool->ws.accum.p, A, FORM_WAVEFRONT, tm, tot))) return rc;
     HIPCHK(launch_count_mismatch((const uint64_t*)s->pool->ws.accum.p, (const uint64_t*)s->pool->ws.accum2.p,
                                  3 * B.n_pixels * R.P.spp, (uint64_t*)s->pool->ws.ctr.p, st));
   }

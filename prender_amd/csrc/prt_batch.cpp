@@ -32,9 +32,9 @@ struct StreamWorkspace {
   DevBuf q[2][RAYQ_COLS], hit_t, hit_id, sq[SHADOWQ_COLS];
   DevBuf accum, ctr, ctl, slot_info, live, free_list, new_tiles;
   DevBuf scenes, tiles, outs, ovf, runs, nruns, desc[2], sh_desc, fetch;
-  // persistent engine: per-sample accumulators, pending glass segments per
-  // thread, the chunk / sample / pixel bases of the scenes and the claim counter
-  DevBuf p_accum, p_pend, p_bases;
+  // persistent form: per-sample accumulators, the chunk / sample / pixel
+  // bases of the scenes and the claim counter
+  DevBuf p_accum, p_bases;
   int64_t ovf_threads = 0;
   int ovf_words = 0;
   StreamCtl* h_ctl = nullptr;  // pinned, two copies (double-buffered status reads)
@@ -44,7 +44,7 @@ struct StreamWorkspace {
     for (auto& b : sq) b.release();
     DevBuf* all[] = {&hit_t,  &hit_id, &accum, &ctr,     &ctl,     &slot_info, &live,    &free_list, &new_tiles,
                      &scenes, &tiles,  &outs,  &ovf,     &runs,    &nruns,     &desc[0], &desc[1],   &sh_desc,
-                     &fetch,  &p_accum, &p_pend, &p_bases};
+                     &fetch,  &p_accum, &p_bases};
     for (DevBuf* b : all) b->release();
     if (h_ctl) (void)hipHostFree(h_ctl);
     h_ctl = nullptr;
@@ -102,7 +102,7 @@ struct BatchConfig {
   int max_vertices = 128;
   bool timing = false;
   int persistent = 0;  // 0 tile queue, 1 one persistent launch, 2 split by NEE
-  int persist_blocks_per_cu = 2;
+  int persist_waves = 0;  // 0: path_grid's choice
   uint64_t seed = 0;
 };
 
@@ -138,14 +138,14 @@ int resolve_config(prt_scene* const* scenes, int n, const prt_batch_opts* o, Bat
   c.seed = opts.seed;
   if (opts.persistent < 0 || opts.persistent > 2) return fail(PRT_E_INVALID, "persistent must be 0, 1 or 2");
   c.persistent = opts.persistent;
-  // the persistent kernel's register budget (waves per SIMD): persist_waves,
-  // else in mode 1 trav_blocks_per_cu (mode 2 sizes the tile-queue part's
-  // grid with it), else the compiler's own budget (2)
+  // the path kernel's register budget (waves per SIMD): persist_waves, else in
+  // mode 1 trav_blocks_per_cu (mode 2 sizes the tile-queue part's grid with
+  // it), else path_grid's choice
   if (opts.persist_waves != 0 && (opts.persist_waves < 2 || opts.persist_waves > 4))
     return fail(PRT_E_INVALID, "persist_waves must be 0, 2, 3 or 4");
-  c.persist_blocks_per_cu = opts.persist_waves > 0                               ? opts.persist_waves
-                            : (opts.persistent == 1 && opts.trav_blocks_per_cu > 0) ? opts.trav_blocks_per_cu
-                                                                                   : 2;
+  c.persist_waves = opts.persist_waves;
+  if (c.persist_waves == 0 && opts.persistent == 1 && opts.trav_blocks_per_cu > 0)
+    c.persist_waves = std::min(4, std::max(2, opts.trav_blocks_per_cu));
   if (c.persistent && opts.tile_stride > 1) return fail(PRT_E_INVALID, "the persistent engine renders every sample");
   return PRT_OK;
 }
@@ -554,17 +554,6 @@ int run_stream(prt_scene* const* scenes, int n, const BatchConfig& c, float* con
   return PRT_OK;
 }
 
-// Chunks of 64 samples a wave claims at a time in the persistent engine
-// (256 samples: one claim atomic per 256 camera samples)
-#ifndef PRT_PERSIST_CLAIM
-#define PRT_PERSIST_CLAIM 4
-#endif
-// 32: the 2-wave persistent kernel keeps 32 stack entries in LDS (two
-// 66-KB blocks per CU; fewer spills: cfg4's persistent half 215 -> 212 ms);
-// 0: the batch's stack_lds decides between 8 and 16
-#ifndef PRT_PERSIST_STACK
-#define PRT_PERSIST_STACK 32
-#endif
 constexpr uint64_t kMaxPersistSamples = (uint64_t)1 << 28;
 
 // One batched render as a single persistent launch (prt_persist.hip), then
@@ -600,19 +589,11 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   if (samples > kMaxPersistSamples)
     return fail(PRT_E_INVALID, "the persistent engine takes at most 2^28 camera samples per batch (" +
                                    std::to_string(samples) + " asked)");
-  // one 256-thread block per CU puts one wave on each SIMD: blocks per CU
-  // picks the register budget (2 = the compiler's own, about 230 VGPRs;
-  // 3 and 4 spill part of the state), capped by what fits
-  const int waves = std::min(4, std::max(2, c.persist_blocks_per_cu));
-  // LDS stack of the persistent kernel: PRT_PERSIST_STACK when set, else from
-  // the batch's stack_lds (8, or 16 for 12..32)
-  const int stack = PRT_PERSIST_STACK == 32 && waves <= 2 ? 32 : (c.stack_lds <= 8 ? 8 : 16);
-  int occ = 0;
-  HIPCHK(persist_blocks_per_cu(stack, waves, &occ));
   const int cu = std::max(1, lead->cu_count);
-  const int per_cu = std::max(1, std::min(occ, waves));
-  const int blocks = cu * per_cu;
-  const int64_t threads = (int64_t)blocks * 256;
+  const PathGrid grid = path_grid(cu, c.persist_waves, samples, true);
+  const int64_t threads = (int64_t)grid.blocks * 256;
+  bool glass = false;
+  for (int i = 0; i < n; ++i) glass |= scenes[i]->has_glass;
 
   if (!lead->pool->sws) lead->pool->sws = new (std::nothrow) StreamWorkspace();
   if (!lead->pool->sws) return fail(PRT_E_NOMEM, "out of host memory");
@@ -630,7 +611,7 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   if ((rc = dev_alloc(w.scenes, (size_t)n * sizeof(Params)))) return rc;
   if ((rc = dev_alloc(w.outs, (size_t)n * 2 * sizeof(float*)))) return rc;
   if ((rc = dev_alloc(w.p_accum, (size_t)samples * 3 * sizeof(uint64_t)))) return rc;
-  if ((rc = dev_alloc(w.p_pend, (size_t)threads * PRT_PEND_DEPTH * sizeof(PendRec)))) return rc;
+  if ((rc = ensure_path_pool(lead->pool->ws.pool, grid, glass))) return rc;
   const size_t bases_bytes = (size_t)(n + 1) * (sizeof(uint32_t) + sizeof(uint64_t) + sizeof(int64_t)) + 64;
   if ((rc = dev_alloc(w.p_bases, bases_bytes))) return rc;
   hipStream_t s = lead->stream;
@@ -669,13 +650,16 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   P.sample_base = d_sample;
   P.next = d_next;
   P.accum = (uint64_t*)w.p_accum.p;
-  P.pend = (PendRec*)w.p_pend.p;
+  P.pool = (PoolRec*)lead->pool->ws.pool.p;
   P.ctr = (uint64_t*)w.ctr.p;
   P.out_rgb = (float* const*)w.outs.p;
   P.out_var = (float* const*)w.outs.p + n;
   P.n_chunks = (uint32_t)chunks;
-  P.claim = PRT_PERSIST_CLAIM;
+  P.claim = grid.claim;
+  P.quota = grid.quota;
+  P.unit = 64;
   P.n_scenes = n;
+  for (int i = 0; i < n; ++i) P.nee |= scenes[i]->P.nee && scenes[i]->P.n_lights > 0;
 
   ScopedEvent e0, e1, e2;
   HIPCHK(hipEventCreate(&e0.e));
@@ -683,9 +667,10 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   HIPCHK(hipEventCreate(&e2.e));
   // counters and the claim counter start at zero (fill kernels, not memsets)
   HIPCHK(launch_fill_u64(P.ctr, 0ull, CTR_COUNT, s));
-  HIPCHK(launch_fill_u32(d_next, 0u, 1, s));
+  HIPCHK(launch_fill_u32(d_next, grid.n_waves() * grid.claim, 1, s));
+  HIPCHK(launch_fill_u64(P.accum, 0ull, 3 * (int64_t)samples, s));
   HIPCHK(hipEventRecord(e0.e, s));
-  HIPCHK(launch_persist(P, stack, waves, blocks, s));
+  HIPCHK(launch_path(PATH_BATCH, P, params[0], grid.waves, grid.blocks, s));
   HIPCHK(hipEventRecord(e1.e, s));
   HIPCHK(launch_persist_resolve(P, pixels, d_pixel, s));
   HIPCHK(hipEventRecord(e2.e, s));
@@ -698,10 +683,10 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   if (ctrh[CTR_DROP] != 0)
     return fail(PRT_E_INTERNAL, "persistent render: " + std::to_string(ctrh[CTR_DROP]) + " glass segments dropped");
   // every sample's camera ray and every emitted child was traced exactly once
-  if (ctrh[CTR_QUEUED] != samples || ctrh[CTR_TRACED] != ctrh[CTR_QUEUED] + ctrh[CTR_EXT])
-    return fail(PRT_E_INTERNAL, "persistent render traced " + std::to_string(ctrh[CTR_TRACED]) + " segments for " +
-                                    std::to_string(ctrh[CTR_QUEUED]) + " samples (of " + std::to_string(samples) +
-                                    ") and " + std::to_string(ctrh[CTR_EXT]) + " children");
+  if (ctrh[CTR_QUEUED] != samples + ctrh[CTR_EXT] || ctrh[CTR_TRACED] != ctrh[CTR_QUEUED])
+    return fail(PRT_E_INTERNAL, "persistent render traced " + std::to_string(ctrh[CTR_TRACED]) + " of " +
+                                    std::to_string(ctrh[CTR_QUEUED]) + " segments of " + std::to_string(samples) +
+                                    " samples and " + std::to_string(ctrh[CTR_EXT]) + " children");
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->node_visits = ctrh[CTR_NODES] + ctrh[CTR_SNODES];
@@ -711,7 +696,7 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
     stats->pickup_hits = ctrh[CTR_PICKUP];
     stats->truncated_paths = ctrh[CTR_TRUNC];
     stats->camera_samples = samples;
-    stats->primary_rays = ctrh[CTR_QUEUED];  // one camera ray per sample in this engine
+    stats->primary_rays = samples;  // one camera ray per sample in this engine
     stats->extension_rays = ctrh[CTR_EXT];
     stats->shadow_rays = ctrh[CTR_SHADOW];
     stats->ms_total = ms_render + ms_resolve;

@@ -32,6 +32,9 @@ static_assert(PRT_MAX_LEAF >= 1 && PRT_MAX_LEAF <= 16, "leaf size must fit the 4
 #ifndef PRT_TOP_NODES
 #define PRT_TOP_NODES 21  // 1 + 4 + 16
 #endif
+// the path kernel keeps five levels (its two blocks per CU leave the LDS)
+#define PRT_WIDE_LEVELS 5
+#define PRT_WIDE_NODES 341  // 1 + 4 + 16 + 64 + 256
 // smallest LDS stack depth any kernel variant uses (sizes the overflow area)
 #define PRT_STACK_LDS_MIN 8
 #define PRT_STACK_TOTAL 128
@@ -107,7 +110,7 @@ struct Params {
   const float* tri_alb_rr;   // albedo for Russian-roulette probabilities (null: tri_alb)
   const DevEntity* ents;
   const DevMaterial* mats;
-  const int32_t* analytic;   // entity indices of spheres / uvplanes
+  const int32_t* analytic;   // entity indices of spheres, then of uvplanes
   const int32_t* lights;     // light entity indices, power-descending
   uint32_t* stack_ovf;       // per-thread traversal stack overflow
   int32_t ovf_threads;
@@ -124,6 +127,8 @@ struct Params {
   int32_t mlt_depths;
   int32_t ovf_words;    // words of one thread's stack overflow area
   int32_t n_top;        // nodes 0..n_top-1 are the top PRT_TOP_LEVELS BVH levels (kept in LDS)
+  int32_t n_spheres;    // the first n_spheres of analytic are spheres, the others uvplanes
+  int32_t n_wide;       // nodes 0..n_wide-1 are the top PRT_WIDE_LEVELS levels (kept in LDS by the path kernel)
 };
 // camera words of a Metropolis proposal: pixel x, y, sub-pixel x, y, tent
 // filter x, y, two spare (render.h:262-300)

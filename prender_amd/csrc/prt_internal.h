@@ -90,6 +90,7 @@ struct Workspace {
   DevBuf counts;              // uint32 [16]: chunks of q0, q1, sq, sq2 at 0..3, entries at 4..7
   DevBuf fetch;               // uint32 claim counters, PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE per launch
   DevBuf ctr;                 // uint64 [CTR_COUNT]
+  DevBuf pool;                // path kernel: waiting glass segments, PoolRec [waves][PRT_PATH_POOL]
   uint32_t* h_counts = nullptr;
   void release();
 };
@@ -254,10 +255,22 @@ struct CallTotals {
 void fill_stats(prt_stats* st, const uint64_t* c);
 // Sizes the scene's workspace for batches of `batch_samples` camera samples.
 int ensure_workspace(prt_scene* s, int64_t batch_samples, bool two_accum);
-// One batch of camera samples (or Metropolis proposals, when P.mlt_u is set)
-// through the wavefront; sample radiance accumulates into accum (fixed point).
-int run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, Timer& tm,
-              CallTotals& tot);
+// Grid and claim sizes of a path-kernel launch over n samples (rays) cut into
+// chunks of at most 64, with the pool sized for it.
+struct PathGrid {
+  int waves = 2, blocks = 0;
+  uint32_t unit = 64, claim = 1, quota = 64;
+  uint32_t n_waves() const { return (uint32_t)blocks * 4u; }
+};
+PathGrid path_grid(int cu_count, int waves, uint64_t n, bool whole_chunks);
+int ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass);
+// How run_batch may trace a batch: wavefront only, the path kernel where the
+// batch or its tail is small, or the path kernel alone.
+enum BatchForm { FORM_WAVEFRONT = 0, FORM_AUTO = 1, FORM_PATH = 2 };
+// One batch of camera samples (or Metropolis proposals, when P.mlt_u is set);
+// sample radiance accumulates into accum (fixed point).
+int run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, BatchForm form,
+              Timer& tm, CallTotals& tot);
 
 }  // namespace prt
 

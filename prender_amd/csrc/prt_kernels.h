@@ -25,18 +25,19 @@ enum {
   CTR_COUNT = 15
 };
 
-// A path segment a lane of the persistent renderer keeps for later: a glass
-// vertex at depth <= 2 emits two children; the lane follows the first and
-// keeps the second here.  A lane's path is a binary tree split at depths 0,
-// 1 and 2 walked depth first, so at most one kept segment per split depth.
-struct PendRec {
+// A path segment waiting in a wave's pool (path kernel): a glass vertex at
+// depth <= 2 emits two children; the lane follows the first, and the second is
+// taken by an idle lane of its wave.  A wave starts new samples only while its
+// pool is empty, and a segment has at most 8 leaves below it (splits at depths
+// 0, 1 and 2), so of the 64 * 8 segments a wave can hold at a time at most
+// 64 * 7 wait.
+struct PoolRec {
   double o[3], d[3];
-  float t[3], p[3], n[3];
-  uint32_t meta;
-  uint32_t pad_[2];
+  float t[3], p[3];
+  uint32_t meta, slot;
 };
-static_assert(sizeof(PendRec) == 96, "pending segment record must be 96 bytes");
-#define PRT_PEND_DEPTH 3
+static_assert(sizeof(PoolRec) == 80, "pool record must be 80 bytes");
+#define PRT_PATH_POOL 448u
 
 struct prt_ray_dev {
   double org[3];

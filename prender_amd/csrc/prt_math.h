@@ -132,6 +132,17 @@ __device__ __forceinline__ void sincos_2pi(double u, double& s, double& c) {
   c = (k == 0) ? cy : (k == 1) ? -sy : (k == 2) ? -cy : sy;
 }
 
+// sphere_t without branches
+__device__ __forceinline__ bool sphere_root(d3 center, double radius, d3 o, d3 d, double& t) {
+  const d3 p_o = center - o;
+  const double b = dot(p_o, d);
+  const double D4 = b * b - dot(p_o, p_o) + radius * radius;
+  const double s = sqrt(D4);
+  const double t1 = b - s, t2 = b + s;
+  t = (t1 > PS_EPS) ? t1 : t2;
+  return !(D4 < 0.0) & !((t1 < PS_EPS) & (t2 < PS_EPS));
+}
+
 // Sphere::intersect, sphere.h:68-87
 __device__ __forceinline__ bool sphere_t(const DevEntity& e, d3 o, d3 d, double& t) {
   const d3 p_o = ld3(e.p0) - o;
@@ -146,7 +157,8 @@ __device__ __forceinline__ bool sphere_t(const DevEntity& e, d3 o, d3 d, double&
 }
 
 // UVPlane::intersect over Plane::intersect, plane.h:86-110, 220-240
-__device__ __forceinline__ bool uvplane_t(const DevEntity& e, d3 o, d3 d, double& t) {
+template <class Entity>
+__device__ __forceinline__ bool uvplane_t(const Entity& e, d3 o, d3 d, double& t) {
   d3 n2 = ld3(e.normal);
   if (e.ninv < 0) n2 = n2 * -1.0;
   const double dd = dot(d, n2);

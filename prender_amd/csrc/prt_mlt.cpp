@@ -126,7 +126,7 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
     HIPCHK(launch_mlt_mutate(CH, 0, first, n, 0u, m.p_large, st));
     Params Pb = P;
     mlt_key(opts.seed, 1, batch, Pb.key0, Pb.key1);
-    if ((rc = run_batch(s, Pb, Batch{0, n}, accum, none, tm, tot))) return rc;
+    if ((rc = run_batch(s, Pb, Batch{0, n}, accum, none, FORM_AUTO, tm, tot))) return rc;
     HIPCHK(launch_mlt_seed_record(accum, CH.pix_new, first, n, SD, st));
   }
   HIPCHK(launch_mlt_scan(SD, st));
@@ -144,7 +144,7 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
       HIPCHK(launch_mlt_mutate(CH, 1, 0u, C, (uint32_t)it, m.p_large, st));
       Params Pi = P;
       mlt_key(opts.seed, 2, (uint64_t)it, Pi.key0, Pi.key1);
-      if ((rc = run_batch(s, Pi, Batch{0, C}, accum, none, tm, tot))) return rc;
+      if ((rc = run_batch(s, Pi, Batch{0, C}, accum, none, FORM_AUTO, tm, tot))) return rc;
       HIPCHK(launch_mlt_step(CH, accum, (uint32_t)it, m.p_large, b, weight, inv_m, ctr, st));
     }
     steps_run = m.steps;
@@ -253,7 +253,7 @@ static int render_erpt(prt_scene* s, const prt_erpt_opts* o, void* d_out, int as
     Pb.mlt_pix = pix;
     Pb.mlt_flags = flags;
     mlt_key(opts.seed, 7, launch++, Pb.key0, Pb.key1);
-    return run_batch(s, Pb, Batch{0, n}, accum, none, tm, tot);
+    return run_batch(s, Pb, Batch{0, n}, accum, none, FORM_AUTO, tm, tot);
   };
   auto t0 = std::chrono::steady_clock::now();
 

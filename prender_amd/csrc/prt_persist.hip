@@ -1,19 +1,37 @@
-// prt_persist.hip — the persistent form of the batched renderer: one kernel
-// launch renders every camera sample of every scene of a batch.
+// prt_persist.hip — the path kernel: one launch follows every camera sample it
+// is given along its whole path, with no ray queue and no launch per depth.
 //
-// Waves claim ranges of 64-sample chunks from one shared counter over the
-// batch's chunk list (scene-major, prt_stream.h Persist) and keep each of
-// their 64 lanes on one camera sample at a time.  Per loop trip a lane
-// advances its sample's path by one segment: next-event estimation of the
-// segment's origin vertex when the segment carries the NEE flag (three light
-// samples, each with its any-hit shadow ray), the segment's closest hit, and
-// one radiance() vertex (prt_shade.h), whose first child becomes the lane's
-// next segment and whose second child (glass at depth <= 2) waits on the
-// lane's pending stack.  When a path has no segment left the lane writes the
-// sample's fixed-point sum to the sample's accumulator and takes the next
-// sample.  Nothing goes through a ray queue, there is no launch per depth,
-// and waves never wait for each other: a wave exits when the counter is past
-// the last chunk and its lanes have finished.
+// It renders the samples of a batch of scenes (the batched renderer's
+// persistent form and frames without light sampling), of one small frame or
+// Metropolis step (a depth-synchronous batch would pay two traversal launches
+// per depth, each as long as its slowest ray), or the last rays of a
+// depth-synchronous batch, from their queue.
+//
+// A wave keeps its 64 lanes on one path segment each.  Per trip: the light
+// samples of the segments' origin vertices (three per diffuse vertex) and the
+// segments' closest hits, then one radiance() vertex per segment (prt_shade.h),
+// whose first child becomes the lane's next segment.  A light sample belongs
+// to no lane: the three samples of every vertex are numbered through the wave
+// and dealt out, first to the lanes without a segment (whose any-hit rays then
+// run in the same traversal as the other lanes' closest hits), the rest 64 at
+// a time, so a wave with few paths traces all rays of a vertex side by side and
+// a full one wastes no lane on a vertex without light samples.  The second
+// child of a glass vertex goes to the wave's pool, from which idle lanes take
+// segments before they start new samples: a path's branches run side by side
+// instead of one after the other.
+//
+// What bounds it: latency.  A trip of a wave is a traversal as long as its
+// slowest ray (38,000 cycles with 7 paths of a 82k-triangle scene per wave,
+// 29,000 per 64 rays of a full one), 6,000 to 10,000 cycles of dependent FP64
+// chains in the vertices and 2,700 in 64 light samples.  So rays of one vertex
+// run side by side, few samples are spread over all waves, records that
+// every lane reads come from LDS, and scenes without light sampling have an
+// instance without it (174 instead of 228 VGPRs).  Measured against one lane
+// per sample that walks its glass tree and its light samples one after the
+// other, and against depth-synchronous batches: spheres 32x24 x 8 spp 834 ->
+// 175 us, 320x240 x 16 spp 1636 -> 951 us; mesh box 128x128 x 8 spp 2707 -> 946
+// us; glass with light sampling 201x151 x 27 spp 6060 -> 3036 us; Metropolis
+// steps of 15,360 chains 2.5 -> 0.43 ms.
 //
 // A wave works on one scene at a time, so the scene's parameters are
 // wave-uniform scalar loads: a lane starts a sample of another scene only
@@ -24,7 +42,8 @@
 // stores them, contributions added in 32.32 fixed point), a sample's random
 // numbers depend only on (pixel, sample, depth, branch), and integer sums do
 // not depend on order, so every image equals the per-scene render bit for
-// bit.  k_persist_resolve then folds each pixel's samples (fold_pixel).
+// bit.  A lane sums its segments' light in LDS and adds it to the sample's
+// accumulator (cleared before the launch) when its chain of segments ends.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -40,6 +59,19 @@ __device__ __forceinline__ uint64_t fix_of(double v) {
   return v > 0.0 ? (uint64_t)(v * PRT_FIX_ONE + 0.5) : 0ull;
 }
 
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ d3 shfl_d3(d3 v, int src) {
+  return mk(__shfl(v.x, src, 64), __shfl(v.y, src, 64), __shfl(v.z, src, 64));
+}
+
+// materials a frame's blocks keep in LDS
+#define PRT_PATH_MATERIALS 16
+
 // Scene owning chunk c (c wave-uniform): the last s with chunk_base[s] <= c.
 __device__ __forceinline__ int32_t scene_of_chunk(const Persist& st, uint32_t c) {
   int32_t lo = 0, hi = st.n_scenes;
@@ -51,88 +83,176 @@ __device__ __forceinline__ int32_t scene_of_chunk(const Persist& st, uint32_t c)
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// WAVES: waves per SIMD the registers are budgeted for (2: the compiler's
-// own choice, about 230 VGPRs; 3 and 4 spill some state to scratch)
-template <int NL, int WAVES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_persist(Persist st) {
-  PRT_DECLARE_STACK_N(S, st.scenes[0], NL, 0);
-  // the top-level node copy serves a batch of one scene only
-  PRT_TOP_CACHE(S, st.scenes[0].nodes, st.n_scenes == 1 ? st.scenes[0].n_top : 0);
-  const uint64_t below = (1ull << lane_id()) - 1ull;
-  PendRec* pend = st.pend + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * PRT_PEND_DEPTH;
+// SRC: PathSource.  NEE: some scene samples lights.  NL: LDS stack entries;
+// NTOP: BVH nodes kept in LDS; WAVES: waves per SIMD the registers are budgeted
+// for.
+template <int SRC, bool NEE, int NL, int NTOP, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_path(Persist st,
+                                                                                                 Params P1) {
+  const Params& P0 = SRC == PATH_BATCH ? st.scenes[0] : P1;
+  PRT_DECLARE_STACK_N(S, P0, NL, 0);
+  // the top-level node copy serves one scene only
+  PRT_TOP_CACHE_N(S, P0.nodes, SRC != PATH_BATCH || st.n_scenes == 1 ? min(P0.n_wide, NTOP) : 0, NTOP);
+  __shared__ uint64_t s_acc[3][256];  // light of each lane's chain so far
+  __shared__ uint32_t s_pool[4];      // pool records of each wave
+  __shared__ uint8_t s_map[256];      // lanes of each wave that hold a vertex to light, by rank
+  // one scene's analytic entities and materials
+  constexpr bool kCache = SRC != PATH_BATCH;
+  __shared__ AnalyticSlot s_ana[kCache ? PRT_LDS_ANALYTIC : 1];
+  __shared__ DevMaterial s_mats[kCache ? PRT_PATH_MATERIALS : 1];
+  const AnalyticSlot* slots = nullptr;
+  const DevMaterial* lds_mats = nullptr;
+  if (kCache) {
+    if (P1.n_analytic <= PRT_LDS_ANALYTIC) {
+      if ((int)threadIdx.x < P1.n_analytic) {
+        AnalyticSlot& a = s_ana[threadIdx.x];
+        a.ei = P1.analytic[threadIdx.x];
+        const DevEntity& e = P1.ents[a.ei];
+        for (int j = 0; j < 3; ++j) {
+          a.p0[j] = e.p0[j];
+          a.u_axis[j] = e.u_axis[j];
+          a.v_axis[j] = e.v_axis[j];
+          a.normal[j] = e.normal[j];
+        }
+        a.radius = e.radius;
+        a.u_len = e.u_len;
+        a.v_len = e.v_len;
+        a.ninv = e.ninv;
+      }
+      slots = s_ana;
+    }
+    if (P1.n_materials <= PRT_PATH_MATERIALS) {
+      if ((int)threadIdx.x < P1.n_materials) s_mats[threadIdx.x] = P1.mats[threadIdx.x];
+      lds_mats = s_mats;
+    }
+    __syncthreads();
+  }
+  const uint32_t lane = lane_id(), wib = threadIdx.x >> 6;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + wib));
+  const uint64_t below = (1ull << lane) - 1ull;
+  const uint32_t wbase = wib * 64u;
+  for (int c = 0; c < 3; ++c) s_acc[c][threadIdx.x] = 0ull;
+  if (lane == 0) s_pool[wib] = 0u;
+  wave_fence();
+  PoolRec* pool = st.pool + (size_t)wave * PRT_PATH_POOL;
   TravStats tc{0, 0, 0}, tsh{0, 0, 0};
   uint32_t n_prim = 0, n_traced = 0, n_shadow = 0, truncated = 0, n_ext = 0, pickups = 0, dropped = 0;
 
-  // wave-uniform work cursor: claimed chunks [cb, ce), next sample co of
-  // chunk cb, which belongs to scene cs (-1: not yet looked up) and holds cn
-  // samples; the wave's current scene
-  uint32_t cb = 0, ce = 0, co = 0, cn = 0;
-  int32_t cs = -1, scene = -1;
-  bool claims_left = true;
+  // wave-uniform work cursor: chunks [cb, ce), next sample co of chunk cb,
+  // which belongs to scene cs (-1: not yet looked up) and holds cn samples; the
+  // wave's current scene.  The first chunks are the wave's own (st.next starts
+  // past them): one atomic per wave at the start would serialise the grid.
+  const uint32_t n_chunks = SRC == PATH_QUEUE ? *st.cl.n : st.n_chunks;
+  uint32_t cb = min(wave * st.claim, n_chunks), ce = min(cb + st.claim, n_chunks), co = 0, cn = 0;
+  int32_t cs = -1, scene = SRC == PATH_BATCH ? -1 : 0;
+  bool claims_left = n_chunks > gridDim.x * (blockDim.x >> 6) * st.claim;
   UniformLight U{};
   bool one_light = false;
+  if (SRC != PATH_BATCH) {
+    one_light = NEE && P1.n_lights == 1;
+    if (one_light) U = uniform_light(P1, P1.lights[0]);
+  }
 
-  // the lane's sample and current segment
+  // the lane's segment
   bool act = false;
   d3 o = mk(0.0, 0.0, 0.0), d = o;
   float tr[3] = {1.0f, 1.0f, 1.0f}, pw[3] = {0.0f, 0.0f, 0.0f}, nr[3] = {0.0f, 0.0f, 0.0f};
-  uint32_t meta = 0, k = 0;
-  int64_t pixel = 0;
-  uint64_t gs = 0;
-  uint64_t acc[3] = {0ull, 0ull, 0ull};
-  int npend = 0;
+  uint32_t meta = 0, slot = 0;  // slot: sample of the scene (frame, queue: of the batch)
 
   while (true) {
-    // ---- idle lanes take the next samples of the wave's scene
+    // ---- idle lanes take the wave's waiting segments, then new samples
     uint64_t need = __ballot(!act);
-    while (need) {
+    const uint32_t waiting = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(s_pool[wib], PRT_PATH_POOL));
+    uint32_t left = waiting;
+    if (need && waiting) {
+      const uint32_t take = min((uint32_t)__popcll(need), waiting), rank = (uint32_t)__popcll(need & below);
+      if (!act && rank < take) {
+        const PoolRec& r = pool[waiting - 1u - rank];
+        o = mk(r.o[0], r.o[1], r.o[2]);
+        d = mk(r.d[0], r.d[1], r.d[2]);
+        for (int j = 0; j < 3; ++j) {
+          tr[j] = r.t[j];
+          pw[j] = r.p[j];
+        }
+        meta = r.meta;
+        slot = r.slot;
+        act = true;
+      }
+      left = waiting - take;
+      if (lane == 0) s_pool[wib] = left;
+      wave_fence();
+      need = __ballot(!act);
+    }
+    uint32_t room = 64u - (uint32_t)__popcll(need);  // segments held
+    room = left == 0u && st.quota > room ? st.quota - room : 0u;
+    while (need && room) {
       if (cb >= ce) {
         if (!claims_left) break;
         uint32_t c0 = 0;
-        if (lane_id() == 0) c0 = atomicAdd(st.next, st.claim);
+        if (lane == 0) c0 = atomicAdd(st.next, st.claim);
         c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)__shfl((int)c0, 0, 64));
-        if (c0 >= st.n_chunks) {
+        if (c0 >= n_chunks) {
           claims_left = false;
           break;
         }
         cb = c0;
-        ce = min(c0 + st.claim, st.n_chunks);
+        ce = min(c0 + st.claim, n_chunks);
         co = 0;
         cs = -1;
       }
       if (cs < 0) {
-        cs = scene_of_chunk(st, cb);
-        const uint64_t first = (uint64_t)(cb - st.chunk_base[cs]) * 64u;
-        const uint64_t n_s = st.sample_base[cs + 1] - st.sample_base[cs];
-        cn = (uint32_t)__builtin_amdgcn_readfirstlane((int)(n_s - first < 64u ? n_s - first : 64u));
+        if (SRC == PATH_BATCH) {
+          cs = scene_of_chunk(st, cb);
+          const uint64_t first = (uint64_t)(cb - st.chunk_base[cs]) * 64u;
+          const uint64_t n_s = st.sample_base[cs + 1] - st.sample_base[cs];
+          cn = (uint32_t)__builtin_amdgcn_readfirstlane((int)(n_s - first < 64u ? n_s - first : 64u));
+        } else if (SRC == PATH_FRAME) {
+          cs = 0;
+          cn = min(st.unit, st.n_samples - cb * st.unit);
+        } else {
+          cs = 0;
+          cn = (uint32_t)__builtin_amdgcn_readfirstlane((int)st.cl.desc[cb].y);
+        }
       }
-      if (cs != scene) {
+      if (SRC == PATH_BATCH && cs != scene) {
         if (__any(act)) break;  // the wave finishes its scene's paths first
         scene = cs;
         const Params& P = scene_params(st.scenes, scene);
-        one_light = P.nee && P.n_lights == 1;
+        one_light = NEE && P.nee && P.n_lights == 1;
         if (one_light) U = uniform_light(P, P.lights[0]);
       }
-      const uint32_t take = min((uint32_t)__popcll(need), cn - co);
+      const uint32_t take = min(min((uint32_t)__popcll(need), room), cn - co);
       const uint32_t rank = (uint32_t)__popcll(need & below);
       if (!act && rank < take) {
-        const Params& P = scene_params(st.scenes, scene);
-        const uint64_t r = (uint64_t)(cb - st.chunk_base[scene]) * 64u + co + rank;  // sample of the scene
-        pixel = (int64_t)(r / (uint32_t)P.spp);
-        k = (uint32_t)(r % (uint32_t)P.spp);
-        const int sub = (int)(k % (uint32_t)(P.SS * P.SS));
-        camera_ray(P, (int)(pixel % P.W), (int)(pixel / P.W), sub % P.SS, sub / P.SS, o, d);
-        tr[0] = tr[1] = tr[2] = 1.0f;
-        pw[0] = pw[1] = pw[2] = 0.0f;
-        nr[0] = nr[1] = nr[2] = 0.0f;
-        meta = rng_c2(0, 1u);
-        gs = st.sample_base[scene] + r;
-        acc[0] = acc[1] = acc[2] = 0ull;
-        npend = 0;
+        const Params& P = SRC == PATH_BATCH ? scene_params(st.scenes, scene) : P1;
+        if (SRC == PATH_QUEUE) {
+          const uint32_t i = st.cl.desc[cb].x + co + rank;
+          o = mk(st.q.ox[i], st.q.oy[i], st.q.oz[i]);
+          d = mk(st.q.dx[i], st.q.dy[i], st.q.dz[i]);
+          tr[0] = st.q.tr[i]; tr[1] = st.q.tg[i]; tr[2] = st.q.tb[i];
+          pw[0] = st.q.pr[i]; pw[1] = st.q.pg[i]; pw[2] = st.q.pb[i];
+          meta = st.q.meta[i] & ~META_NEE;
+          slot = st.q.slot[i];
+        } else {
+          if (SRC == PATH_BATCH) slot = (cb - st.chunk_base[scene]) * 64u + co + rank;
+          else slot = cb * st.unit + co + rank;
+          if (SRC == PATH_FRAME && P.mlt_u != nullptr) {  // a Metropolis proposal's own camera ray
+            o = mk(st.q.ox[slot], st.q.oy[slot], st.q.oz[slot]);
+            d = mk(st.q.dx[slot], st.q.dy[slot], st.q.dz[slot]);
+          } else {
+            const int64_t pixel = st.batch.pixel_base + (int64_t)(slot / (uint32_t)P.spp);
+            const int sub = (int)(slot % (uint32_t)P.spp % (uint32_t)(P.SS * P.SS));
+            camera_ray(P, (int)(pixel % P.W), (int)(pixel / P.W), sub % P.SS, sub / P.SS, o, d);
+          }
+          tr[0] = tr[1] = tr[2] = 1.0f;
+          pw[0] = pw[1] = pw[2] = 0.0f;
+          meta = rng_c2(0, 1u);
+          ++n_prim;
+        }
         act = true;
-        ++n_prim;
       }
       co += take;
+      room -= take;
       if (co >= cn) {
         ++cb;
         co = 0;
@@ -144,50 +264,90 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
       if (!claims_left && cb >= ce) break;
       continue;
     }
-    const Params& P = scene_params(st.scenes, scene);
-    // ---- next-event estimation of the segment's origin vertex
-    // (k_stream_nee / k_stream_shadow on this segment's queue entry)
-    if (act && (meta & META_NEE)) {
-      uint32_t w[9];
-      nee_words(P, (uint32_t)pixel, k, (int)(meta & 0xFFu) - 1, META_BRANCH(meta), w);
-      const d3 x = o, nrm = mk(nr[0], nr[1], nr[2]), ct = mk(tr[0], tr[1], tr[2]);
-      for (int m = 0; m < 3; ++m) {
-        ShadowRay sr;
-        int32_t l = -1;
-        const bool ok = one_light ? nee_one_single(U, w, m, x, nrm, ct, sr, l) : nee_one(P, w, m, x, nrm, ct, sr, l);
-        if (ok) {
-          ++n_shadow;
-          if (!occluded(P, sr.o2, sr.dir, sr.tmax, S, tsh)) {
-            acc[0] += fix_of(sr.c[0]);
-            acc[1] += fix_of(sr.c[1]);
-            acc[2] += fix_of(sr.c[2]);
+    const Params& P = SRC == PATH_BATCH ? scene_params(st.scenes, scene) : P1;
+    const uint32_t pixel = (uint32_t)(st.batch.pixel_base + (int64_t)(slot / (uint32_t)P.spp));
+    const uint32_t k = slot % (uint32_t)P.spp;
+    // ---- light samples and closest hits
+    double t = PS_INF;
+    int32_t id = -1;
+    if (!NEE) {
+      if (act) {
+        (void)trace_lane(P, slots, o + d * 0.000001, d, false, t, id, S, tc, tsh);
+        ++n_traced;
+      }
+    } else {
+      const bool lit = act && (meta & META_NEE);
+      const uint64_t lit_m = __ballot(lit);
+      const uint32_t n_items = 3u * (uint32_t)__popcll(lit_m);
+      if (lit) s_map[wbase + (uint32_t)__popcll(lit_m & below)] = (uint8_t)lane;
+      wave_fence();
+      const uint32_t n_idle = 64u - (uint32_t)__popcll(__ballot(act));
+      uint32_t item = act ? 0xFFFFFFFFu : (uint32_t)__popcll(__ballot(!act) & below);  // this round's light sample
+      for (uint32_t base = n_idle;; base += 64u) {
+        const bool first = base == n_idle;
+        const bool has = item < n_items;
+        bool shadow = false;
+        ShadowRay sr{};
+        int src = (int)lane;
+        if (__any(has)) {
+          if (has) src = (int)s_map[wbase + item / 3u];
+          const d3 x = shfl_d3(o, src);
+          const d3 nrm = mk(__shfl(nr[0], src, 64), __shfl(nr[1], src, 64), __shfl(nr[2], src, 64));
+          const d3 ct = mk(__shfl(tr[0], src, 64), __shfl(tr[1], src, 64), __shfl(tr[2], src, 64));
+          const uint32_t sp = (uint32_t)__shfl((int)pixel, src, 64), sk = (uint32_t)__shfl((int)k, src, 64);
+          const uint32_t sm = (uint32_t)__shfl((int)meta, src, 64);
+          if (has) {
+            uint32_t w[3];
+            nee_words_of(P, sp, sk, (int)(sm & 0xFFu) - 1, META_BRANCH(sm), (int)(item % 3u), w);
+            int32_t l = -1;
+            shadow = one_light ? nee_one_single(U, w, 0, x, nrm, ct, sr, l) : nee_one(P, w, 0, x, nrm, ct, sr, l);
           }
         }
+        const bool closest = first && act;
+        if (closest || shadow) {
+          double tt = closest ? PS_INF : sr.tmax;
+          int32_t hid = -1;
+          const bool blocked = trace_lane(P, slots, closest ? o + d * 0.000001 : sr.o2, closest ? d : sr.dir, !closest, tt, hid,
+                                          S, tc, tsh);
+          if (closest) {
+            t = tt;
+            id = hid;
+            ++n_traced;
+          } else {
+            ++n_shadow;
+            if (!blocked) {
+              for (int c = 0; c < 3; ++c)
+                if (const uint64_t v = fix_of(sr.c[c]))
+                  atomicAdd((unsigned long long*)&s_acc[c][wbase + (uint32_t)src], (unsigned long long)v);
+            }
+          }
+        }
+        if (base >= n_items) break;
+        item = base + lane;
       }
     }
-    // ---- the segment's closest hit and its vertex
+    wave_fence();
+    // ---- the segments' vertices
     if (act) {
-      double t, u, v;
-      int32_t id;
-      closest_hit(P, o, d, t, id, u, v, S, tc);
-      ++n_traced;
       LaneCtx C;
       C.has0 = false;
-      C.pend = pend;
-      C.npend = npend;
+      C.pool = pool;
+      C.pool_n = &s_pool[wib];
+      C.slot = slot;
       C.truncated = C.n_ext = C.pickups = C.dropped = C.direct = 0;
       VertexAdj va;
-      const d3 add = shade_vertex(P, P.mats, C, o, d, t, id, mk(tr[0], tr[1], tr[2]), mk(pw[0], pw[1], pw[2]),
-                                  (uint32_t)pixel, k, (int)(meta & 0xFFu), META_BRANCH(meta), va);
-      acc[0] += fix_of(add.x);
-      acc[1] += fix_of(add.y);
-      acc[2] += fix_of(add.z);
-      npend = C.npend;
+      const int depth = (int)(meta & 0xFFu);
+      const d3 add = shade_vertex(P, lds_mats ? lds_mats : P.mats, C, o, d, t, id, mk(tr[0], tr[1], tr[2]), mk(pw[0], pw[1], pw[2]), pixel, k,
+                                  depth, META_BRANCH(meta), va);
+      uint64_t acc[3] = {fix_of(add.x), fix_of(add.y), fix_of(add.z)};
       truncated += C.truncated;
       n_ext += C.n_ext;
       pickups += C.pickups;
       dropped += C.dropped;
+      if (SRC == PATH_FRAME && depth == 0 && P.mlt_flags != nullptr) P.mlt_flags[slot] = C.direct;
       if (C.has0) {
+        for (int c = 0; c < 3; ++c)
+          if (acc[c]) s_acc[c][threadIdx.x] += acc[c];
         o = C.o0;
         d = C.d0;
         for (int j = 0; j < 3; ++j) {
@@ -196,21 +356,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           nr[j] = C.n0[j];
         }
         meta = C.meta0;
-      } else if (npend > 0) {
-        const PendRec& r = pend[--npend];
-        o = mk(r.o[0], r.o[1], r.o[2]);
-        d = mk(r.d[0], r.d[1], r.d[2]);
-        for (int j = 0; j < 3; ++j) {
-          tr[j] = r.t[j];
-          pw[j] = r.p[j];
-          nr[j] = r.n[j];
-        }
-        meta = r.meta;
       } else {
-        uint64_t* a = st.accum + 3 * gs;
-        a[0] = acc[0];
-        a[1] = acc[1];
-        a[2] = acc[2];
+        const uint64_t at = (SRC == PATH_BATCH ? st.sample_base[scene] : 0ull) + slot;
+        for (int c = 0; c < 3; ++c) {
+          acc[c] += s_acc[c][threadIdx.x];
+          s_acc[c][threadIdx.x] = 0ull;
+          if (acc[c]) atomicAdd((unsigned long long*)&st.accum[3 * at + c], (unsigned long long)acc[c]);
+        }
         act = false;
       }
     }
@@ -220,18 +372,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   const uint64_t s_prim = wave_sum_u32(n_prim), s_tr = wave_sum_u32(n_traced), s_sh = wave_sum_u32(n_shadow);
   const uint64_t s_ext = wave_sum_u32(n_ext), s_pick = wave_sum_u32(pickups), s_trunc = wave_sum_u32(truncated);
   const uint64_t s_drop = wave_sum_u32(dropped);
-  if (lane_id() == 0) {
-    if (s_prim) atomicAdd((unsigned long long*)&st.ctr[CTR_QUEUED], (unsigned long long)s_prim);
-    if (s_tr) atomicAdd((unsigned long long*)&st.ctr[CTR_TRACED], (unsigned long long)s_tr);
-    if (s_sh) atomicAdd((unsigned long long*)&st.ctr[CTR_SHADOW], (unsigned long long)s_sh);
-    if (s_sh) atomicAdd((unsigned long long*)&st.ctr[CTR_STRACED], (unsigned long long)s_sh);
-    if (s_ext) atomicAdd((unsigned long long*)&st.ctr[CTR_EXT], (unsigned long long)s_ext);
-    if (s_pick) atomicAdd((unsigned long long*)&st.ctr[CTR_PICKUP], (unsigned long long)s_pick);
-    if (s_trunc) atomicAdd((unsigned long long*)&st.ctr[CTR_TRUNC], (unsigned long long)s_trunc);
-    if (s_drop) atomicAdd((unsigned long long*)&st.ctr[CTR_DROP], (unsigned long long)s_drop);
+  if (lane == 0) {
+    auto count = [&](int c, uint64_t v) {
+      if (v) atomicAdd((unsigned long long*)&st.ctr[c], (unsigned long long)v);
+    };
+    count(CTR_QUEUED, s_prim + s_ext);
+    count(CTR_TRACED, s_tr);
+    count(CTR_SHADOW, s_sh);
+    count(CTR_STRACED, s_sh);
+    count(CTR_EXT, s_ext);
+    count(CTR_PICKUP, s_pick);
+    count(CTR_TRUNC, s_trunc);
+    count(CTR_DROP, s_drop);
   }
 }
-
 // Every pixel of every scene of the batch: fold its samples' accumulators
 // into the scene's image (fold_pixel: 1/spp scale, luminance clamp,
 // sensor_response, variance of the mean).  pixel_base[s]: first pixel of
@@ -260,35 +414,34 @@ __global__ __launch_bounds__(256) void k_persist_resolve(Persist st, int64_t n_p
 }
 
 // ------------------------------------------------------------ launchers
-// The kernel instance for an LDS stack depth (8 or 16 entries) and a register
-// budget of `waves` waves per SIMD (2, 3 or 4).
+// 3 waves per SIMD for launches that fill them (the no-NEE instance fits 168
+// VGPRs: spheres 320x240 x 16 spp 1033 -> 951 us, glass with NEE 3260 -> 3063
+// although it spills), 2 for smaller ones, which gain nothing from more waves
+// and lose the LDS (Metropolis steps 425 -> 490 us at 3); 4 spill too much
+// (spheres 2.5 ms) and stay for callers that ask for them.
+// LDS of the instances: at 2 waves per SIMD (two blocks per CU) 12 stack
+// entries and five BVH levels, so that the tree's top costs an LDS access
+// instead of an L2 one, or for a batch of scenes, which shares no tree, 32
+// entries; at 3 waves 14 entries and four levels, or 20; at 4 waves 12 and
+// three levels.
+template <int SRC, bool NEE, class F>
+static hipError_t with_path_waves(int waves, F&& f) {
+  constexpr bool batch = SRC == PATH_BATCH;
+  if (waves <= 2) return f(k_path<SRC, NEE, batch ? 32 : 12, batch ? PRT_TOP_NODES : PRT_WIDE_NODES, 2>);
+  if (waves == 3) return f(k_path<SRC, NEE, batch ? 20 : 14, batch ? PRT_TOP_NODES : 85, 3>);
+  return f(k_path<SRC, NEE, 12, PRT_TOP_NODES, 4>);
+}
 template <class F>
-static hipError_t with_persist_kernel(int stack_lds, int waves, F&& f) {
-  if (stack_lds <= 8) {
-    if (waves <= 2) return f(k_persist<8, 2>);
-    if (waves == 3) return f(k_persist<8, 3>);
-    return f(k_persist<8, 4>);
-  }
-  if (stack_lds <= 16) {
-    if (waves <= 2) return f(k_persist<16, 2>);
-    if (waves == 3) return f(k_persist<16, 3>);
-    return f(k_persist<16, 4>);
-  }
-  // 32 entries (64 KB of LDS per block) only at the 2-wave budget, where two
-  // blocks per CU fit
-  return f(k_persist<32, 2>);
+static hipError_t with_path_kernel(PathSource src, bool nee, int waves, F&& f) {
+  if (src == PATH_BATCH) return nee ? with_path_waves<PATH_BATCH, true>(waves, f) : with_path_waves<PATH_BATCH, false>(waves, f);
+  if (src == PATH_FRAME) return nee ? with_path_waves<PATH_FRAME, true>(waves, f) : with_path_waves<PATH_FRAME, false>(waves, f);
+  return with_path_waves<PATH_QUEUE, true>(waves, f);
 }
 
-hipError_t launch_persist(const Persist& p, int stack_lds, int waves, int blocks, hipStream_t s) {
-  return with_persist_kernel(stack_lds, waves, [&](void (*k)(Persist)) {
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, p);
+hipError_t launch_path(PathSource src, const Persist& p, const Params& P, int waves, int blocks, hipStream_t s) {
+  return with_path_kernel(src, p.nee != 0, waves, [&](void (*k)(Persist, Params)) {
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, p, P);
     return hipGetLastError();
-  });
-}
-
-hipError_t persist_blocks_per_cu(int stack_lds, int waves, int* blocks) {
-  return with_persist_kernel(stack_lds, waves, [&](void (*k)(Persist)) {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, k, 256, 0);
   });
 }
 

@@ -98,18 +98,19 @@ __device__ __forceinline__ void emit_child(ShadeCtx& C, d3 o, d3 d, d3 ct, d3 pw
   C.n_ext++;
 }
 
-// The children of one vertex in the persistent renderer: the first becomes
-// the lane's next segment (registers), a second goes to the lane's pending
-// stack.  Throughput, pickup weight and NEE normal are rounded to float as a
-// queue entry stores them (emit_child above), so a segment continues
-// bit-identically to the queued renderers.
+// The children of one vertex in the path kernel: the first becomes the
+// lane's next segment (registers), a second goes to the wave's pool, from
+// which any idle lane of the wave takes it.  Throughput, pickup weight and NEE
+// normal are rounded to float as a queue entry stores them (emit_child
+// above), so a segment continues bit-identically to the queued renderers.
 struct LaneCtx {
   d3 o0, d0;
   float t0[3], p0[3], n0[3];
   uint32_t meta0;
   bool has0;
-  PendRec* pend;
-  int npend;
+  PoolRec* pool;     // the wave's records
+  uint32_t* pool_n;  // their count (LDS)
+  uint32_t slot;
   uint32_t truncated, n_ext, pickups, dropped;
   uint32_t direct;
 };
@@ -117,7 +118,6 @@ struct LaneCtx {
 __device__ __forceinline__ void emit_child(LaneCtx& C, d3 o, d3 d, d3 ct, d3 pw, uint32_t meta, d3 nrm) {
   const float t[3] = {(float)ct.x, (float)ct.y, (float)ct.z};
   const float p[3] = {(float)pw.x, (float)pw.y, (float)pw.z};
-  const float n[3] = {(float)nrm.x, (float)nrm.y, (float)nrm.z};
   if (!C.has0) {
     C.has0 = true;
     C.o0 = o;
@@ -125,22 +125,25 @@ __device__ __forceinline__ void emit_child(LaneCtx& C, d3 o, d3 d, d3 ct, d3 pw,
     for (int k = 0; k < 3; ++k) {
       C.t0[k] = t[k];
       C.p0[k] = p[k];
-      C.n0[k] = n[k];
     }
+    C.n0[0] = (float)nrm.x; C.n0[1] = (float)nrm.y; C.n0[2] = (float)nrm.z;
     C.meta0 = meta;
-  } else if (C.npend < PRT_PEND_DEPTH) {
-    PendRec& r = C.pend[C.npend++];
+  } else {
+    // the second child of a glass vertex: no NEE flag, so no normal
+    const uint32_t j = agg_append(C.pool_n);
+    if (j >= PRT_PATH_POOL) {
+      C.dropped++;
+      return;
+    }
+    PoolRec& r = C.pool[j];
     r.o[0] = o.x; r.o[1] = o.y; r.o[2] = o.z;
     r.d[0] = d.x; r.d[1] = d.y; r.d[2] = d.z;
     for (int k = 0; k < 3; ++k) {
       r.t[k] = t[k];
       r.p[k] = p[k];
-      r.n[k] = n[k];
     }
     r.meta = meta;
-  } else {
-    C.dropped++;
-    return;
+    r.slot = C.slot;
   }
   C.n_ext++;
 }
@@ -454,6 +457,19 @@ __device__ __forceinline__ void nee_words(const Params& P, uint32_t pixel, uint3
   w[0] = b1[0]; w[1] = b1[1]; w[2] = b1[2]; w[3] = b1[3];
   w[4] = b2[0]; w[5] = b2[1]; w[6] = b2[2]; w[7] = b2[3];
   w[8] = b3[0];
+}
+
+// The three words of light sample m alone (w[3m .. 3m + 2] of nee_words), at
+// two Philox blocks instead of three.
+__device__ __forceinline__ void nee_words_of(const Params& P, uint32_t pixel, uint32_t sample, int depth,
+                                             uint32_t branch, int m, uint32_t w[3]) {
+  const uint32_t c2 = rng_c2(depth, branch), first = m == 2 ? 2u : 1u;
+  uint32_t a[4], b[4];
+  philox(pixel, sample, c2, first, P.key0, P.key1, a);
+  philox(pixel, sample, c2, first + 1u, P.key0, P.key1, b);
+  w[0] = m == 0 ? a[0] : m == 1 ? a[3] : a[2];
+  w[1] = m == 0 ? a[1] : m == 1 ? b[0] : a[3];
+  w[2] = m == 0 ? a[2] : m == 1 ? b[1] : b[0];
 }
 
 // Light sample m (0..2) of a diffuse vertex at x (orienting normal nrm,

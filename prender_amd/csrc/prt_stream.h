@@ -149,32 +149,44 @@ struct Stream {
   int32_t nee_max_lights;   // most lights of any scene (picks how k_stream_nee reads light records)
 };
 
-// The persistent form of the batched renderer (prt_persist.hip): one launch
-// renders every camera sample of the batch.  Camera samples are numbered
-// scene by scene (scene s owns samples sample_base[s] ..., pixel-major, spp
-// per pixel) and cut into 64-sample chunks (scene s owns chunks
-// chunk_base[s] .. chunk_base[s+1]-1; a scene's last chunk may be short).
+// Work of one path-kernel launch (prt_persist.hip), in chunks that waves claim
+// claim at a time, the first ones by their number.
+//   A batch's camera samples are numbered scene by scene (scene s owns samples
+// sample_base[s] ..., pixel-major, spp per pixel) and cut into 64-sample chunks
+// (scene s owns chunks chunk_base[s] .. chunk_base[s+1]-1; a scene's last
+// chunk may be short).  A frame's n_samples are cut into chunks of unit.  A
+// queue brings its own chunk list.
 struct Persist {
-  const Params* scenes;         // [n_scenes]
+  const Params* scenes;         // [n_scenes] (batch)
   const uint32_t* chunk_base;   // [n_scenes + 1]
   const uint64_t* sample_base;  // [n_scenes + 1]; sample_base[n_scenes] = all samples
-  uint32_t* next;               // claim counter: first chunk not yet handed out
-  uint64_t* accum;              // [all samples][3] fixed point, written once per sample
-  PendRec* pend;                // [grid threads][PRT_PEND_DEPTH] pending glass segments
+  uint32_t* next;               // claim counter: first chunk not yet handed out, (waves * claim) at the start
+  uint64_t* accum;              // [all samples][3] fixed point, zero at the start
+  PoolRec* pool;                // [grid waves][PRT_PATH_POOL] (unused without glass)
   uint64_t* ctr;                // [CTR_COUNT]
   float* const* out_rgb;        // [n_scenes] W*H*3 device images
   float* const* out_var;        // [n_scenes] (entries may be null)
   uint32_t n_chunks;
   uint32_t claim;               // chunks per claim
   int32_t n_scenes;
-  int32_t pad_;
+  uint32_t quota;               // segments a wave holds before it starts no further sample
+  uint32_t unit;                // samples per chunk of a frame
+  uint32_t n_samples;           // of a frame
+  int32_t nee;                  // some scene samples lights
+  Batch batch;                  // pixels of a frame or queue
+  RayQ q;                       // a queue's rays; the camera rays of Metropolis proposals
+  ChunkList cl;                 // a queue's chunks
 };
 
-// stack_lds: 8, 16 or (at 2 waves, where two 66-KB blocks fit a CU) 32 LDS
-// stack entries; waves: waves per SIMD its registers are budgeted for (2..4).
-hipError_t launch_persist(const Persist& p, int stack_lds, int waves, int blocks, hipStream_t s);
-// Resident 256-thread blocks per CU of that kernel instance.
-hipError_t persist_blocks_per_cu(int stack_lds, int waves, int* blocks);
+// Where a launch's segments come from.
+enum PathSource {
+  PATH_BATCH = 0,  // the camera samples of n_scenes scenes, 64 per chunk
+  PATH_FRAME = 1,  // the camera samples of one scene (or its Metropolis proposals), unit per chunk
+  PATH_QUEUE = 2   // the rays of a queue, whose vertices have had their light samples
+};
+// waves: waves per SIMD its registers are budgeted for (2..4).  P: the scene
+// of a frame or queue.
+hipError_t launch_path(PathSource src, const Persist& p, const Params& P, int waves, int blocks, hipStream_t s);
 hipError_t launch_persist_resolve(const Persist& p, int64_t n_pixels_total, const int64_t* d_pixel_base,
                                   hipStream_t s);
 

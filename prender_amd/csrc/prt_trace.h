@@ -78,10 +78,11 @@ typedef StackN<PRT_STACK_LDS> Stack;
 #define PRT_DECLARE_STACK(S, P, REGION) PRT_DECLARE_STACK_N(S, P, PRT_STACK_LDS, REGION)
 
 // Copies BVH nodes 0..NTOP-1 (the top levels, numbered first by the builder;
-// NTOP <= PRT_TOP_NODES) into the block's LDS for stack S.  Every thread of
+// NTOP <= PRT_TOP_NODES, or <= CAP) into the block's LDS for stack S.  Every thread of
 // the block must reach it.
-#define PRT_TOP_CACHE(S, NODES, NTOP)                                                        \
-  __shared__ float4 s_top_[PRT_TOP_NODES * 8];                                               \
+#define PRT_TOP_CACHE(S, NODES, NTOP) PRT_TOP_CACHE_N(S, NODES, NTOP, PRT_TOP_NODES)
+#define PRT_TOP_CACHE_N(S, NODES, NTOP, CAP)                                                 \
+  __shared__ float4 s_top_[(CAP) * 8];                                                       \
   {                                                                                          \
     const int nt_ = (NTOP);                                                                  \
     const float4* g_ = reinterpret_cast<const float4*>(NODES);                               \
@@ -211,9 +212,11 @@ __device__ __forceinline__ int32_t hit_entity(const float4* tris4, int32_t id) {
 // closest hit is the one over all triangles, with the tie rule of
 // nearer_hit.
 #define PRT_TRAV_DONE 0x7FFFFFFF
-template <bool ANY, class Stk>
-__device__ __forceinline__ bool traverse_ww(const Params& P, d3 o, d3 d, double& t_best, int32_t& id_best, double& ub,
-                                            double& vb, Stk& S, TravStats& ts) {
+// any (the same for every ray of a launch, or a lane's own): stop at the first
+// hit below t_best instead.
+template <class Stk>
+__device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 d, double& t_best, int32_t& id_best,
+                                            double& ub, double& vb, Stk& S, TravStats& ts) {
   if (P.n_nodes <= 0) return false;
   const float ox = (float)o.x, oy = (float)o.y, oz = (float)o.z;
   float ix = (float)(1.0 / d.x), iy = (float)(1.0 / d.y), iz = (float)(1.0 / d.z);
@@ -226,7 +229,7 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, d3 o, d3 d, double&
   bool found = false;
   int sp = 0;
   const float4* tris4 = reinterpret_cast<const float4*>(P.tris);
-  int32_t e_best = ANY ? 0 : hit_entity(tris4, id_best);
+  int32_t e_best = any ? 0 : hit_entity(tris4, id_best);
   // cur: internal node (0 <= cur < PRT_TRAV_DONE), leaf code (< 0) or
   // PRT_TRAV_DONE; lf: parked leaf (< 0) or none (>= 0)
   int32_t cur = 0, lf = 0;
@@ -272,8 +275,8 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, d3 o, d3 d, double&
         ts.tris++;
         double t, u, v;
         if (mt_test(a, b, c, o, d, t, u, v) &&
-            (ANY ? t < t_best : nearer_hit(t, __float_as_int(a.w), t_best, e_best))) {
-          if (ANY) {
+            (any ? t < t_best : nearer_hit(t, __float_as_int(a.w), t_best, e_best))) {
+          if (any) {
             id_best = (int32_t)(first + k);
             return true;
           }
@@ -294,14 +297,6 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, d3 o, d3 d, double&
   return found;
 }
 
-// Closest (ANY = false) or any (ANY = true) hit over the BVH triangles with
-// t in (1e-6, t_best).  o is the already-nudged origin.
-template <bool ANY, class Stk>
-__device__ __forceinline__ bool traverse(const Params& P, d3 o, d3 d, double& t_best, int32_t& id_best, double& ub,
-                                         double& vb, Stk& S, TravStats& ts) {
-  return traverse_ww<ANY>(P, o, d, t_best, id_best, ub, vb, S, ts);
-}
-
 // Closest hit over analytic entities then the BVH; o_in is the ray origin
 // before the 1e-6 nudge.  id >= 0: triangle slot; id <= -2: analytic entity
 // -2-id; -1: miss.
@@ -320,7 +315,7 @@ __device__ __forceinline__ void closest_hit(const Params& P, d3 o_in, d3 d, doub
       id = -2 - ei;
     }
   }
-  traverse<false>(P, o, d, t, id, u, v, S, ts);
+  traverse_ww(P, false, o, d, t, id, u, v, S, ts);
 }
 
 // Any blocker with t in (1e-6, tmax) from the already-nudged origin o.
@@ -332,7 +327,70 @@ __device__ __forceinline__ bool occluded(const Params& P, d3 o, d3 d, double tma
   }
   int32_t id = -1;
   double u, v;
-  return traverse<true>(P, o, d, tmax, id, u, v, S, ts);
+  return traverse_ww(P, true, o, d, tmax, id, u, v, S, ts);
+}
+
+// The analytic entities of a scene (at most PRT_LDS_ANALYTIC) as a block
+// keeps them in LDS, spheres first.
+#define PRT_LDS_ANALYTIC 16
+struct AnalyticSlot {
+  double p0[3], radius;                                 // sphere; uvplane: p0
+  double u_axis[3], v_axis[3], normal[3], u_len, v_len; // uvplane
+  int32_t ei, ninv;
+};
+
+// One ray per lane, closest and any hits side by side: closest_hit's hit of
+// the lanes without `any` (t, id; t enters as PS_INF), occluded's answer below
+// t of the others.  o is the already-nudged origin.  slots: the scene's
+// analytic entities in LDS, or null.
+//
+// A wave here often runs alone on its SIMD, so a test's time is the latency of
+// its chain: the records come from LDS instead of through three dependent
+// global loads, and the spheres are tested without branches, so that several
+// chains overlap (nine spheres: 13,800 -> 6,400 cycles).
+template <class Stk>
+__device__ __forceinline__ bool trace_lane(const Params& P, const AnalyticSlot* slots, d3 o, d3 d, bool any, double& t,
+                                           int32_t& id, Stk& S, TravStats& tc, TravStats& tsh) {
+  bool blocked = false;
+  int32_t e_best = 0x7FFFFFFF;
+  auto meet = [&](bool hit, double tt, int32_t ei) {
+    const bool near = hit && (any ? tt < t : nearer_hit(tt, ei, t, e_best));
+    if (near && !any) {
+      t = tt;
+      id = -2 - ei;
+      e_best = ei;
+    }
+    blocked |= near && any;
+  };
+  if (slots != nullptr) {
+#pragma unroll 3
+    for (int k = 0; k < P.n_spheres; ++k) {
+      const AnalyticSlot& e = slots[k];
+      double tt;
+      const bool hit = sphere_root(ld3(e.p0), e.radius, o, d, tt);
+      meet(hit, tt, e.ei);
+    }
+    for (int k = P.n_spheres; k < P.n_analytic; ++k) {
+      const AnalyticSlot& e = slots[k];
+      double tt;
+      const bool hit = uvplane_t(e, o, d, tt);
+      meet(hit, tt, e.ei);
+    }
+  } else {
+    for (int k = 0; k < P.n_analytic; ++k) {
+      const int32_t ei = P.analytic[k];
+      double tt;
+      const bool hit = analytic_t(P.ents[ei], o, d, tt);
+      meet(hit, tt, ei);
+    }
+  }
+  if (blocked) return true;
+  TravStats ts{0, 0, 0};
+  double u, v;
+  blocked = traverse_ww(P, any, o, d, t, id, u, v, S, ts) && any;
+  (any ? tsh : tc).nodes += ts.nodes;
+  (any ? tsh : tc).tris += ts.tris;
+  return blocked;
 }
 
 // ------------------------------------------------ chunk claims
