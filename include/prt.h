@@ -236,7 +236,7 @@ int prt_trace_closest_device(prt_scene* scene, const prt_ray* d_rays, int64_t n,
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the same query and the same hits as
  * prt_trace_closest_device, with no hipMalloc, hipFree or event creation in
- * the call.  Its traversal counters live in a fixed 256-byte device array of
+ * the call.  Its traversal counters live in a fixed 4-KB device array of
  * the library (one per GPU, held until the process ends), cleared on every
  * call; no argument size changes what it needs, so no call is refused for
  * size.  Calls that overlap on one GPU (two threads or two streams) share

@@ -547,8 +547,8 @@ static int trace_device(prt_scene* s, const prt_ray* d_rays, int64_t n, prt_hit*
   HIPCHK(hipSetDevice(s->device));
   std::lock_guard<std::recursive_mutex> pool_lock(s->pool->m);
   int rc;
-  if ((rc = dev_alloc(s->pool->ws.ctr, CTR_COUNT * sizeof(uint64_t)))) return rc;
-  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_COUNT, s->stream));
+  if ((rc = dev_alloc(s->pool->ws.ctr, CTR_WORDS * sizeof(uint64_t)))) return rc;
+  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_WORDS, s->stream));
   ScopedEvent e0, e1;
   HIPCHK(hipEventCreate(&e0.e));
   HIPCHK(hipEventCreate(&e1.e));
@@ -557,9 +557,10 @@ static int trace_device(prt_scene* s, const prt_ray* d_rays, int64_t n, prt_hit*
     HIPCHK(launch_trace(s->P, (const prt_ray_dev*)d_rays, n, (prt_hit_dev*)d_hits, (uint64_t*)s->pool->ws.ctr.p,
                         s->max_trav_blocks, s->stream));
   HIPCHK(hipEventRecord(e1.e, s->stream));
-  uint64_t c[CTR_COUNT];
-  HIPCHK(hipMemcpyAsync(c, s->pool->ws.ctr.p, sizeof(c), hipMemcpyDeviceToHost, s->stream));
+  uint64_t raw[CTR_WORDS], c[CTR_COUNT];
+  HIPCHK(hipMemcpyAsync(raw, s->pool->ws.ctr.p, sizeof(raw), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
+  sum_counters(raw, c);
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, e0.e, e1.e));
   if (stats) {
@@ -591,13 +592,14 @@ int prt_trace_closest_device_noalloc(prt_scene* s, const prt_ray* d_rays, int64_
   HIPCHK(hipSetDevice(s->device));
   uint64_t* ctr = nullptr;
   HIPCHK(noalloc_scratch(s->device, &ctr));
-  HIPCHK(launch_fill_u64(ctr, 0, CTR_COUNT, s->stream));
+  HIPCHK(launch_fill_u64(ctr, 0, CTR_WORDS, s->stream));
   if (n > 0)
     HIPCHK(launch_trace(s->P, (const prt_ray_dev*)d_rays, n, (prt_hit_dev*)d_hits, ctr, s->max_trav_blocks,
                         s->stream));
-  uint64_t c[CTR_COUNT];
-  HIPCHK(hipMemcpyAsync(c, ctr, sizeof(c), hipMemcpyDeviceToHost, s->stream));
+  uint64_t raw[CTR_WORDS], c[CTR_COUNT];
+  HIPCHK(hipMemcpyAsync(raw, ctr, sizeof(raw), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
+  sum_counters(raw, c);
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     fill_stats(stats, c);
@@ -678,7 +680,7 @@ extern "C++" int prt::ensure_workspace(prt_scene* s, int64_t batch_samples, bool
   if ((rc = dev_alloc(w.counts, 16 * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(w.fetch, (size_t)FETCH_LAUNCHES * PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE * sizeof(uint32_t))))
     return rc;
-  if ((rc = dev_alloc(w.ctr, CTR_COUNT * sizeof(uint64_t)))) return rc;
+  if ((rc = dev_alloc(w.ctr, CTR_WORDS * sizeof(uint64_t)))) return rc;
   if (!w.h_counts) HIPCHK(hipHostMalloc((void**)&w.h_counts, 16 * sizeof(uint32_t), hipHostMallocDefault));
   w.batch_samples = batch_samples;
   w.queue_cap = qcap;
@@ -692,7 +694,7 @@ static int ensure_path_workspace(prt_scene* s, int64_t samples) {
   int rc;
   if ((rc = dev_alloc(w.accum, (size_t)samples * 3 * sizeof(uint64_t)))) return rc;
   if ((rc = dev_alloc(w.counts, 16 * sizeof(uint32_t)))) return rc;
-  return dev_alloc(w.ctr, CTR_COUNT * sizeof(uint64_t));
+  return dev_alloc(w.ctr, CTR_WORDS * sizeof(uint64_t));
 }
 
 // Settings of one render call derived from the scene and the options.
@@ -1019,8 +1021,10 @@ extern "C++" int prt::run_batch(prt_scene* s, const Params& P, const Batch& B, u
 static int finish_stats(prt_scene* s, const RenderSetup& R, Timer& tm, const CallTotals& tot, prt_stats* stats,
                         uint64_t* c) {
   hipStream_t st = s->stream;
-  HIPCHK(hipMemcpyAsync(c, s->pool->ws.ctr.p, CTR_COUNT * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+  uint64_t raw[CTR_WORDS];
+  HIPCHK(hipMemcpyAsync(raw, s->pool->ws.ctr.p, sizeof(raw), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  sum_counters(raw, c);
   if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
   // every queued ray must have been traced exactly once
   if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
@@ -1151,7 +1155,7 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
     return rc;
   }
   hipStream_t st = s->stream;
-  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_COUNT, st));
+  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_WORDS, st));
   Timer tm;
   if ((rc = tm.begin(path || (o && o->timing != 0), st, &s->timer_events))) return rc;
   CallTotals tot;
@@ -1317,7 +1321,7 @@ int prt_adjoint_device(prt_scene* s, const prt_render_opts* o, const float* d_di
   double* g_alb = (double*)s->grad_buf.p;
   double* g_e = g_alb + 3 * nf;
   HIPCHK(launch_fill_u64((uint64_t*)g_alb, 0ull, 3 * nf + 3, st));
-  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_COUNT, st));
+  HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_WORDS, st));
   Timer tm;
   if ((rc = tm.begin(o && o->timing != 0, st, &s->timer_events))) return rc;
   CallTotals tot;

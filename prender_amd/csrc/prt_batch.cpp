@@ -234,7 +234,7 @@ int ensure_stream_workspace(prt_scene* lead, const BatchConfig& c, const StreamG
   }
   const size_t W = PRT_SLAB_WAVES;
   if ((rc = dev_alloc(w.accum, (size_t)inflight * 3 * sizeof(uint64_t)))) return rc;
-  if ((rc = dev_alloc(w.ctr, CTR_COUNT * sizeof(uint64_t)))) return rc;
+  if ((rc = dev_alloc(w.ctr, CTR_WORDS * sizeof(uint64_t)))) return rc;
   if ((rc = dev_alloc(w.ctl, sizeof(StreamCtl)))) return rc;
   if ((rc = dev_alloc(w.slot_info, (size_t)c.n_slots * sizeof(SlotInfo)))) return rc;
   if ((rc = dev_alloc(w.live, (size_t)c.n_slots * sizeof(int32_t)))) return rc;
@@ -446,7 +446,7 @@ int run_stream(prt_scene* const* scenes, int n, const BatchConfig& c, float* con
 
   hipError_t he = hipEventRecord(e0, s);
   if (he == hipSuccess) he = launch_fill_u64(S.accum, 0ull, (int64_t)c.n_slots * T * 3, s);
-  if (he == hipSuccess) he = launch_fill_u64(S.ctr, 0ull, CTR_COUNT, s);
+  if (he == hipSuccess) he = launch_fill_u64(S.ctr, 0ull, CTR_WORDS, s);
   if (he == hipSuccess) he = launch_stream_init(S, s);
   if (he != hipSuccess) {
     cleanup();
@@ -506,11 +506,12 @@ int run_stream(prt_scene* const* scenes, int n, const BatchConfig& c, float* con
   }
   he = join();
   if (he == hipSuccess) he = hipEventRecord(e1, s);
-  uint64_t ctrh[CTR_COUNT];
+  uint64_t raw[CTR_WORDS], ctrh[CTR_COUNT] = {};
   StreamCtl final_ctl;
-  if (he == hipSuccess) he = hipMemcpyAsync(ctrh, S.ctr, sizeof(ctrh), hipMemcpyDeviceToHost, s);
+  if (he == hipSuccess) he = hipMemcpyAsync(raw, S.ctr, sizeof(raw), hipMemcpyDeviceToHost, s);
   if (he == hipSuccess) he = hipMemcpyAsync(&final_ctl, S.ctl, sizeof(StreamCtl), hipMemcpyDeviceToHost, s);
   if (he == hipSuccess) he = hipStreamSynchronize(s);
+  if (he == hipSuccess) sum_counters(raw, ctrh);
   float ms = 0;
   if (he == hipSuccess) he = hipEventElapsedTime(&ms, e0, e1);
   double cat[T_NCAT] = {0, 0, 0, 0, 0, 0};
@@ -607,7 +608,7 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
     w.ovf_words = ovf_words;
   }
   if (threads > w.ovf_threads) return fail(PRT_E_INTERNAL, "persistent grid larger than the overflow area");
-  if ((rc = dev_alloc(w.ctr, CTR_COUNT * sizeof(uint64_t)))) return rc;
+  if ((rc = dev_alloc(w.ctr, CTR_WORDS * sizeof(uint64_t)))) return rc;
   if ((rc = dev_alloc(w.scenes, (size_t)n * sizeof(Params)))) return rc;
   if ((rc = dev_alloc(w.outs, (size_t)n * 2 * sizeof(float*)))) return rc;
   if ((rc = dev_alloc(w.p_accum, (size_t)samples * 3 * sizeof(uint64_t)))) return rc;
@@ -666,7 +667,7 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   HIPCHK(hipEventCreate(&e1.e));
   HIPCHK(hipEventCreate(&e2.e));
   // counters and the claim counter start at zero (fill kernels, not memsets)
-  HIPCHK(launch_fill_u64(P.ctr, 0ull, CTR_COUNT, s));
+  HIPCHK(launch_fill_u64(P.ctr, 0ull, CTR_WORDS, s));
   HIPCHK(launch_fill_u32(d_next, grid.n_waves() * grid.claim, 1, s));
   HIPCHK(launch_fill_u64(P.accum, 0ull, 3 * (int64_t)samples, s));
   HIPCHK(hipEventRecord(e0.e, s));
@@ -674,9 +675,10 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   HIPCHK(hipEventRecord(e1.e, s));
   HIPCHK(launch_persist_resolve(P, pixels, d_pixel, s));
   HIPCHK(hipEventRecord(e2.e, s));
-  uint64_t ctrh[CTR_COUNT];
-  HIPCHK(hipMemcpyAsync(ctrh, P.ctr, sizeof(ctrh), hipMemcpyDeviceToHost, s));
+  uint64_t raw[CTR_WORDS], ctrh[CTR_COUNT];
+  HIPCHK(hipMemcpyAsync(raw, P.ctr, sizeof(raw), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  sum_counters(raw, ctrh);
   float ms_render = 0, ms_resolve = 0;
   HIPCHK(hipEventElapsedTime(&ms_render, e0.e, e1.e));
   HIPCHK(hipEventElapsedTime(&ms_resolve, e1.e, e2.e));

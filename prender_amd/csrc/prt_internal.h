@@ -89,7 +89,7 @@ struct Workspace {
   DevBuf accum, accum2;       // fixed-point sample radiance (accum2: adjoint primal)
   DevBuf counts;              // uint32 [16]: chunks of q0, q1, sq, sq2 at 0..3, entries at 4..7
   DevBuf fetch;               // uint32 claim counters, PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE per launch
-  DevBuf ctr;                 // uint64 [CTR_COUNT]
+  DevBuf ctr;                 // uint64 [CTR_WORDS]
   DevBuf pool;                // path kernel: waiting glass segments, PoolRec [waves][PRT_PATH_POOL]
   uint32_t* h_counts = nullptr;
   void release();

@@ -24,6 +24,27 @@ enum {
   CTR_MLT_ACCEPT = 14,  // Metropolis proposals accepted
   CTR_COUNT = 15
 };
+// The counters are kept in CTR_COPIES copies of one 128-byte line each, by
+// block, and summed by the host (sum_counters).  Atomics on one address
+// serialise across the device at about 7 ns each, and every wave of a launch
+// adds its counts at its end: with one copy a full grid's 8,192 waves took
+// 170 us to add three of them, the time of a launch with few rays.
+#define CTR_LINE 16
+#define CTR_COPIES 32
+#define CTR_WORDS (CTR_LINE * CTR_COPIES)
+static_assert(CTR_COUNT <= CTR_LINE, "a copy of the counters fits its line");
+inline void sum_counters(const uint64_t* raw, uint64_t* c) {
+  for (int k = 0; k < CTR_COUNT; ++k) {
+    c[k] = 0;
+    for (int i = 0; i < CTR_COPIES; ++i) c[k] += raw[i * CTR_LINE + k];
+  }
+}
+// Adds v to counter idx (one lane per wave or block calls it).
+__device__ __forceinline__ void ctr_add(uint64_t* ctr, int idx, uint64_t v) {
+  if (v)
+    atomicAdd((unsigned long long*)&ctr[(blockIdx.x % (uint32_t)CTR_COPIES) * (uint32_t)CTR_LINE + (uint32_t)idx],
+              (unsigned long long)v);
+}
 
 // A path segment waiting in a wave's pool (path kernel): a glass vertex at
 // depth <= 2 emits two children; the lane follows the first, and the second is
@@ -127,9 +148,8 @@ hipError_t launch_trace(const Params& P, const prt_ray_dev* rays, int64_t n, prt
                         int max_blocks, hipStream_t s);
 // Words of the library's file-scope device array that holds the counters of
 // the allocation-free trace entry point (one copy per GPU).
-#define PRT_NOALLOC_SCRATCH_WORDS 32
+#define PRT_NOALLOC_SCRATCH_WORDS CTR_WORDS
 #define PRT_NOALLOC_MAX_DEVICES 64
-static_assert(CTR_COUNT <= PRT_NOALLOC_SCRATCH_WORDS, "trace counters must fit the allocation-free scratch");
 // Device address of that array on `device`, which must be current: looked
 // up with hipGetSymbolAddress on the first call for a device and kept.
 hipError_t noalloc_scratch(int device, uint64_t** out);

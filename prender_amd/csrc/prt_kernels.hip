@@ -312,10 +312,10 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
   const uint64_t s_ext = wave_sum_u32(C.n_ext), s_drop = wave_sum_u32(C.dropped);
   if (lane_id() == 0) {
     slabs[wave] = make_uint2(C.off, min(s_cnt[wib], C.cap));
-    if (s_pick) atomicAdd((unsigned long long*)&ctr[CTR_PICKUP], (unsigned long long)s_pick);
-    if (s_tr) atomicAdd((unsigned long long*)&ctr[CTR_TRUNC], (unsigned long long)s_tr);
-    if (s_ext) atomicAdd((unsigned long long*)&ctr[CTR_EXT], (unsigned long long)s_ext);
-    if (s_drop) atomicAdd((unsigned long long*)&ctr[CTR_DROP], (unsigned long long)s_drop);
+    ctr_add(ctr, CTR_PICKUP, s_pick);
+    ctr_add(ctr, CTR_TRUNC, s_tr);
+    ctr_add(ctr, CTR_EXT, s_ext);
+    ctr_add(ctr, CTR_DROP, s_drop);
   }
 }
 
@@ -392,8 +392,8 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_NEE) void k_nee(
   const uint64_t s_sh = wave_sum_u32(emitted), s_drop = wave_sum_u32(dropped);
   if (lane_id() == 0) {
     slabs[wave] = make_uint2(off, min(s_cnt[wib], slab_cap));
-    if (s_sh) atomicAdd((unsigned long long*)&ctr[CTR_SHADOW], (unsigned long long)s_sh);
-    if (s_drop) atomicAdd((unsigned long long*)&ctr[CTR_DROP], (unsigned long long)s_drop);
+    ctr_add(ctr, CTR_SHADOW, s_sh);
+    ctr_add(ctr, CTR_DROP, s_drop);
   }
 }
 
@@ -458,9 +458,8 @@ __global__ __launch_bounds__(256) void k_slab_index(const uint2* __restrict__ sl
     const uint32_t tot_ent = s_part[1][0] + s_part[1][1] + s_part[1][2] + s_part[1][3];
     *n_chunks = min(sum_ch, max_chunks);
     *n_entries = tot_ent;
-    if (ctr_entries >= 0 && tot_ent) atomicAdd((unsigned long long*)&ctr[ctr_entries], (unsigned long long)tot_ent);
-    if (sum_ch > max_chunks)
-      atomicAdd((unsigned long long*)&ctr[CTR_DROP], (unsigned long long)(sum_ch - max_chunks) * 64ull);
+    if (ctr_entries >= 0) ctr_add(ctr, ctr_entries, tot_ent);
+    if (sum_ch > max_chunks) ctr_add(ctr, CTR_DROP, (uint64_t)(sum_ch - max_chunks) * 64u);
   }
 }
 
@@ -516,7 +515,7 @@ __global__ void k_count_mismatch(const uint64_t* a, const uint64_t* b, int64_t n
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     bad += a[i] != b[i];
   const uint64_t w = wave_sum_u32(bad);
-  if (lane_id() == 0 && w) atomicAdd((unsigned long long*)&ctr[CTR_REPLAY_MISMATCH], (unsigned long long)w);
+  if (lane_id() == 0) ctr_add(ctr, CTR_REPLAY_MISMATCH, w);
 }
 
 // ------------------------------------------------------------ launchers

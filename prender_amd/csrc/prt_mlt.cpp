@@ -112,7 +112,7 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
   hipStream_t st = s->stream;
   uint64_t* ctr = (uint64_t*)s->pool->ws.ctr.p;
   uint64_t* accum = (uint64_t*)s->pool->ws.accum.p;
-  HIPCHK(launch_fill_u64(ctr, 0ull, CTR_COUNT, st));
+  HIPCHK(launch_fill_u64(ctr, 0ull, CTR_WORDS, st));
   HIPCHK(launch_fill_u64(CH.img, 0ull, 3 * n_pix, st));
   Timer tm;
   if ((rc = tm.begin(false, st))) return rc;
@@ -152,9 +152,10 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
   // image * sensor_response / samples, with the MLT mode's 0.25 factor
   // (scene_env.h:1955) and the chains in the reference's place of samples
   HIPCHK(launch_mlt_resolve(CH.img, 3 * n_pix, P.sensor_response * 0.25 / (double)C, d_out, as_f64, st));
-  uint64_t c[CTR_COUNT];
-  HIPCHK(hipMemcpyAsync(c, ctr, sizeof(c), hipMemcpyDeviceToHost, st));
+  uint64_t raw[CTR_WORDS], c[CTR_COUNT];
+  HIPCHK(hipMemcpyAsync(raw, ctr, sizeof(raw), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  sum_counters(raw, c);
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
   if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
@@ -239,7 +240,7 @@ static int render_erpt(prt_scene* s, const prt_erpt_opts* o, void* d_out, int as
   uint64_t* ctr = (uint64_t*)s->pool->ws.ctr.p;
   uint64_t* accum = (uint64_t*)s->pool->ws.accum.p;
   uint64_t* sums = (uint64_t*)w.sums.p;
-  HIPCHK(launch_fill_u64(ctr, 0ull, CTR_COUNT, st));
+  HIPCHK(launch_fill_u64(ctr, 0ull, CTR_WORDS, st));
   HIPCHK(launch_fill_u64(CH.img, 0ull, 3 * n_pix, st));
   HIPCHK(launch_fill_u64(sums, 0ull, 3, st));
   Timer tm;
@@ -306,9 +307,10 @@ static int render_erpt(prt_scene* s, const prt_erpt_opts* o, void* d_out, int as
   // the reference multiplies only image[0] by sensor_response (render.h:1075-1078);
   // every pixel is scaled here, with ERPT's 0.25 factor (scene_env.h:1970)
   HIPCHK(launch_mlt_resolve(CH.img, 3 * n_pix, P.sensor_response * 0.25, d_out, as_f64, st));
-  uint64_t c[CTR_COUNT];
-  HIPCHK(hipMemcpyAsync(c, ctr, sizeof(c), hipMemcpyDeviceToHost, st));
+  uint64_t raw[CTR_WORDS], c[CTR_COUNT];
+  HIPCHK(hipMemcpyAsync(raw, ctr, sizeof(raw), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  sum_counters(raw, c);
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
   if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])

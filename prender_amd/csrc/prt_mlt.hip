@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void k_mlt_step(MltChains C, const uint64_t* _
     }
   }
   const uint64_t n_acc = __popcll(__ballot(acc));
-  if (lane_id() == 0 && n_acc) atomicAdd((unsigned long long*)&ctr[CTR_MLT_ACCEPT], (unsigned long long)n_acc);
+  if (lane_id() == 0) ctr_add(ctr, CTR_MLT_ACCEPT, n_acc);
 }
 
 __global__ __launch_bounds__(256) void k_mlt_resolve(const uint64_t* __restrict__ img, int64_t n, double scale,
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void k_erpt_step(ErptChains C, const uint64_t*
     if (run < ERPT_MAX_STACK && l > 0.0) splat(C.img, py, C.dep / l, fy);
   }
   const uint64_t n_acc = __popcll(__ballot(acc));
-  if (lane_id() == 0 && n_acc) atomicAdd((unsigned long long*)&ctr[CTR_MLT_ACCEPT], (unsigned long long)n_acc);
+  if (lane_id() == 0) ctr_add(ctr, CTR_MLT_ACCEPT, n_acc);
 }
 
 inline unsigned grid_of(uint64_t n, unsigned block = 256) { return (unsigned)((n + block - 1) / block); }

@@ -373,9 +373,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   const uint64_t s_ext = wave_sum_u32(n_ext), s_pick = wave_sum_u32(pickups), s_trunc = wave_sum_u32(truncated);
   const uint64_t s_drop = wave_sum_u32(dropped);
   if (lane == 0) {
-    auto count = [&](int c, uint64_t v) {
-      if (v) atomicAdd((unsigned long long*)&st.ctr[c], (unsigned long long)v);
-    };
+    auto count = [&](int c, uint64_t v) { ctr_add(st.ctr, c, v); };
     count(CTR_QUEUED, s_prim + s_ext);
     count(CTR_TRACED, s_tr);
     count(CTR_SHADOW, s_sh);

@@ -138,7 +138,7 @@ struct Stream {
                             // the shadow launches of queue parity 0 and 1
   StreamCtl* ctl;
   uint64_t* accum;          // [n_slots << tile_shift][3] fixed point
-  uint64_t* ctr;            // [CTR_COUNT]
+  uint64_t* ctr;            // [CTR_WORDS]
   int32_t n_scenes, n_tiles, n_slots, tile_shift;
   uint32_t slab_ray;        // entries per shade slab
   uint32_t slab_sh;         // entries per NEE slab
@@ -163,7 +163,7 @@ struct Persist {
   uint32_t* next;               // claim counter: first chunk not yet handed out, (waves * claim) at the start
   uint64_t* accum;              // [all samples][3] fixed point, zero at the start
   PoolRec* pool;                // [grid waves][PRT_PATH_POOL] (unused without glass)
-  uint64_t* ctr;                // [CTR_COUNT]
+  uint64_t* ctr;                // [CTR_WORDS]
   float* const* out_rgb;        // [n_scenes] W*H*3 device images
   float* const* out_var;        // [n_scenes] (entries may be null)
   uint32_t n_chunks;

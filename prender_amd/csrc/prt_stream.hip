@@ -377,11 +377,10 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
   const uint64_t s_ext = wave_sum_u32(C.n_ext), s_drop = wave_sum_u32(C.dropped);
   if (lane_id() == 0) {
     st.ray_nruns[wave] = log.n < st.max_runs ? log.n : st.max_runs;
-    if (s_pick) atomicAdd((unsigned long long*)&st.ctr[CTR_PICKUP], (unsigned long long)s_pick);
-    if (s_tr) atomicAdd((unsigned long long*)&st.ctr[CTR_TRUNC], (unsigned long long)s_tr);
-    if (s_ext) atomicAdd((unsigned long long*)&st.ctr[CTR_EXT], (unsigned long long)s_ext);
-    if (s_drop + log.dropped)
-      atomicAdd((unsigned long long*)&st.ctr[CTR_DROP], (unsigned long long)(s_drop + log.dropped));
+    ctr_add(st.ctr, CTR_PICKUP, s_pick);
+    ctr_add(st.ctr, CTR_TRUNC, s_tr);
+    ctr_add(st.ctr, CTR_EXT, s_ext);
+    ctr_add(st.ctr, CTR_DROP, s_drop + log.dropped);
   }
 }
 
@@ -463,7 +462,7 @@ __global__ __launch_bounds__(256) void k_stream_index(Stream st, int which) {
     }
   }
   const uint64_t s_lost = wave_sum_u32(lost);
-  if (lane == 0 && s_lost) atomicAdd((unsigned long long*)&st.ctr[CTR_DROP], (unsigned long long)s_lost);
+  if (lane == 0) ctr_add(st.ctr, CTR_DROP, s_lost);
   if (totals && tid == 0) {
     StreamCtl* c = st.ctl;
     const uint32_t n_ch = min(sum_ch, max_desc);
@@ -558,9 +557,8 @@ __global__ __launch_bounds__(256) void k_stream_nee(Stream st, RayQ q, int nxt, 
   const uint64_t s_sh = wave_sum_u32(emitted), s_drop = wave_sum_u32(dropped);
   if (lane_id() == 0) {
     st.sh_nruns[wave] = log.n < st.max_runs ? log.n : st.max_runs;
-    if (s_sh) atomicAdd((unsigned long long*)&st.ctr[CTR_SHADOW], (unsigned long long)s_sh);
-    if (s_drop + log.dropped)
-      atomicAdd((unsigned long long*)&st.ctr[CTR_DROP], (unsigned long long)(s_drop + log.dropped));
+    ctr_add(st.ctr, CTR_SHADOW, s_sh);
+    ctr_add(st.ctr, CTR_DROP, s_drop + log.dropped);
   }
 }
 

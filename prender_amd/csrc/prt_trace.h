@@ -630,8 +630,8 @@ __device__ __forceinline__ void flush_stats(uint64_t* ctr, int idx_nodes, TravSt
   const uint64_t n = wave_sum_u32(ts.nodes), t = wave_sum_u32(ts.tris);
   const uint64_t r = idx_rays >= 0 ? wave_sum_u32(ts.rays) : 0;
   if (lane_id() == 0) {
-    if (n) atomicAdd((unsigned long long*)&ctr[idx_nodes], (unsigned long long)n);
-    if (t) atomicAdd((unsigned long long*)&ctr[idx_nodes + 1], (unsigned long long)t);
-    if (r) atomicAdd((unsigned long long*)&ctr[idx_rays], (unsigned long long)r);
+    ctr_add(ctr, idx_nodes, n);
+    ctr_add(ctr, idx_nodes + 1, t);
+    ctr_add(ctr, idx_rays, r);
   }
 }
