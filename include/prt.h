@@ -198,7 +198,7 @@ typedef struct prt_render_opts {
     int32_t timing;            /* 1 = per-kernel device timing into prt_stats */
     int32_t image_f64;         /* 1 = out_rgb / out_var are double arrays (device entry points) */
     int32_t engine;            /* 0 = auto: scenes without next-event estimation and small
-                                  frames (up to 2^20 camera samples, 3 * 2^20 with glass)
+                                  frames (up to 3 * 2^17 camera samples, 2^21 with glass)
                                   render in one launch that follows each sample's whole
                                   path, larger frames with glass stream through the
                                   batched renderer's tile queue, others run
@@ -376,7 +376,8 @@ typedef struct prt_batch_opts {
                                    The images are the same bit for bit in every mode. */
     int32_t persist_waves;      /* waves per SIMD the persistent kernel's registers are budgeted for
                                    (2..4) in modes 1 and 2; 0 = mode 1: trav_blocks_per_cu if given, else 3
-                                   for batches that fill them (2 below that) */
+                                   for batches that fill them (2 below that).  Launches with light sampling
+                                   run at 2, others at most at 3 */
 } prt_batch_opts;
 /* d_rgb[i] / d_var[i]: W_i*H_i*3 float device buffers of scene i (d_var or
  * its entries may be NULL).  All scenes must live on one device; the call

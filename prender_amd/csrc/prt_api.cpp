@@ -555,7 +555,7 @@ static int trace_device(prt_scene* s, const prt_ray* d_rays, int64_t n, prt_hit*
   HIPCHK(hipEventRecord(e0.e, s->stream));
   if (n > 0)
     HIPCHK(launch_trace(s->P, (const prt_ray_dev*)d_rays, n, (prt_hit_dev*)d_hits, (uint64_t*)s->pool->ws.ctr.p,
-                        s->max_trav_blocks, s->stream));
+                        std::max(1, s->cu_count), s->stream));
   HIPCHK(hipEventRecord(e1.e, s->stream));
   uint64_t raw[CTR_WORDS], c[CTR_COUNT];
   HIPCHK(hipMemcpyAsync(raw, s->pool->ws.ctr.p, sizeof(raw), hipMemcpyDeviceToHost, s->stream));
@@ -594,8 +594,8 @@ int prt_trace_closest_device_noalloc(prt_scene* s, const prt_ray* d_rays, int64_
   HIPCHK(noalloc_scratch(s->device, &ctr));
   HIPCHK(launch_fill_u64(ctr, 0, CTR_WORDS, s->stream));
   if (n > 0)
-    HIPCHK(launch_trace(s->P, (const prt_ray_dev*)d_rays, n, (prt_hit_dev*)d_hits, ctr, s->max_trav_blocks,
-                        s->stream));
+    HIPCHK(launch_trace(s->P, (const prt_ray_dev*)d_rays, n, (prt_hit_dev*)d_hits, ctr,
+                        std::max(1, s->cu_count), s->stream));
   uint64_t raw[CTR_WORDS], c[CTR_COUNT];
   HIPCHK(hipMemcpyAsync(raw, ctr, sizeof(raw), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
@@ -739,26 +739,27 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 // Largest batches of scenes with next-event estimation that the path kernel
 // traces alone (camera samples), and the queue size at which it takes over a
 // batch's tail (rays).  A depth-synchronous depth or a tile-queue iteration
-// costs two traversal launches of 70 to 130 us each, however few its rays; the
-// path kernel pays no launch per depth, but its waves wait for their slowest
-// ray in every trip.  Measured (path kernel / queued engine, ms): mesh box, 0.6 M
-// samples 3.4 / 4.5, 0.8 M 4.4 / 5.2, 1.05 M 5.5 / 5.6 and 6.0 / 6.1 (5k and 82k
-// triangles); glass, where the tile queue drains through long tails, spheres 2.1 M
-// 4.0 / 7.7, spheres and 20k triangles 3.1 M 11.4 / 16.9, field of 400k triangles
-// 2.5 M 5.0 / 5.9.
+// costs two traversal launches however few its rays; the path kernel pays no
+// launch per depth, but its waves wait for their slowest ray in every trip.
+// Measured (path kernel / queued engine, ms): mesh box, 0.13 M samples 0.90 /
+// 1.96, 0.15 M 0.93 / 2.04, 0.6 M 3.2 / 2.8, 1.05 M 5.1 / 3.7; with glass, where the
+// tile queue drains through long tails, spheres 2.1 M 4.0 / 6.3, spheres and 60k
+// triangles 2.6 M 8.8 / 11.5, 4.2 M 14.5 / 14.4, field of 200k triangles 1.6 M 3.1
+// / 3.4, of 400k 2.5 M 4.7 / 4.5.
 #ifndef PRT_PATH_SAMPLES
-#define PRT_PATH_SAMPLES (1 << 20)
+#define PRT_PATH_SAMPLES (3 << 17)
 #endif
 #ifndef PRT_PATH_SAMPLES_GLASS
-#define PRT_PATH_SAMPLES_GLASS (3 << 20)
+#define PRT_PATH_SAMPLES_GLASS (1 << 21)
 #endif
 #ifndef PRT_PATH_TAIL
 #define PRT_PATH_TAIL (1 << 16)
 #endif
 
-extern "C++" PathGrid prt::path_grid(int cu_count, int waves, uint64_t n, bool whole_chunks) {
+extern "C++" PathGrid prt::path_grid(int cu_count, int waves, uint64_t n, bool nee, bool whole_chunks) {
   PathGrid g;
   if (waves == 0) waves = n >= (uint64_t)std::max(1, cu_count) * 2 * 256 ? 3 : 2;
+  waves = nee ? 2 : std::min(3, std::max(2, waves));  // the instances there are
   g.waves = waves;
   g.blocks = std::max(1, cu_count) * waves;  // one 256-thread block per CU puts one wave on each SIMD
   const uint64_t per_wave = (n + g.n_waves() - 1) / g.n_waves();
@@ -822,7 +823,7 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
   hipStream_t st = s->stream;
   const int64_t ns = B.n_pixels * P.spp;
   if (form == FORM_PATH || (form == FORM_AUTO && ns <= path_samples(s))) {
-    const PathGrid g = path_grid(s->cu_count, 0, (uint64_t)ns, false);
+    const PathGrid g = path_grid(s->cu_count, 0, (uint64_t)ns, P.nee && P.n_lights > 0, false);
     int rc = ensure_path_pool(w.pool, g, s->has_glass);
     if (rc) return rc;
     HIPCHK(launch_fill_u64(accum, 0ull, 3 * ns, st));
@@ -978,7 +979,7 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
       if (rays == 0) break;
       if (form == FORM_AUTO && rays <= PRT_PATH_TAIL) {
         // the rest of the batch in one launch
-        const PathGrid g = path_grid(s->cu_count, 2, rays, true);
+        const PathGrid g = path_grid(s->cu_count, 2, rays, true, true);
         if ((rc = ensure_path_pool(w.pool, g, s->has_glass))) return rc;
         if ((rc = run_path(s, PATH_QUEUE, P, B, cur, accum, g))) return rc;
         if ((rc = tm.mark(T_EXTEND))) return rc;

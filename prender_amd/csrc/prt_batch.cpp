@@ -591,10 +591,13 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
     return fail(PRT_E_INVALID, "the persistent engine takes at most 2^28 camera samples per batch (" +
                                    std::to_string(samples) + " asked)");
   const int cu = std::max(1, lead->cu_count);
-  const PathGrid grid = path_grid(cu, c.persist_waves, samples, true);
+  bool glass = false, nee = false;
+  for (int i = 0; i < n; ++i) {
+    glass |= scenes[i]->has_glass;
+    nee |= scenes[i]->P.nee && scenes[i]->P.n_lights > 0;
+  }
+  const PathGrid grid = path_grid(cu, c.persist_waves, samples, nee, true);
   const int64_t threads = (int64_t)grid.blocks * 256;
-  bool glass = false;
-  for (int i = 0; i < n; ++i) glass |= scenes[i]->has_glass;
 
   if (!lead->pool->sws) lead->pool->sws = new (std::nothrow) StreamWorkspace();
   if (!lead->pool->sws) return fail(PRT_E_NOMEM, "out of host memory");
@@ -660,7 +663,7 @@ int run_persistent(prt_scene* const* scenes, int n, const BatchConfig& c, float*
   P.quota = grid.quota;
   P.unit = 64;
   P.n_scenes = n;
-  for (int i = 0; i < n; ++i) P.nee |= scenes[i]->P.nee && scenes[i]->P.n_lights > 0;
+  P.nee = nee;
 
   ScopedEvent e0, e1, e2;
   HIPCHK(hipEventCreate(&e0.e));

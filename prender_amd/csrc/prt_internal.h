@@ -262,7 +262,7 @@ struct PathGrid {
   uint32_t unit = 64, claim = 1, quota = 64;
   uint32_t n_waves() const { return (uint32_t)blocks * 4u; }
 };
-PathGrid path_grid(int cu_count, int waves, uint64_t n, bool whole_chunks);
+PathGrid path_grid(int cu_count, int waves, uint64_t n, bool nee, bool whole_chunks);
 int ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass);
 // How run_batch may trace a batch: wavefront only, the path kernel where the
 // batch or its tail is small, or the path kernel alone.

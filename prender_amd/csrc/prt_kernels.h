@@ -144,8 +144,9 @@ struct ChunkList {
   const uint32_t* n;   // number of chunks (device)
 };
 
+// cu: compute units of the device (the stack overflow area holds 8 blocks each).
 hipError_t launch_trace(const Params& P, const prt_ray_dev* rays, int64_t n, prt_hit_dev* hits, uint64_t* ctr,
-                        int max_blocks, hipStream_t s);
+                        int cu, hipStream_t s);
 // Words of the library's file-scope device array that holds the counters of
 // the allocation-free trace entry point (one copy per GPU).
 #define PRT_NOALLOC_SCRATCH_WORDS CTR_WORDS

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "prt_device.h"
@@ -44,31 +45,45 @@ static_assert(PRT_STACK_LDS_SHADOW >= PRT_STACK_LDS_MIN, "the overflow area is s
 #define PRT_WAVES_ATTR(n) __attribute__((amdgpu_waves_per_eu((n) > 0 ? (n) : 1)))
 
 // ------------------------------------------------------------ trace API kernel
+// Closest hits of a ray array, an even share of it per wave.  Small batches are
+// bound by the latency of their slowest ray, whose lanes a wave's other rays
+// lengthen; large ones like traverse_pool.
 __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_TRAVERSE) void k_trace(
-    Params P, const prt_ray_dev* __restrict__ rays, int64_t n, prt_hit_dev* __restrict__ hits, uint64_t* ctr) {
+    Params P, const prt_ray_dev* __restrict__ rays, uint32_t n, prt_hit_dev* __restrict__ hits, uint64_t* ctr) {
   PRT_DECLARE_STACK(S, P, 0);
-  PRT_TOP_CACHE(S, P.nodes, P.n_top);
+  __shared__ AnalyticSlot s_ana[PRT_LDS_ANALYTIC];
+  const AnalyticSlot* slots = load_analytic_slots(P, s_ana);
+  PRT_TOP_CACHE(S, P.nodes, P.n_top);  // its barrier covers the slots
+  ShareSource src(P, n);
   TravStats ts{0, 0, 0};
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const prt_ray_dev r = rays[i];
-    double t, u, v;
-    int32_t id;
-    closest_hit(P, mk(r.org[0], r.org[1], r.org[2]), mk(r.dir[0], r.dir[1], r.dir[2]), t, id, u, v, S, ts);
-    prt_hit_dev h;
-    if (id >= 0) {
-      const float4* tr = reinterpret_cast<const float4*>(P.tris) + (size_t)id * 3;
-      h.entity = __float_as_int(tr[0].w);
-      h.prim = __float_as_int(tr[1].w);
-      h.t = t; h.u = u; h.v = v;
-    } else if (id <= -2) {
-      h.entity = -2 - id;
-      h.prim = -1;
-      h.t = t; h.u = -PS_INF; h.v = -PS_INF;
-    } else {
-      h.entity = -1; h.prim = -1; h.t = PS_INF; h.u = -PS_INF; h.v = -PS_INF;
-    }
-    hits[i] = h;
-  }
+  traverse_pool<false>(
+      src, slots, S, ts,
+      [&](uint32_t i, d3& o, d3& d, double& tmax) {
+        const prt_ray_dev r = rays[i];
+        o = mk(r.org[0], r.org[1], r.org[2]);
+        d = mk(r.dir[0], r.dir[1], r.dir[2]);
+        tmax = PS_INF;
+      },
+      [&](uint32_t i, double t, int32_t id, bool, d3 o, d3 d) {
+        prt_hit_dev h;
+        h.t = t;
+        h.u = h.v = -PS_INF;
+        h.entity = h.prim = -1;
+        if (id >= 0) {
+          // the barycentrics of the hit, by the same test of the same triangle
+          const float4* tr = reinterpret_cast<const float4*>(P.tris) + (size_t)id * 3;
+          const float4 a = tr[0], b = tr[1], c = tr[2];
+          double tt;
+          (void)mt_test(a, b, c, o, d, tt, h.u, h.v);
+          h.entity = __float_as_int(a.w);
+          h.prim = __float_as_int(b.w);
+        } else if (id <= -2) {
+          h.entity = -2 - id;
+        } else {
+          h.t = PS_INF;
+        }
+        hits[i] = h;
+      });
   flush_stats(ctr, CTR_NODES, ts);
 }
 
@@ -99,17 +114,19 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_TRAVERSE) void k_exte
     Params P, RayQ q, ChunkList cl, uint32_t* fetch, double* __restrict__ hit_t, int32_t* __restrict__ hit_id,
     uint64_t* ctr) {
   PRT_DECLARE_STACK(S, P, 0);
-  PRT_TOP_CACHE(S, P.nodes, P.n_top);
-  const uint32_t n_chunks = *cl.n;
+  __shared__ AnalyticSlot s_ana[PRT_LDS_ANALYTIC];
+  const AnalyticSlot* slots = load_analytic_slots(P, s_ana);
+  PRT_TOP_CACHE(S, P.nodes, P.n_top);  // its barrier covers the slots
+  ChunkSource src(P, cl, fetch);
   TravStats ts{0, 0, 0};
   traverse_pool<false>(
-      P, n_chunks, cl.desc, fetch, S, ts,
+      src, slots, S, ts,
       [&](uint32_t j, d3& o, d3& d, double& tmax) {
         o = mk(q.ox[j], q.oy[j], q.oz[j]);
         d = mk(q.dx[j], q.dy[j], q.dz[j]);
         tmax = PS_INF;
       },
-      [&](uint32_t j, double t, int32_t id, bool) {
+      [&](uint32_t j, double t, int32_t id, bool, d3, d3) {
         hit_t[j] = t;
         hit_id[j] = id;
       });
@@ -122,8 +139,10 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADOW) void k_shadow
     Params P, Batch B, ShadowQ q, ChunkList cl, uint32_t* fetch, uint64_t* __restrict__ accum, Adjoint A,
     uint64_t* ctr) {
   PRT_DECLARE_STACK_N(S, P, PRT_STACK_LDS_SHADOW, 1);
-  PRT_TOP_CACHE(S, P.nodes, P.n_top);
-  const uint32_t n_chunks = *cl.n;
+  __shared__ AnalyticSlot s_ana[PRT_LDS_ANALYTIC];
+  const AnalyticSlot* slots = load_analytic_slots(P, s_ana);
+  PRT_TOP_CACHE(S, P.nodes, P.n_top);  // its barrier covers the slots
+  ChunkSource src(P, cl, fetch);
   TravStats ts{0, 0, 0};
   double ge[3] = {0.0, 0.0, 0.0};
   auto lit = [&](uint32_t i) {
@@ -141,13 +160,13 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADOW) void k_shadow
     }
   };
   traverse_pool<true>(
-      P, n_chunks, cl.desc, fetch, S, ts,
+      src, slots, S, ts,
       [&](uint32_t j, d3& o, d3& d, double& tmax) {
         o = mk(q.ox[j], q.oy[j], q.oz[j]);
         d = mk(q.dx[j], q.dy[j], q.dz[j]);
         tmax = q.tmax[j];
       },
-      [&](uint32_t j, double, int32_t, bool blocked) {
+      [&](uint32_t j, double, int32_t, bool blocked, d3, d3) {
         if (!blocked) lit(j);
       });
   flush_stats(ctr, CTR_SNODES, ts, CTR_STRACED);
@@ -527,9 +546,24 @@ static int grid_for(int64_t n, int per_block = 256, int max_blocks = 1 << 16) {
 }
 
 hipError_t launch_trace(const Params& P, const prt_ray_dev* rays, int64_t n, prt_hit_dev* hits, uint64_t* ctr,
-                        int max_blocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_trace, dim3(grid_for(n, 256, max_blocks)), dim3(256), 0, s, P, rays, n, hits, ctr);
-  return hipGetLastError();
+                        int cu, hipStream_t s) {
+  // One ray per wave up to one block per CU, four up to two, then blocks of 64
+  // rays per wave, at most the five per CU that are resident together.  With
+  // 4 / 16 / 64 / 256 rays per block: 1,000 rays 64 / 73 / 77 / 87 us, 10,000 rays
+  // 95 / 90 / 92 / 100, 65,537 rays 122 (the grid's limit) / 122 / 107 / 104;
+  // 2^20 rays 232 us with eight blocks per CU, 201 with five.  (One lane per
+  // ray over the whole batch, without refill: 88 / 100 / 101 / 363 us.)
+  constexpr int64_t kSlice = (int64_t)1 << 30;  // ray numbers are 32-bit
+  hipError_t e = hipSuccess;
+  for (int64_t at = 0; at < n && e == hipSuccess; at += kSlice) {
+    const int64_t m = std::min(n - at, kSlice);
+    const int64_t want = std::max(std::max(std::min<int64_t>((m + 3) / 4, cu), std::min<int64_t>((m + 15) / 16, 2 * cu)),
+                                  (m + 255) / 256);
+    const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>(want, 5 * cu));
+    hipLaunchKernelGGL(k_trace, dim3(blocks), dim3(256), 0, s, P, rays + at, (uint32_t)m, hits + at, ctr);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 // Counters of prt_trace_closest_device_noalloc: a fixed device array instead

@@ -69,7 +69,17 @@ __device__ __forceinline__ double u01(uint32_t w) { return (double)w * 2.3283064
 // Per-vertex random-number counter: (pixel, sample, depth | branch << 8, block)
 __device__ __forceinline__ uint32_t rng_c2(int depth, uint32_t branch) { return ((uint32_t)depth & 0xFFu) | (branch << 8); }
 
-// Triangle::CheckIntersection2 + acceptance t > PS_EPS (polygon.h:78-166)
+// v with its sign flipped where `sign` holds a sign bit
+__device__ __forceinline__ double flip_sign(double v, uint32_t sign) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  return __longlong_as_double((long long)(((uint64_t)((uint32_t)(b >> 32) ^ sign) << 32) | (uint32_t)b));
+}
+
+// Triangle::CheckIntersection2 + acceptance t > PS_EPS (polygon.h:78-166).  The
+// reference's two orientations (det > eps, det < -eps) are one after flipping
+// the signs of det, u and v together, which rounds nothing; the bounds are
+// tested without branches, whose sides the lanes of a wave would all take
+// anyway.
 __device__ __forceinline__ bool mt_test(const float4 a, const float4 b, const float4 c, d3 o, d3 d, double& t,
                                         double& u, double& v) {
   const d3 v0 = mk(a.x, a.y, a.z);
@@ -79,26 +89,17 @@ __device__ __forceinline__ bool mt_test(const float4 a, const float4 b, const fl
   const double det = dot(edge1, p);
   const d3 tv = o - v0;
   const d3 q = cross(tv, edge1);
-  const double eps = PS_EPS * 0.1;
-  if (det > eps) {
-    u = dot(tv, p);
-    if (u < 0.0 || u > det) return false;
-    v = dot(d, q);
-    if (v < 0.0 || u + v > det) return false;
-  } else if (det < -eps) {
-    u = dot(tv, p);
-    if (u > 0.0 || u < det) return false;
-    v = dot(d, q);
-    if (v > 0.0 || u + v < det) return false;
-  } else {
-    return false;
-  }
+  u = dot(tv, p);
+  v = dot(d, q);
+  const uint32_t sign = (uint32_t)((uint64_t)__double_as_longlong(det) >> 32) & 0x80000000u;
+  const double ad = fabs(det), su = flip_sign(u, sign), sv = flip_sign(v, sign);
+  const bool out = !(ad > PS_EPS * 0.1) | (su < 0.0) | (su > ad) | (sv < 0.0) | (su + sv > ad);
+  if (out) return false;
   const double inv_det = 1.0 / det;
   t = dot(edge2, q) * inv_det;
-  if (!(t > PS_EPS)) return false;
   u *= inv_det;
   v *= inv_det;
-  return true;
+  return t > PS_EPS;
 }
 
 // sin(2 pi u) and cos(2 pi u) for u in [0, 1].  The quadrant q = rint(4u) is

@@ -26,12 +26,12 @@
 // chains in the vertices and 2,700 in 64 light samples.  So rays of one vertex
 // run side by side, few samples are spread over all waves, records that
 // every lane reads come from LDS, and scenes without light sampling have an
-// instance without it (174 instead of 228 VGPRs).  Measured against one lane
+// instance without it (173 instead of 213 VGPRs).  Measured against one lane
 // per sample that walks its glass tree and its light samples one after the
 // other, and against depth-synchronous batches: spheres 32x24 x 8 spp 834 ->
-// 175 us, 320x240 x 16 spp 1636 -> 951 us; mesh box 128x128 x 8 spp 2707 -> 946
-// us; glass with light sampling 201x151 x 27 spp 6060 -> 3036 us; Metropolis
-// steps of 15,360 chains 2.5 -> 0.43 ms.
+// 175 us, 320x240 x 16 spp 1636 -> 951 us; mesh box 128x128 x 8 spp 2707 -> 926
+// us; glass with light sampling 201x151 x 27 spp 5997 -> 3176 us; Metropolis
+// steps of 15,360 chains 2.5 -> 0.41 ms.
 //
 // A wave works on one scene at a time, so the scene's parameters are
 // wave-uniform scalar loads: a lane starts a sample of another scene only
@@ -100,30 +100,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   constexpr bool kCache = SRC != PATH_BATCH;
   __shared__ AnalyticSlot s_ana[kCache ? PRT_LDS_ANALYTIC : 1];
   __shared__ DevMaterial s_mats[kCache ? PRT_PATH_MATERIALS : 1];
+  // its lights (at most NEE_LDS_LIGHTS); in a batch each wave's scene's, if it
+  // has one light
+  __shared__ LightSlot s_lights[!NEE ? 1 : kCache ? NEE_LDS_LIGHTS : 4];
+  const LightSlot* lights = nullptr;
   const AnalyticSlot* slots = nullptr;
   const DevMaterial* lds_mats = nullptr;
   if (kCache) {
-    if (P1.n_analytic <= PRT_LDS_ANALYTIC) {
-      if ((int)threadIdx.x < P1.n_analytic) {
-        AnalyticSlot& a = s_ana[threadIdx.x];
-        a.ei = P1.analytic[threadIdx.x];
-        const DevEntity& e = P1.ents[a.ei];
-        for (int j = 0; j < 3; ++j) {
-          a.p0[j] = e.p0[j];
-          a.u_axis[j] = e.u_axis[j];
-          a.v_axis[j] = e.v_axis[j];
-          a.normal[j] = e.normal[j];
-        }
-        a.radius = e.radius;
-        a.u_len = e.u_len;
-        a.v_len = e.v_len;
-        a.ninv = e.ninv;
-      }
-      slots = s_ana;
-    }
+    slots = load_analytic_slots(P1, s_ana);
     if (P1.n_materials <= PRT_PATH_MATERIALS) {
       if ((int)threadIdx.x < P1.n_materials) s_mats[threadIdx.x] = P1.mats[threadIdx.x];
       lds_mats = s_mats;
+    }
+    if (NEE && P1.n_lights <= NEE_LDS_LIGHTS) {
+      if (threadIdx.x < 64u) load_light_slots(P1, s_lights);
+      lights = s_lights;
     }
     __syncthreads();
   }
@@ -146,12 +137,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   uint32_t cb = min(wave * st.claim, n_chunks), ce = min(cb + st.claim, n_chunks), co = 0, cn = 0;
   int32_t cs = -1, scene = SRC == PATH_BATCH ? -1 : 0;
   bool claims_left = n_chunks > gridDim.x * (blockDim.x >> 6) * st.claim;
-  UniformLight U{};
-  bool one_light = false;
-  if (SRC != PATH_BATCH) {
-    one_light = NEE && P1.n_lights == 1;
-    if (one_light) U = uniform_light(P1, P1.lights[0]);
-  }
 
   // the lane's segment
   bool act = false;
@@ -218,8 +203,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
         if (__any(act)) break;  // the wave finishes its scene's paths first
         scene = cs;
         const Params& P = scene_params(st.scenes, scene);
-        one_light = NEE && P.nee && P.n_lights == 1;
-        if (one_light) U = uniform_light(P, P.lights[0]);
+        lights = nullptr;
+        if (NEE && P.nee && P.n_lights == 1) {
+          load_light_slots(P, s_lights + wib);
+          lights = s_lights + wib;
+        }
       }
       const uint32_t take = min(min((uint32_t)__popcll(need), room), cn - co);
       const uint32_t rank = (uint32_t)__popcll(need & below);
@@ -300,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
             uint32_t w[3];
             nee_words_of(P, sp, sk, (int)(sm & 0xFFu) - 1, META_BRANCH(sm), (int)(item % 3u), w);
             int32_t l = -1;
-            shadow = one_light ? nee_one_single(U, w, 0, x, nrm, ct, sr, l) : nee_one(P, w, 0, x, nrm, ct, sr, l);
+            shadow = lights ? nee_one_slots(P, lights, w, 0, x, nrm, ct, sr, l) : nee_one(P, w, 0, x, nrm, ct, sr, l);
           }
         }
         const bool closest = first && act;
@@ -412,22 +400,20 @@ __global__ __launch_bounds__(256) void k_persist_resolve(Persist st, int64_t n_p
 }
 
 // ------------------------------------------------------------ launchers
-// 3 waves per SIMD for launches that fill them (the no-NEE instance fits 168
-// VGPRs: spheres 320x240 x 16 spp 1033 -> 951 us, glass with NEE 3260 -> 3063
-// although it spills), 2 for smaller ones, which gain nothing from more waves
-// and lose the LDS (Metropolis steps 425 -> 490 us at 3); 4 spill too much
-// (spheres 2.5 ms) and stay for callers that ask for them.
-// LDS of the instances: at 2 waves per SIMD (two blocks per CU) 12 stack
-// entries and five BVH levels, so that the tree's top costs an LDS access
-// instead of an L2 one, or for a batch of scenes, which shares no tree, 32
-// entries; at 3 waves 14 entries and four levels, or 20; at 4 waves 12 and
-// three levels.
+// Two register budgets, neither of which spills vector registers: 2 waves per
+// SIMD, and without light sampling 3 (166 VGPRs), for launches that fill them
+// (spheres 320x240 x 16 spp 1033 -> 951 us).  A smaller launch gains nothing
+// from more waves and loses the LDS.
+// LDS of the instances: at 2 waves (two blocks per CU) 12 stack entries and
+// five BVH levels, so that the tree's top costs an LDS access instead of an L2
+// one, or for a batch of scenes, which shares no tree, 32 entries; at 3 waves 14
+// entries and four levels, or 20.
 template <int SRC, bool NEE, class F>
 static hipError_t with_path_waves(int waves, F&& f) {
   constexpr bool batch = SRC == PATH_BATCH;
-  if (waves <= 2) return f(k_path<SRC, NEE, batch ? 32 : 12, batch ? PRT_TOP_NODES : PRT_WIDE_NODES, 2>);
-  if (waves == 3) return f(k_path<SRC, NEE, batch ? 20 : 14, batch ? PRT_TOP_NODES : 85, 3>);
-  return f(k_path<SRC, NEE, 12, PRT_TOP_NODES, 4>);
+  if constexpr (!NEE)
+    if (waves >= 3) return f(k_path<SRC, NEE, batch ? 20 : 14, batch ? PRT_TOP_NODES : 85, 3>);
+  return f(k_path<SRC, NEE, batch ? 32 : 12, batch ? PRT_TOP_NODES : PRT_WIDE_NODES, 2>);
 }
 template <class F>
 static hipError_t with_path_kernel(PathSource src, bool nee, int waves, F&& f) {

@@ -184,8 +184,9 @@ enum PathSource {
   PATH_FRAME = 1,  // the camera samples of one scene (or its Metropolis proposals), unit per chunk
   PATH_QUEUE = 2   // the rays of a queue, whose vertices have had their light samples
 };
-// waves: waves per SIMD its registers are budgeted for (2..4).  P: the scene
-// of a frame or queue.
+// waves: waves per SIMD to budget its registers for (2, or 3 without light
+// sampling; launches with light sampling take 2).  P: the scene of a frame or
+// queue.
 hipError_t launch_path(PathSource src, const Persist& p, const Params& P, int waves, int blocks, hipStream_t s);
 hipError_t launch_persist_resolve(const Persist& p, int64_t n_pixels_total, const int64_t* d_pixel_base,
                                   hipStream_t s);

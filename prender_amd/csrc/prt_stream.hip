@@ -21,10 +21,6 @@
 
 __device__ __forceinline__ uint32_t round64(uint32_t n) { return (n + 63u) & ~63u; }
 
-// chunks per claim of the traversal kernels
-#define FETCH_CHUNKS 2u
-
-
 // Chunk c of a chunk list (c wave-uniform), read with scalar loads.
 __device__ __forceinline__ ChunkDesc chunk_at(const ChunkDesc* list, uint32_t c) {
   const uint64_t a = (uint64_t)(list + c);
@@ -32,6 +28,38 @@ __device__ __forceinline__ ChunkDesc chunk_at(const ChunkDesc* list, uint32_t c)
                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
   return *(const ChunkDesc*)(const __attribute__((address_space(4))) ChunkDesc*)au;
 }
+
+// Chunks claimed from a chunk list whose chunks belong to several scenes: a
+// wave takes a chunk of another scene once it holds no ray of the last one.
+struct StreamSource {
+  const Params* scenes;
+  const ChunkDesc* desc;
+  ClaimRange cr;
+  uint32_t c, c1;
+  int32_t scene;
+  bool more;
+  __device__ __forceinline__ StreamSource(const Params* p, const ChunkDesc* d, uint32_t* fetch, uint32_t n_chunks)
+      : scenes(p), desc(d), cr(claim_range(fetch, n_chunks)), c(0), c1(0), scene(0), more(cr.b < cr.e) {}
+  __device__ __forceinline__ const Params& params() const { return scene_params(scenes, scene); }
+  __device__ __forceinline__ bool next(uint32_t& base, uint32_t& n, bool idle) {
+    if (c >= c1) {
+      if (!more || !claim(cr, (uint32_t)PRT_FETCH_RAYS / 64u, c, c1)) {
+        more = false;
+        return false;
+      }
+      more = c1 < cr.e;
+    }
+    const ChunkDesc d = chunk_at(desc, c);
+    if (d.scene != scene) {
+      if (!idle) return false;
+      scene = d.scene;
+    }
+    ++c;
+    base = d.base;
+    n = d.cnt;
+    return true;
+  }
+};
 
 // Adds delta to the live-ray count of tile slot ts (one atomic per distinct
 // slot of the wave, without a return value, so no wave waits on it).  A ray's
@@ -265,26 +293,24 @@ template <int NL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PRT_STREAM_WAVES(NL)))) void k_stream_extend(Stream st, RayQ q, int cur, double* __restrict__ hit_t,
                                                        int32_t* __restrict__ hit_id) {
   PRT_DECLARE_STACK_N(S, st.scenes[0], NL, 0);
-  // the top-level node copy serves a batch of one scene only
+  // the LDS copies of analytic entities and top-level nodes serve a batch of one
+  // scene only
+  __shared__ AnalyticSlot s_ana[PRT_LDS_ANALYTIC];
+  const AnalyticSlot* slots = st.n_scenes == 1 ? load_analytic_slots(st.scenes[0], s_ana) : nullptr;
   PRT_TOP_CACHE(S, st.scenes[0].nodes, st.n_scenes == 1 ? st.scenes[0].n_top : 0);
-  const ChunkDesc* desc = st.desc[cur];
-  const ClaimRange cr = claim_range(st.fetch, st.ctl->ext_chunks);
+  StreamSource src(st.scenes, st.desc[cur], st.fetch, st.ctl->ext_chunks);
   TravStats ts{0, 0, 0};
-  uint32_t c, c1;
-  while (claim(cr, FETCH_CHUNKS, c, c1)) {
-    for (; c < c1; ++c) {
-      const ChunkDesc dc = chunk_at(desc, c);
-      const Params& P = scene_params(st.scenes, dc.scene);
-      if (lane_id() < dc.cnt) {
-        const uint32_t i = dc.base + lane_id();
-        double t, u, v;
-        int32_t id;
-        closest_hit(P, mk(q.ox[i], q.oy[i], q.oz[i]), mk(q.dx[i], q.dy[i], q.dz[i]), t, id, u, v, S, ts);
+  traverse_pool<false>(
+      src, slots, S, ts,
+      [&](uint32_t i, d3& o, d3& d, double& tmax) {
+        o = mk(q.ox[i], q.oy[i], q.oz[i]);
+        d = mk(q.dx[i], q.dy[i], q.dz[i]);
+        tmax = PS_INF;
+      },
+      [&](uint32_t i, double t, int32_t id, bool, d3, d3) {
         hit_t[i] = t;
         hit_id[i] = id;
-      }
-    }
-  }
+      });
   flush_stats(st.ctr, CTR_NODES, ts);
 }
 
@@ -568,26 +594,28 @@ template <int NL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PRT_STREAM_WAVES(NL)))) void k_stream_shadow(
     Stream st, ShadowQ sq, int par) {
   PRT_DECLARE_STACK_N(S, st.scenes[0], NL, 1);
+  // the LDS copies of analytic entities and top-level nodes serve a batch of one
+  // scene only
+  __shared__ AnalyticSlot s_ana[PRT_LDS_ANALYTIC];
+  const AnalyticSlot* slots = st.n_scenes == 1 ? load_analytic_slots(st.scenes[0], s_ana) : nullptr;
   PRT_TOP_CACHE(S, st.scenes[0].nodes, st.n_scenes == 1 ? st.scenes[0].n_top : 0);
-  const ClaimRange cr =
-      claim_range(st.fetch + (size_t)(1 + par) * PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE, st.ctl->sh_chunks);
+  StreamSource src(st.scenes, st.sh_desc, st.fetch + (size_t)(1 + par) * PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE,
+                   st.ctl->sh_chunks);
   TravStats ts{0, 0, 0};
-  uint32_t c, c1;
-  while (claim(cr, FETCH_CHUNKS, c, c1)) {
-    for (; c < c1; ++c) {
-      const ChunkDesc dc = chunk_at(st.sh_desc, c);
-      const Params& P = scene_params(st.scenes, dc.scene);
-      if (lane_id() < dc.cnt) {
-        const uint32_t i = dc.base + lane_id();
+  traverse_pool<true>(
+      src, slots, S, ts,
+      [&](uint32_t i, d3& o, d3& d, double& tmax) {
+        o = mk(sq.ox[i], sq.oy[i], sq.oz[i]);
+        d = mk(sq.dx[i], sq.dy[i], sq.dz[i]);
+        tmax = sq.tmax[i];
+      },
+      [&](uint32_t i, double, int32_t, bool blocked, d3, d3) {
+        if (blocked) return;
         const uint32_t slot = sq.slot[i];
-        if (!occluded(P, mk(sq.ox[i], sq.oy[i], sq.oz[i]), mk(sq.dx[i], sq.dy[i], sq.dz[i]), sq.tmax[i], S, ts)) {
-          accum_add(&st.accum[3 * (size_t)slot + 0], sq.cr[i]);
-          accum_add(&st.accum[3 * (size_t)slot + 1], sq.cg[i]);
-          accum_add(&st.accum[3 * (size_t)slot + 2], sq.cb[i]);
-        }
-      }
-    }
-  }
+        accum_add(&st.accum[3 * (size_t)slot + 0], sq.cr[i]);
+        accum_add(&st.accum[3 * (size_t)slot + 1], sq.cg[i]);
+        accum_add(&st.accum[3 * (size_t)slot + 2], sq.cb[i]);
+      });
   flush_stats(st.ctr, CTR_SNODES, ts);
 }
 

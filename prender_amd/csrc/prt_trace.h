@@ -108,17 +108,24 @@ __device__ __forceinline__ uint32_t entry_rows(float ix, float iy, float iz) {
   return (ix < 0.0f ? 48u : 0u) | ((iy < 0.0f ? 64u : 16u) << 8) | ((iz < 0.0f ? 80u : 32u) << 16);
 }
 
+// 1 / d for the float slab test, to float accuracy (an approximate reciprocal
+// and one Newton step instead of a division); where that overflows, +-1e30.
+__device__ __forceinline__ float ray_inverse(double d) {
+  const double y = __builtin_amdgcn_rcp(d);
+  const float i = (float)__builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+  return fabsf(i) < __builtin_inff() ? i : __builtin_copysignf(1.0e30f, (float)d);
+}
+
 // Slab test of the 4 children of node `cur` against the ray's float slabs:
 // entry distances sorted ascending with their child references (+inf: miss).
 // Each axis reads its entry and exit planes from the rows entry_rows picks:
 // fma(c, i, -oi) is monotonic in the plane coordinate c and every child has
 // lo <= hi (an empty slot lo = hi = +inf), so the entry plane's distance is
 // exactly the smaller of the two, without a min / max per axis.
-// The sort is branch-free: each distance (>= 0, sign cleared so -0 sorts as
-// 0) becomes a 32-bit key whose bit pattern orders like the float, with the
-// child slot in its two low bits, and a min/max network sorts the keys.  The
-// distance read back from a key is rounded down by at most 3 ulp, so culling
-// against it stays conservative; +inf stays +inf.
+// The sort exchanges (distance, child) pairs by selects: 25 instructions,
+// where sorting 32-bit keys that carry the slot and picking the children by
+// slot afterwards took 45 (field of 2.1 M triangles 62.4 -> 61.0 ms a frame,
+// 2^20 rays 429 -> 407 us).
 // Nodes of the top levels come from the block's LDS copy.
 template <class Stk>
 __device__ __forceinline__ void node_children(const Stk& S, const DevNode* nodes, int32_t cur, uint32_t rows,
@@ -148,7 +155,6 @@ __device__ __forceinline__ void node_children(const Stk& S, const DevNode* nodes
                             __float_as_int(nd[6].w));
   const float exa[4] = {ex.x, ex.y, ex.z, ex.w}, eya[4] = {ey.x, ey.y, ey.z, ey.w}, eza[4] = {ez.x, ez.y, ez.z, ez.w};
   const float xxa[4] = {xx.x, xx.y, xx.z, xx.w}, xya[4] = {xy.x, xy.y, xy.z, xy.w}, xza[4] = {xz.x, xz.y, xz.z, xz.w};
-  uint32_t key[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const float x0 = __builtin_fmaf(exa[k], ix, -oix), x1 = __builtin_fmaf(xxa[k], ix, -oix);
@@ -156,23 +162,24 @@ __device__ __forceinline__ void node_children(const Stk& S, const DevNode* nodes
     const float z0 = __builtin_fmaf(eza[k], iz, -oiz), z1 = __builtin_fmaf(xza[k], iz, -oiz);
     const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, 0.0f));
     const float tfar = fminf(fminf(x1, y1), fminf(z1, tb));
-    const uint32_t tk = (tnear <= tfar) ? (__float_as_uint(tnear) & 0x7FFFFFFCu) : 0x7F800000u;
-    key[k] = tk | (uint32_t)k;
+    tn[k] = (tnear <= tfar) ? tnear : __builtin_inff();
   }
-#define PRT_KSORT(a, b)                                \
-  {                                                    \
-    const uint32_t lo_ = min(key[a], key[b]);          \
-    key[b] = max(key[a], key[b]);                      \
-    key[a] = lo_;                                      \
+  cc[0] = ch.x; cc[1] = ch.y; cc[2] = ch.z; cc[3] = ch.w;
+#define PRT_KSORT(a, b)                           \
+  {                                               \
+    const bool sw_ = tn[b] < tn[a];               \
+    const float t_ = sw_ ? tn[b] : tn[a];         \
+    tn[b] = sw_ ? tn[a] : tn[b];                  \
+    tn[a] = t_;                                   \
+    const int32_t c_ = sw_ ? cc[b] : cc[a];       \
+    cc[b] = sw_ ? cc[a] : cc[b];                  \
+    cc[a] = c_;                                   \
   }
-  PRT_KSORT(0, 1) PRT_KSORT(2, 3) PRT_KSORT(0, 2) PRT_KSORT(1, 3) PRT_KSORT(1, 2)
+  PRT_KSORT(0, 1) PRT_KSORT(2, 3) PRT_KSORT(0, 2) PRT_KSORT(1, 3)
+#if !defined(PRT_SORT4)
+  PRT_KSORT(1, 2)
+#endif
 #undef PRT_KSORT
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t slot = key[j] & 3u;
-    tn[j] = key[j] >= 0x7F800000u ? __builtin_inff() : __uint_as_float(key[j] & ~3u);
-    cc[j] = (slot & 2u) ? ((slot & 1u) ? ch.w : ch.z) : ((slot & 1u) ? ch.y : ch.x);
-  }
 }
 
 // Pushes children 3, 2, 1 of a sorted node test (farthest first) that were
@@ -207,6 +214,104 @@ __device__ __forceinline__ int32_t hit_entity(const float4* tris4, int32_t id) {
   return id >= 0 ? __float_as_int(tris4[(size_t)id * 3].w) : (id <= -2 ? -2 - id : 0x7FFFFFFF);
 }
 
+// The analytic entities of a scene (at most PRT_LDS_ANALYTIC) as a block
+// keeps them in LDS, spheres first.
+#define PRT_LDS_ANALYTIC 16
+struct AnalyticSlot {
+  double p0[3], radius;  // sphere; uvplane: p0
+  double u_axis[3], v_axis[3], u_len, v_len, u_max, v_max;  // uvplane
+  double normal[3];      // uvplane: with the entity's sign
+  int32_t ei, pad_;
+};
+// Copies them into slots (block-wide, a barrier follows); null if they are too
+// many.
+__device__ __forceinline__ const AnalyticSlot* load_analytic_slots(const Params& P, AnalyticSlot* slots) {
+  if (P.n_analytic > PRT_LDS_ANALYTIC) return nullptr;
+  if ((int)threadIdx.x < P.n_analytic) {
+    AnalyticSlot& a = slots[threadIdx.x];
+    a.ei = P.analytic[threadIdx.x];
+    const DevEntity& e = P.ents[a.ei];
+    const double sign = e.ninv < 0 ? -1.0 : 1.0;
+    for (int j = 0; j < 3; ++j) {
+      a.p0[j] = e.p0[j];
+      a.u_axis[j] = e.u_axis[j];
+      a.v_axis[j] = e.v_axis[j];
+      a.normal[j] = e.normal[j] * sign;
+    }
+    a.radius = e.radius;
+    a.u_len = e.u_len;
+    a.v_len = e.v_len;
+    // above these the plane coordinate's quotient by its length exceeds the
+    // length whatever its rounding
+    a.u_max = e.u_len * e.u_len * (1.0 + 1.0e-12);
+    a.v_max = e.v_len * e.v_len * (1.0 + 1.0e-12);
+  }
+  return slots;
+}
+// uvplane_t of a slot: its answer and its t.  The quotients that bound the plane
+// coordinates are formed only near the rectangle.
+__device__ __forceinline__ bool uvplane_slot(const AnalyticSlot& e, d3 o, d3 d, double& t) {
+  const d3 n2 = ld3(e.normal);
+  const double dd = dot(d, n2), num = dot(ld3(e.p0) - o, n2);
+  // behind the origin, whatever the quotient's rounding; NaN goes on
+  if (fabs(dd) < PS_EPS14 || (num < 0.0 && dd > 0.0) || (num > 0.0 && dd < 0.0)) return false;
+  t = num / dd;
+  const d3 pos = d * t + o;
+  if (t < PS_EPS) return false;
+  const d3 rel = pos - ld3(e.p0);
+  const double a = dot(rel, ld3(e.u_axis)), b = dot(rel, ld3(e.v_axis));
+  if (a < -1.0e-200 || b < -1.0e-200 || a > e.u_max || b > e.v_max) return false;
+  const double hu = a / e.u_len, hv = b / e.v_len;
+  if (hu < 0 || hu > e.u_len) return false;
+  if (hv < 0 || hv > e.v_len) return false;
+  return true;
+}
+
+// The analytic part of a ray's hit: updates a closest hit (t, id) or tells
+// whether an any hit lies below t.  slots: the scene's analytic entities in
+// LDS, or null.  The tests are chains of dependent FP64 operations run by lanes
+// that have just started a ray, so their records come from LDS instead of
+// through three dependent global loads each, and the spheres are tested
+// without branches, so that several chains overlap (nine spheres: 13,800 ->
+// 6,400 cycles).
+__device__ __forceinline__ bool analytic_hits(const Params& P, const AnalyticSlot* slots, d3 o, d3 d, bool any,
+                                              double& t, int32_t& id) {
+  bool blocked = false;
+  int32_t e_best = 0x7FFFFFFF;
+  auto meet = [&](bool hit, double tt, int32_t ei) {
+    const bool near = hit && (any ? tt < t : nearer_hit(tt, ei, t, e_best));
+    if (near && !any) {
+      t = tt;
+      id = -2 - ei;
+      e_best = ei;
+    }
+    blocked |= near && any;
+  };
+  if (slots != nullptr) {
+#pragma unroll 3
+    for (int k = 0; k < P.n_spheres; ++k) {
+      const AnalyticSlot& e = slots[k];
+      double tt;
+      const bool hit = sphere_root(ld3(e.p0), e.radius, o, d, tt);
+      meet(hit, tt, e.ei);
+    }
+    for (int k = P.n_spheres; k < P.n_analytic; ++k) {
+      const AnalyticSlot& e = slots[k];
+      double tt;
+      const bool hit = uvplane_slot(e, o, d, tt);
+      meet(hit, tt, e.ei);
+    }
+  } else {
+    for (int k = 0; k < P.n_analytic; ++k) {
+      const int32_t ei = P.analytic[k];
+      double tt;
+      const bool hit = analytic_t(P.ents[ei], o, d, tt);
+      meet(hit, tt, ei);
+    }
+  }
+  return blocked;
+}
+
 // Every triangle a ray tests is one whose box the conservative culling
 // leaves open (a box whose entry equals the best t stays open), so the
 // closest hit is the one over all triangles, with the tie rule of
@@ -219,10 +324,7 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 
                                             double& ub, double& vb, Stk& S, TravStats& ts) {
   if (P.n_nodes <= 0) return false;
   const float ox = (float)o.x, oy = (float)o.y, oz = (float)o.z;
-  float ix = (float)(1.0 / d.x), iy = (float)(1.0 / d.y), iz = (float)(1.0 / d.z);
-  if (__builtin_isinf(ix)) ix = __builtin_copysignf(1.0e30f, ix);
-  if (__builtin_isinf(iy)) iy = __builtin_copysignf(1.0e30f, iy);
-  if (__builtin_isinf(iz)) iz = __builtin_copysignf(1.0e30f, iz);
+  const float ix = ray_inverse(d.x), iy = ray_inverse(d.y), iz = ray_inverse(d.z);
   const float oix = ox * ix, oiy = oy * iy, oiz = oz * iz;
   const uint32_t rows = entry_rows(ix, iy, iz);
   float tb = t_best < 1.0e30 ? fup(t_best) : __builtin_inff();
@@ -297,93 +399,15 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 
   return found;
 }
 
-// Closest hit over analytic entities then the BVH; o_in is the ray origin
-// before the 1e-6 nudge.  id >= 0: triangle slot; id <= -2: analytic entity
-// -2-id; -1: miss.
-template <class Stk>
-__device__ __forceinline__ void closest_hit(const Params& P, d3 o_in, d3 d, double& t, int32_t& id, double& u,
-                                            double& v, Stk& S, TravStats& ts) {
-  const d3 o = o_in + d * 0.000001;
-  t = PS_INF;
-  id = -1;
-  u = v = -PS_INF;
-  for (int k = 0; k < P.n_analytic; ++k) {
-    const int32_t ei = P.analytic[k];
-    double tt;
-    if (analytic_t(P.ents[ei], o, d, tt) && nearer_hit(tt, ei, t, id <= -2 ? -2 - id : 0x7FFFFFFF)) {
-      t = tt;
-      id = -2 - ei;
-    }
-  }
-  traverse_ww(P, false, o, d, t, id, u, v, S, ts);
-}
-
-// Any blocker with t in (1e-6, tmax) from the already-nudged origin o.
-template <class Stk>
-__device__ __forceinline__ bool occluded(const Params& P, d3 o, d3 d, double tmax, Stk& S, TravStats& ts) {
-  for (int k = 0; k < P.n_analytic; ++k) {
-    double tt;
-    if (analytic_t(P.ents[P.analytic[k]], o, d, tt) && tt < tmax) return true;
-  }
-  int32_t id = -1;
-  double u, v;
-  return traverse_ww(P, true, o, d, tmax, id, u, v, S, ts);
-}
-
-// The analytic entities of a scene (at most PRT_LDS_ANALYTIC) as a block
-// keeps them in LDS, spheres first.
-#define PRT_LDS_ANALYTIC 16
-struct AnalyticSlot {
-  double p0[3], radius;                                 // sphere; uvplane: p0
-  double u_axis[3], v_axis[3], normal[3], u_len, v_len; // uvplane
-  int32_t ei, ninv;
-};
-
-// One ray per lane, closest and any hits side by side: closest_hit's hit of
-// the lanes without `any` (t, id; t enters as PS_INF), occluded's answer below
-// t of the others.  o is the already-nudged origin.  slots: the scene's
-// analytic entities in LDS, or null.
-//
-// A wave here often runs alone on its SIMD, so a test's time is the latency of
-// its chain: the records come from LDS instead of through three dependent
-// global loads, and the spheres are tested without branches, so that several
-// chains overlap (nine spheres: 13,800 -> 6,400 cycles).
+// One ray per lane (o: its already-nudged origin), closest and any hits side by
+// side.  Without `any`: the closest hit over analytic entities and the BVH, t
+// (entered as PS_INF) and id (>= 0: triangle slot; <= -2: analytic entity
+// -2 - id; -1: miss).  With it: whether anything lies in (1e-6, t).  slots: the
+// scene's analytic entities in LDS, or null.
 template <class Stk>
 __device__ __forceinline__ bool trace_lane(const Params& P, const AnalyticSlot* slots, d3 o, d3 d, bool any, double& t,
                                            int32_t& id, Stk& S, TravStats& tc, TravStats& tsh) {
-  bool blocked = false;
-  int32_t e_best = 0x7FFFFFFF;
-  auto meet = [&](bool hit, double tt, int32_t ei) {
-    const bool near = hit && (any ? tt < t : nearer_hit(tt, ei, t, e_best));
-    if (near && !any) {
-      t = tt;
-      id = -2 - ei;
-      e_best = ei;
-    }
-    blocked |= near && any;
-  };
-  if (slots != nullptr) {
-#pragma unroll 3
-    for (int k = 0; k < P.n_spheres; ++k) {
-      const AnalyticSlot& e = slots[k];
-      double tt;
-      const bool hit = sphere_root(ld3(e.p0), e.radius, o, d, tt);
-      meet(hit, tt, e.ei);
-    }
-    for (int k = P.n_spheres; k < P.n_analytic; ++k) {
-      const AnalyticSlot& e = slots[k];
-      double tt;
-      const bool hit = uvplane_t(e, o, d, tt);
-      meet(hit, tt, e.ei);
-    }
-  } else {
-    for (int k = 0; k < P.n_analytic; ++k) {
-      const int32_t ei = P.analytic[k];
-      double tt;
-      const bool hit = analytic_t(P.ents[ei], o, d, tt);
-      meet(hit, tt, ei);
-    }
-  }
+  bool blocked = analytic_hits(P, slots, o, d, any, t, id);
   if (blocked) return true;
   TravStats ts{0, 0, 0};
   double u, v;
@@ -391,6 +415,17 @@ __device__ __forceinline__ bool trace_lane(const Params& P, const AnalyticSlot* 
   (any ? tsh : tc).nodes += ts.nodes;
   (any ? tsh : tc).tris += ts.tris;
   return blocked;
+}
+
+// *p, p the same for every lane, through the scalar cache (nothing may write it
+// during the kernel).
+__device__ __forceinline__ uint2 uniform_load(const uint2* p) {
+  const uint64_t a = (uint64_t)p;
+  const uint64_t au = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32) |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  const u2 v = *(const __attribute__((address_space(4))) u2*)au;
+  return make_uint2(v.x, v.y);
 }
 
 // ------------------------------------------------ chunk claims
@@ -439,47 +474,108 @@ __device__ __forceinline__ bool claim(const ClaimRange& r, uint32_t k, uint32_t&
 
 // ------------------------------------------------ queue traversal with refill
 //
-// Closest or any hit for the rays of a chunked queue (chunk c holds desc[c].y
-// rays from queue index desc[c].x on), the while-while loop of traverse_ww
-// with lanes refilled as their rays finish.  A wave claims PRT_FETCH_RAYS /
-// 64 chunks per atomic from its claim sub-range (claim_range), keeps the
-// claimed entries not yet started as a pool, and hands
-// them to idle lanes at the top of each round once at least PRT_REFILL_MIN
-// lanes are idle.  Without refill a wave lives as long as its slowest ray
-// and the other lanes idle meanwhile.  Each ray's own traversal is
-// traverse_ww's, so its hit is the same.
+// Closest or any hit for the rays that a source hands out, with lanes
+// refilled as their rays finish: without refill a wave lives as long as its
+// slowest ray and the other lanes idle meanwhile.  Each step of a wave is a
+// node visit or a triangle test, whichever more of its lanes wait for (a node
+// visit counting PRT_VOTE_NODE times), so that both run with most lanes
+// active; a lane that has found a leaf keeps walking until it finds a second
+// one, as in traverse_ww.  Once PRT_REFILL_MIN rays have finished they are
+// handed over and their lanes take new ones.  A ray's hit is traverse_ww's.
 //
+// What bounds it: vector instructions, issued in 80 % of a SIMD's cycles, and
+// so the lanes that share each of them.  Walking until every lane holds a
+// leaf and then testing all leaves ran 23.8 lanes per node visit and 30.8 per
+// triangle test (closest hits of the 82k-triangle box); the vote runs 43 and
+// 38.  A refill is some 250 instructions at the refilled lanes only, plus the
+// reads of the new rays, so it waits for half the wave: 38.0, 37.0, 36.4 ms a
+// frame at 16, 24, 32 lanes (32, 24 and 40 are alike on other scenes).  The
+// registers have to stay within 96 for five waves per SIMD: counts are kept per
+// wave, and a hit's entity, needed only for equal distances, is read again.
+// Frame of that box 41.5 -> 34.7 ms, with the analytic entities in LDS and the
+// shorter tests; the field of 2.1 M triangles 72.8 -> 60.1 ms and the batch of
+// eight scenes 54.4 -> 42.3 ms, whose tile queue had no refill.
+//
+// Source: next(base, n, idle) gives the wave's next rays base .. base + n - 1
+// (n > 0; idle: no lane of the wave holds a ray), false when there are none
+// now; params() the scene of the rays handed out last.  Every lane of the wave
+// calls next together.
 // Load(j, o, d, tmax): ray j's origin (before the 1e-6 nudge for a closest
 // hit, already nudged for an any hit), direction and t bound.
-// Done(j, t, id, blocked): the finished ray (closest hit t / id as
-// closest_hit; any hit: blocked).
+// Done(j, t, id, blocked, o, d): the finished ray (closest hit t / id as
+// trace_lane; any hit: blocked; o the nudged origin).
 #ifndef PRT_REFILL_MIN
-#define PRT_REFILL_MIN 16
+#define PRT_REFILL_MIN 32
+#endif
+#ifndef PRT_VOTE_NODE
+#define PRT_VOTE_NODE 2
 #endif
 #ifndef PRT_FETCH_RAYS
 #define PRT_FETCH_RAYS 128
 #endif
-template <bool ANY, class Stk, class Load, class Done>
-__device__ __forceinline__ void traverse_pool(const Params& P, uint32_t n_chunks, const uint2* __restrict__ desc,
-                                              uint32_t* fetch, Stk& S, TravStats& ts, Load&& load, Done&& done) {
-  const float4* tris4 = reinterpret_cast<const float4*>(P.tris);
+
+// Chunks claimed from a chunk list (claim_range), PRT_FETCH_RAYS rays per
+// atomic.
+struct ChunkSource {
+  const Params& P;
+  const uint2* desc;
+  ClaimRange cr;
+  uint32_t c, c1;
+  bool more;
+  __device__ __forceinline__ ChunkSource(const Params& p, const ChunkList& cl, uint32_t* fetch)
+      : P(p), desc(cl.desc), cr(claim_range(fetch, *cl.n)), c(0), c1(0), more(cr.b < cr.e) {}
+  __device__ __forceinline__ const Params& params() const { return P; }
+  __device__ __forceinline__ bool next(uint32_t& base, uint32_t& n, bool) {
+    if (c >= c1) {
+      if (!more || !claim(cr, (uint32_t)PRT_FETCH_RAYS / 64u, c, c1)) {
+        more = false;
+        return false;
+      }
+      more = c1 < cr.e;
+    }
+    const uint2 d = uniform_load(desc + c);
+    ++c;
+    base = d.x;
+    n = d.y;
+    return true;
+  }
+};
+
+// An even share of the rays 0 .. n - 1 per wave of the grid, no counter.
+struct ShareSource {
+  const Params& P;
+  uint32_t b, e;
+  __device__ __forceinline__ ShareSource(const Params& p, uint32_t n) : P(p) {
+    const uint64_t wave = (uint64_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const uint32_t n_waves = (gridDim.x * blockDim.x) >> 6;
+    b = (uint32_t)(wave * n / n_waves);
+    e = (uint32_t)((wave + 1) * n / n_waves);
+  }
+  __device__ __forceinline__ const Params& params() const { return P; }
+  __device__ __forceinline__ bool next(uint32_t& base, uint32_t& n, bool) {
+    if (b >= e) return false;
+    base = b;
+    n = e - b;
+    b = e;
+    return true;
+  }
+};
+
+template <bool ANY, class Stk, class Source, class Load, class Done>
+__device__ __forceinline__ void traverse_pool(Source& src, const AnalyticSlot* slots, Stk& S, TravStats& ts, Load&& load,
+                                              Done&& done) {
   const uint32_t lane = lane_id();
   const uint64_t below = (1ull << lane) - 1ull;
-  constexpr uint32_t kClaim = (uint32_t)PRT_FETCH_RAYS / 64u;  // chunks per claim
-  const ClaimRange cr = claim_range(fetch, n_chunks);
   d3 o = mk(0.0, 0.0, 0.0), d = o;
   float ix = 0.0f, iy = 0.0f, iz = 0.0f, oix = 0.0f, oiy = 0.0f, oiz = 0.0f, tb = 0.0f;
   uint32_t rows = 0;
   double t_best = 0.0;
-  int32_t id_best = -1, e_best = 0x7FFFFFFF, cur = PRT_TRAV_DONE, lf = 0;
+  int32_t id_best = -1, cur = PRT_TRAV_DONE, lf = 0;
   int sp = 0;
   uint32_t ri = 0;
   bool act = false, blocked = false;
-  // wave-uniform: claimed entries pool_base .. pool_base + pool_n - 1 (entry
-  // g = chunk * 64 + lane slot) not yet started; more: the sub-range may hold
-  // unclaimed chunks
-  uint32_t pool_base = 0, pool_n = 0;
-  bool more = cr.b < cr.e;
+  uint32_t base = 0, left = 0;  // wave-uniform: rays handed out and not yet started
+  uint32_t n_nodes = 0, n_tris = 0, n_rays = 0;  // wave-uniform counts
   auto pop_next = [&]() -> int32_t {
     while (sp > 0) {
       int32_t node;
@@ -490,139 +586,113 @@ __device__ __forceinline__ void traverse_pool(const Params& P, uint32_t n_chunks
     return PRT_TRAV_DONE;
   };
   while (true) {
-    // ---- refill idle lanes
+    // ---- idle lanes take new rays
     const uint64_t idle = __ballot(!act);
     const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= (uint32_t)PRT_REFILL_MIN && (pool_n > 0 || more)) {
+    if (n_idle >= (uint32_t)PRT_REFILL_MIN) {
       const uint32_t rank = (uint32_t)__popcll(idle & below);
-      const uint32_t take = n_idle < pool_n ? n_idle : pool_n;
-      int64_t g = -1;
-      if (!act && rank < take) g = pool_base + rank;
-      pool_base += take;
-      pool_n -= take;
-      if (n_idle > take && more) {
-        uint32_t c0, c1;
-        if (!claim(cr, kClaim, c0, c1)) {
-          more = false;
-        } else {
-          const uint32_t ent = (c1 - c0) * 64u;
-          const uint32_t need = n_idle - take, used = need < ent ? need : ent;
-          if (!act && rank >= take && rank - take < ent) g = c0 * 64u + (rank - take);
-          pool_base = c0 * 64u + used;
-          pool_n = ent - used;
-          if (c1 >= cr.e) more = false;
+      uint32_t got = 0;
+      bool has = false;
+      while (got < n_idle) {
+        if (left == 0 && !src.next(base, left, n_idle == 64u && got == 0u)) break;
+        const uint32_t take = min(n_idle - got, left);
+        if (!act && rank >= got && rank < got + take) {
+          ri = base + (rank - got);
+          has = true;
+        }
+        base += take;
+        left -= take;
+        got += take;
+      }
+      if (got == 0u && n_idle == 64u) break;  // nothing running and nothing left
+      if (has) {
+        // analytic entities first
+        const Params& P = src.params();
+        act = true;
+        load(ri, o, d, t_best);
+        if (!ANY) o = o + d * 0.000001;
+        id_best = -1;
+        blocked = analytic_hits(P, slots, o, d, ANY, t_best, id_best);
+        lf = 0;
+        sp = 0;
+        cur = PRT_TRAV_DONE;
+        if (!blocked && P.n_nodes > 0) {
+          ix = ray_inverse(d.x);
+          iy = ray_inverse(d.y);
+          iz = ray_inverse(d.z);
+          oix = (float)o.x * ix;
+          oiy = (float)o.y * iy;
+          oiz = (float)o.z * iz;
+          rows = entry_rows(ix, iy, iz);
+          tb = t_best < 1.0e30 ? fup(t_best) : __builtin_inff();
+          cur = 0;
         }
       }
-      if (g >= 0) {
-        const uint2 dc = desc[(uint32_t)g >> 6];
-        if (((uint32_t)g & 63u) < dc.y) {
-          // start ray ri: analytic entities first, as closest_hit / occluded
-          ri = dc.x + ((uint32_t)g & 63u);
-          act = true;
-          blocked = false;
-          d3 oo;
-          double tmax;
-          load(ri, oo, d, tmax);
-          o = ANY ? oo : oo + d * 0.000001;
-          t_best = tmax;
-          id_best = -1;
-          e_best = 0x7FFFFFFF;
-          for (int k = 0; k < P.n_analytic; ++k) {
-            const int32_t ei = P.analytic[k];
-            double tt;
-            if (analytic_t(P.ents[ei], o, d, tt) && (ANY ? tt < t_best : nearer_hit(tt, ei, t_best, e_best))) {
-              if (ANY) {
-                blocked = true;
-                break;
-              }
-              t_best = tt;
-              id_best = -2 - ei;
-              e_best = ei;
+    }
+    const Params& P = src.params();
+    const float4* tris4 = reinterpret_cast<const float4*>(P.tris);
+    // ---- node and triangle steps until enough rays have finished
+    while (true) {
+      const bool walk = (uint32_t)cur < (uint32_t)PRT_TRAV_DONE;
+      const uint32_t nw = (uint32_t)__popcll(__ballot(walk)), nl = (uint32_t)__popcll(__ballot(lf < 0));
+      if (nw + nl == 0u) break;
+      if (nw * (uint32_t)PRT_VOTE_NODE >= nl) {
+        n_nodes += nw;
+        if (walk) {
+          float tn[4];
+          int32_t cc[4];
+          node_children(S, P.nodes, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, tn, cc);
+          push_children(S, sp, tn, cc);
+          cur = (tn[0] != __builtin_inff()) ? cc[0] : pop_next();
+          if (cur < 0 && lf >= 0) {  // park the first leaf and keep walking
+            lf = cur;
+            cur = pop_next();
+          }
+        }
+      } else {
+        n_tris += nl;
+        if (lf < 0) {
+          const uint32_t code = ~(uint32_t)lf;
+          const uint32_t tri = code & 0x07FFFFFFu;
+          const float4* tr = tris4 + (size_t)tri * 3;
+          const float4 a = tr[0], b = tr[1], c = tr[2];
+          double t, u, v;
+          if (mt_test(a, b, c, o, d, t, u, v) &&
+              (ANY ? t < t_best
+                   : (t < t_best || (t == t_best && __float_as_int(a.w) < hit_entity(tris4, id_best))))) {
+            if (ANY) {
+              blocked = true;
+            } else {
+              t_best = t;
+              id_best = (int32_t)tri;
+              tb = fup(t);
             }
           }
-          lf = 0;
-          sp = 0;
-          cur = PRT_TRAV_DONE;
-          if (!blocked && P.n_nodes > 0) {
-            ix = (float)(1.0 / d.x);
-            iy = (float)(1.0 / d.y);
-            iz = (float)(1.0 / d.z);
-            if (__builtin_isinf(ix)) ix = __builtin_copysignf(1.0e30f, ix);
-            if (__builtin_isinf(iy)) iy = __builtin_copysignf(1.0e30f, iy);
-            if (__builtin_isinf(iz)) iz = __builtin_copysignf(1.0e30f, iz);
-            oix = (float)o.x * ix;
-            oiy = (float)o.y * iy;
-            oiz = (float)o.z * iz;
-            rows = entry_rows(ix, iy, iz);
-            tb = t_best < 1.0e30 ? fup(t_best) : __builtin_inff();
-            cur = 0;
+          if (ANY && blocked) {
+            lf = 0;
+            cur = PRT_TRAV_DONE;
+          } else if ((code >> 27) != 0u) {
+            lf = (int32_t)~(code + 1u - (1u << 27));  // the leaf's next triangle
+          } else {
+            lf = cur < 0 ? cur : 0;  // a second leaf met while walking
+            if (cur < 0) cur = pop_next();
           }
         }
       }
-    }
-    if (!__any(act)) {
-      if (pool_n == 0 && !more) break;  // nothing running and nothing left to start
-      continue;                         // the claimed entries were padding
-    }
-    // ---- walk internal nodes until every walking lane holds a leaf
-    while ((uint32_t)cur < (uint32_t)PRT_TRAV_DONE) {
-      float tn[4];
-      int32_t cc[4];
-      node_children(S, P.nodes, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, tn, cc);
-      ts.nodes++;
-      push_children(S, sp, tn, cc);
-      cur = (tn[0] != __builtin_inff()) ? cc[0] : pop_next();
-      if (cur < 0 && lf >= 0) {
-        lf = cur;
-        cur = pop_next();
-      }
-      if (!__any(lf >= 0)) break;
-    }
-    // ---- test the parked leaves (triangle k + 1 is loaded before triangle k
-    // is tested, so a leaf costs one memory round trip rather than one per
-    // triangle)
-    while (lf < 0) {
-      const uint32_t code = ~(uint32_t)lf;
-      const uint32_t first = code & 0x07FFFFFFu;
-      const uint32_t count = (code >> 27) + 1u;
-      const float4* tr0 = tris4 + (size_t)first * 3;
-      float4 na = tr0[0], nb = tr0[1], nc = tr0[2];
-      for (uint32_t k = 0; k < count; ++k) {
-        const float4 a = na, b = nb, c = nc;
-        if (k + 1 < count) {
-          const float4* tr = tris4 + (size_t)(first + k + 1) * 3;
-          na = tr[0];
-          nb = tr[1];
-          nc = tr[2];
-        }
-        ts.tris++;
-        double t, u, v;
-        if (mt_test(a, b, c, o, d, t, u, v) &&
-            (ANY ? t < t_best : nearer_hit(t, __float_as_int(a.w), t_best, e_best))) {
-          if (ANY) {
-            blocked = true;
-            break;
-          }
-          t_best = t;
-          id_best = (int32_t)(first + k);
-          e_best = __float_as_int(a.w);
-          tb = fup(t);
-        }
-      }
-      if (ANY && blocked) {
-        lf = 0;
-        cur = PRT_TRAV_DONE;
-      } else {
-        lf = cur;
-        if (cur < 0) cur = pop_next();
-      }
+      if ((uint32_t)__popcll(__ballot(act && cur == PRT_TRAV_DONE && lf >= 0)) >= (uint32_t)PRT_REFILL_MIN) break;
     }
     // ---- hand over finished rays
-    if (act && cur == PRT_TRAV_DONE && lf >= 0) {
-      done(ri, t_best, id_best, blocked);
+    const bool fin = act && cur == PRT_TRAV_DONE && lf >= 0;
+    n_rays += (uint32_t)__popcll(__ballot(fin));
+    if (fin) {
+      done(ri, t_best, id_best, blocked, o, d);
       act = false;
-      ts.rays++;
     }
+  }
+  if (lane == 0) {
+    ts.nodes += n_nodes;
+    ts.tris += n_tris;
+    ts.rays += n_rays;
   }
 }
 
