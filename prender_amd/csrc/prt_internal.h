@@ -13,6 +13,7 @@
 #include "../../include/prt.h"
 #include "prt_device.h"
 #include "prt_kernels.h"
+#include "prt_mlt.h"
 
 namespace prt {
 
@@ -271,6 +272,11 @@ enum BatchForm { FORM_WAVEFRONT = 0, FORM_AUTO = 1, FORM_PATH = 2 };
 // sample radiance accumulates into accum (fixed point).
 int run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, BatchForm form,
               Timer& tm, CallTotals& tot);
+// Whether n Markov chains of the scene run each at their own pace (run_chains),
+// not step by step as batches; steps steps of them.  P.mlt_u: their proposals.
+bool chains_async(const prt_scene* s, uint32_t n);
+int run_chains(prt_scene* s, const Params& P, const ChainRun& R, uint32_t n, uint32_t steps, Timer& tm,
+               CallTotals& tot);
 
 }  // namespace prt
 

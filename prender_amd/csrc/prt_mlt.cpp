@@ -34,8 +34,9 @@ uint64_t splitmix64(uint64_t x) {
 
 // Philox key of one random stream of a render: phase 1 = seed-path batch
 // `idx`, 2 = chain step `idx`, 3 = chain control.
+uint64_t mlt_phase(uint64_t seed, uint64_t phase) { return splitmix64(seed ^ (phase * 0xA0761D6478BD642Full)); }
 void mlt_key(uint64_t seed, uint64_t phase, uint64_t idx, uint32_t& k0, uint32_t& k1) {
-  const uint64_t h = splitmix64(splitmix64(seed ^ (phase * 0xA0761D6478BD642Full)) + idx);
+  const uint64_t h = splitmix64(mlt_phase(seed, phase) + idx);
   k0 = (uint32_t)h;
   k1 = (uint32_t)(h >> 32);
 }
@@ -140,12 +141,23 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
     HIPCHK(launch_mlt_init(CH, SD, st));
     const double weight = 4.0 * (double)n_pix;  // generate_new_path pdf: W*H, x4 for the tent filter
     const double inv_m = 1.0 / (double)m.steps;
-    for (int64_t it = 0; it < m.steps; ++it) {
-      HIPCHK(launch_mlt_mutate(CH, 1, 0u, C, (uint32_t)it, m.p_large, st));
-      Params Pi = P;
-      mlt_key(opts.seed, 2, (uint64_t)it, Pi.key0, Pi.key1);
-      if ((rc = run_batch(s, Pi, Batch{0, C}, accum, none, FORM_AUTO, tm, tot))) return rc;
-      HIPCHK(launch_mlt_step(CH, accum, (uint32_t)it, m.p_large, b, weight, inv_m, ctr, st));
+    if (chains_async(s, C)) {
+      ChainRun R{};
+      R.mlt = CH;
+      R.p_large = m.p_large;
+      R.b = b;
+      R.weight = weight;
+      R.inv_m = inv_m;
+      R.key0 = mlt_phase(opts.seed, 2);
+      if ((rc = run_chains(s, P, R, C, (uint32_t)m.steps, tm, tot))) return rc;
+    } else {
+      for (int64_t it = 0; it < m.steps; ++it) {
+        HIPCHK(launch_mlt_mutate(CH, 1, 0u, C, (uint32_t)it, m.p_large, st));
+        Params Pi = P;
+        mlt_key(opts.seed, 2, (uint64_t)it, Pi.key0, Pi.key1);
+        if ((rc = run_batch(s, Pi, Batch{0, C}, accum, none, FORM_AUTO, tm, tot))) return rc;
+        HIPCHK(launch_mlt_step(CH, accum, (uint32_t)it, m.p_large, b, weight, inv_m, ctr, st));
+      }
     }
     steps_run = m.steps;
   }
@@ -295,10 +307,22 @@ static int render_erpt(prt_scene* s, const prt_erpt_opts* o, void* d_out, int as
       CH.n = (uint32_t)std::min<uint64_t>(B, n_chains - j0);
       CH.base = (uint32_t)(chain_base + j0);
       HIPCHK(launch_erpt_chain_init(CH, E, fresh.prop, j0, first, ss2, P.W, P.H, st));
-      for (int step = 0; step < M; ++step) {
-        HIPCHK(launch_erpt_perturb(CH, (uint32_t)step, d, st));
-        if ((rc = trace(CH.prop, CH.pix_new, nullptr, CH.n))) return rc;
-        HIPCHK(launch_erpt_step(CH, accum, (uint32_t)step, ctr, st));
+      if (chains_async(s, CH.n)) {
+        Params Pb = P;
+        Pb.mlt_u = CH.prop;
+        ChainRun R{};
+        R.erpt = CH;
+        R.erpt_on = 1;
+        R.d = d;
+        R.key0 = mlt_phase(opts.seed, 7) + launch;
+        if ((rc = run_chains(s, Pb, R, CH.n, (uint32_t)M, tm, tot))) return rc;
+        launch += (uint64_t)M;
+      } else {
+        for (int step = 0; step < M; ++step) {
+          HIPCHK(launch_erpt_perturb(CH, (uint32_t)step, d, st));
+          if ((rc = trace(CH.prop, CH.pix_new, nullptr, CH.n))) return rc;
+          HIPCHK(launch_erpt_step(CH, accum, (uint32_t)step, ctr, st));
+        }
       }
       proposals += (uint64_t)CH.n * (uint64_t)M;
     }

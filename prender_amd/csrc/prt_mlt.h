@@ -1,9 +1,10 @@
 // prt_mlt.h — device side of the primary-sample-space Metropolis renderer
 // (Kelemen et al. 2002 as Render::RunMLT runs it, render.h:360-780).
 //
-// Each Markov chain is one slot of a wavefront batch: per iteration the
-// chain's proposal (its primary samples mutated, or all fresh for a large
-// step) is traced through the same extend / shade / NEE / shadow kernels as a
+// Each Markov chain is one slot of a batch.  Up to some hundred thousand chains
+// of a scene without glass run each at its own pace in the path kernel
+// (run_chains); otherwise, per iteration, every chain's proposal (its primary
+// samples mutated, or all fresh for a large step) is traced as one batch like a
 // camera sample, and k_mlt_step then splats the current and the proposed path
 // with Kelemen's weights and accepts or rejects.  All random decisions of the
 // chain logic come from Philox streams keyed by (chain, iteration, tag), so a
@@ -133,6 +134,18 @@ hipError_t launch_erpt_perturb(const ErptChains& C, uint32_t step, double d, hip
 // row fell on one pixel (render.h:975-1007).
 hipError_t launch_erpt_step(const ErptChains& C, const uint64_t* accum, uint32_t step, uint64_t* ctr,
                             hipStream_t s);
+
+// Steps [it0, it1) of every chain of a launch of the path kernel, each chain
+// at its own pace.
+struct ChainRun {
+  MltChains mlt;
+  ErptChains erpt;
+  double p_large, b, weight, inv_m;  // Metropolis (launch_mlt_step)
+  double d;                          // energy redistribution (launch_erpt_perturb)
+  uint64_t key0;                     // step it's paths take the Philox key splitmix64(key0 + it)
+  uint32_t it0, it1;
+  int32_t erpt_on;
+};
 
 // Final image: img * scale, float or double.
 hipError_t launch_mlt_resolve(const uint64_t* img, int64_t n, double scale, void* out, int as_f64, hipStream_t s);

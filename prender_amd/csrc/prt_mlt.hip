@@ -7,51 +7,15 @@
 
 #include <algorithm>
 
+#include "prt_chain.h"
 #include "prt_math.h"
 #include "prt_mlt.h"
 #include "prt_shade.h"
 
 namespace {
 
-__device__ __forceinline__ uint32_t word_of(double x) {
-  // x in [0, 1]; 1 wraps to 0 (the primary sample space is a torus)
-  return x >= 1.0 ? 0u : (uint32_t)(x * 4294967296.0);
-}
-
-// Mutate0 (mlt.h:42-54), LuxRender's small step: an exponentially
-// distributed offset between s1 / (s1/s2 + 1) and s2, up or down with equal
-// probability, wrapped into [0, 1).  fabsf keeps the reference's float
-// absolute value.
-__device__ __forceinline__ uint32_t mutate0(uint32_t w, double r) {
-  const double x = u01(w);
-  const double s1 = 1.0 / 512.0, s2 = 1.0 / 16.0;
-  const double dx = s1 / (s1 / s2 + (double)fabsf((float)(2.0 * r - 1.0))) - s1 / (s1 / s2 + 1.0);
-  if (r < 0.5) {
-    const double x1 = x + dx;
-    return word_of((x1 < 1.0) ? x1 : x1 - 1.0);
-  }
-  const double x1 = x - dx;
-  return word_of((x1 < 0.0) ? x1 + 1.0 : x1);
-}
-
-__device__ __forceinline__ bool large_step(const MltChains& C, uint32_t chain, uint32_t iter, double p_large) {
-  uint32_t b[4];
-  philox(chain, iter, MLT_TAG_LARGE, 0u, C.k0, C.k1, b);
-  return u01(b[0]) < p_large;
-}
-
 __device__ __forceinline__ void seed_words(const MltChains& C, uint32_t seed, uint32_t blk, uint32_t w[4]) {
   philox(seed, 0u, MLT_TAG_SEED, blk, C.k0, C.k1, w);
-}
-
-// mlt.h:171-174 with the Vector3d dot pairing
-__device__ __forceinline__ double lum3(const double f[3]) { return (0.2126 * f[0] + 0.0722 * f[2]) + 0.7152 * f[1]; }
-
-__device__ __forceinline__ void splat(uint64_t* img, uint32_t pix, double w, const double f[3]) {
-  for (int k = 0; k < 3; ++k) {
-    const double v = w * f[k];
-    if (v > 0.0) atomicAdd((unsigned long long*)&img[3 * (size_t)pix + k], (unsigned long long)(v * MLT_FIX_ONE + 0.5));
-  }
 }
 
 // One thread per (chain, block of 4 words).
@@ -62,49 +26,24 @@ __global__ __launch_bounds__(256) void k_mlt_mutate(MltChains C, int mode, uint3
   if (t >= (uint64_t)n * blocks) return;
   const uint32_t chain = (uint32_t)(t / blocks), blk = (uint32_t)(t % blocks);
   uint4* out = reinterpret_cast<uint4*>(C.prop + (size_t)chain * C.stride) + blk;
-  uint32_t w[4];
   if (mode == 0) {
+    uint32_t w[4];
     seed_words(C, first + chain, blk, w);
-  } else if (large_step(C, chain, iter, p_large)) {
-    // large step: fresh primary samples (mlt.h:116-121)
-    philox(chain, iter, MLT_TAG_FRESH, blk, C.k0, C.k1, w);
+    *out = make_uint4(w[0], w[1], w[2], w[3]);
   } else {
-    // small step: Mutate0 of every word (mlt.h:123-135; mutating the words a
-    // path does not use changes nothing it evaluates, and the lazy catch-up
-    // there applies the same mutations when a word is next used)
     const uint4 v = reinterpret_cast<const uint4*>(C.cur + (size_t)chain * C.stride)[blk];
-    uint32_t r[4];
-    philox(chain, iter, MLT_TAG_MUTATE, blk, C.k0, C.k1, r);
-    w[0] = mutate0(v.x, u01(r[0]));
-    w[1] = mutate0(v.y, u01(r[1]));
-    w[2] = mutate0(v.z, u01(r[2]));
-    w[3] = mutate0(v.w, u01(r[3]));
+    *out = mlt_propose(C, chain, iter, blk, p_large, v);
   }
-  *out = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// generate_new_path's camera part (render.h:262-300) with the tent filter the
-// MLT mode switches on (scene_env.h:1954): pixel (u0 W, u1 H), sub-pixel
-// (u2 < 1/2, u3 < 1/2) of a 2x2 grid, tent offsets from u4, u5.
 __global__ __launch_bounds__(256) void k_mlt_gen(Params P, uint32_t n, RayQ q) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t* u = P.mlt_u + (size_t)i * (uint32_t)P.mlt_stride;
-  const int x = min((int)(u01(u[0]) * (double)P.W), P.W - 1);
-  const int y = min((int)(u01(u[1]) * (double)P.H), P.H - 1);
-  const int sx = u01(u[2]) < 0.5 ? 0 : 1;
-  const int sy = u01(u[3]) < 0.5 ? 0 : 1;
-  const double rr1 = 2.0 * u01(u[4]), rr2 = 2.0 * u01(u[5]);
-  const double dx = rr1 < 1.0 ? sqrt(rr1) - 1.0 : 1.0 - sqrt(2.0 - rr1);
-  const double dy = rr2 < 1.0 ? sqrt(rr2) - 1.0 : 1.0 - sqrt(2.0 - rr2);
-  const double r1 = (sx + 0.5 + dx) * 0.5;
-  const double r2 = (sy + 0.5 + dy) * 0.5;
-  const d3 sp = ld3(P.center) + ld3(P.screen_x) * ((r1 + x) * P.iw - 0.5) + ld3(P.screen_y) * ((r2 + y) * P.ih - 0.5);
-  const d3 o = ld3(P.cam_pos);
-  const d3 d = normalize(sp - o);
+  d3 o, d;
+  P.mlt_pix[i] = mlt_camera_ray(P, u, o, d);
   q.ox[i] = o.x; q.oy[i] = o.y; q.oz[i] = o.z;
   q.dx[i] = d.x; q.dy[i] = d.y; q.dz[i] = d.z;
-  P.mlt_pix[i] = (uint32_t)((P.H - y - 1) * P.W + x);  // render.h:585-586
 }
 
 __global__ __launch_bounds__(256) void k_mlt_seed_record(const uint64_t* __restrict__ accum,
@@ -210,10 +149,6 @@ __global__ __launch_bounds__(256) void k_mlt_init(MltChains C, MltSeeds S) {
   C.pix_old[c] = S.pix[seed];
 }
 
-// render.h:574-630: a = min(1, L_new / L_old) (1 when L_old is ~0); the
-// proposal gets (a + large) / (L_new / b + p_large) / M, the current path
-// (1 - a) / (L_old / b + p_large) / M, each times the path weight 4*W*H and
-// its radiance; then accept with probability a.
 __global__ __launch_bounds__(256) void k_mlt_step(MltChains C, const uint64_t* __restrict__ accum, uint32_t iter,
                                                   double p_large, double b, double weight, double inv_m,
                                                   uint64_t* ctr) {
@@ -222,26 +157,11 @@ __global__ __launch_bounds__(256) void k_mlt_step(MltChains C, const uint64_t* _
   if (c < C.n) {
     const double fn[3] = {accum_get(accum + 3 * (size_t)c), accum_get(accum + 3 * (size_t)c + 1),
                           accum_get(accum + 3 * (size_t)c + 2)};
-    const double fo[3] = {C.f_old[3 * (size_t)c], C.f_old[3 * (size_t)c + 1], C.f_old[3 * (size_t)c + 2]};
-    const double l_new = lum3(fn), l_old = lum3(fo);
-    const double a = l_old > 1.0e-16 ? fmin(1.0, l_new / l_old) : 1.0;
-    const double large = large_step(C, c, iter, p_large) ? 1.0 : 0.0;
-    const double w_new = (a + large) / (l_new / b + p_large) * inv_m;
-    const double w_old = (1.0 - a) / (l_old / b + p_large) * inv_m;
-    const uint32_t p_new = C.pix_new[c], p_old = C.pix_old[c];
-    splat(C.img, p_old, w_old * weight, fo);
-    splat(C.img, p_new, w_new * weight, fn);
-    uint32_t r[4];
-    philox(c, iter, MLT_TAG_ACCEPT, 0u, C.k0, C.k1, r);
-    if (u01(r[0]) < a) {
-      acc = true;
+    acc = mlt_accept(C, c, iter, p_large, b, weight, inv_m, fn, C.pix_new[c]);
+    if (acc) {
       const uint4* src = reinterpret_cast<const uint4*>(C.prop + (size_t)c * C.stride);
       uint4* dst = reinterpret_cast<uint4*>(C.cur + (size_t)c * C.stride);
       for (uint32_t blk = 0; blk < C.stride / 4u; ++blk) dst[blk] = src[blk];
-      C.f_old[3 * (size_t)c] = fn[0];
-      C.f_old[3 * (size_t)c + 1] = fn[1];
-      C.f_old[3 * (size_t)c + 2] = fn[2];
-      C.pix_old[c] = p_new;
     }
   }
   const uint64_t n_acc = __popcll(__ballot(acc));
@@ -333,17 +253,7 @@ __global__ __launch_bounds__(256) void k_erpt_perturb(ErptChains C, uint32_t ste
   if (t >= (uint64_t)C.n * blocks) return;
   const uint32_t j = (uint32_t)(t / blocks), blk = (uint32_t)(t % blocks);
   const uint4 v = reinterpret_cast<const uint4*>(C.cur + (size_t)j * C.stride)[blk];
-  uint32_t r[4];
-  philox(C.base + j, step, ERPT_TAG_PERTURB, blk, C.k0, C.k1, r);
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  uint32_t o[4];
-  for (int k = 0; k < 4; ++k) {
-    double x = u01(w[k]) + d * (2.0 * u01(r[k]) - 1.0);  // erpt.h:29-34
-    if (x > 1.0) x -= 1.0;
-    if (x < 0.0) x += 1.0;
-    o[k] = word_of(x);
-  }
-  reinterpret_cast<uint4*>(C.prop + (size_t)j * C.stride)[blk] = make_uint4(o[0], o[1], o[2], o[3]);
+  reinterpret_cast<uint4*>(C.prop + (size_t)j * C.stride)[blk] = erpt_propose(C, j, step, blk, d, v);
 }
 
 __global__ __launch_bounds__(256) void k_erpt_step(ErptChains C, const uint64_t* __restrict__ accum, uint32_t step,
@@ -353,34 +263,12 @@ __global__ __launch_bounds__(256) void k_erpt_step(ErptChains C, const uint64_t*
   if (j < C.n) {
     const double fz[3] = {accum_get(accum + 3 * (size_t)j), accum_get(accum + 3 * (size_t)j + 1),
                           accum_get(accum + 3 * (size_t)j + 2)};
-    double fy[3] = {C.f_y[3 * (size_t)j], C.f_y[3 * (size_t)j + 1], C.f_y[3 * (size_t)j + 2]};
-    const double lz = lum3(fz), ly = lum3(fy);
-    const double q = fmin(1.0, ly > 1.0e-16 ? lz / ly : 0.0);  // render.h:978-980
-    uint32_t r[4];
-    philox(C.base + j, step, ERPT_TAG_ACCEPT, 0u, C.k0, C.k1, r);
-    uint32_t py = C.pix_y[j];
-    if (q > u01(r[0])) {
-      acc = true;
+    acc = erpt_accept(C, j, step, fz, C.pix_new[j]);
+    if (acc) {
       const uint4* src = reinterpret_cast<const uint4*>(C.prop + (size_t)j * C.stride);
       uint4* dst = reinterpret_cast<uint4*>(C.cur + (size_t)j * C.stride);
       for (uint32_t blk = 0; blk < C.stride / 4u; ++blk) dst[blk] = src[blk];
-      for (int k = 0; k < 3; ++k) {
-        fy[k] = fz[k];
-        C.f_y[3 * (size_t)j + k] = fz[k];
-      }
-      py = C.pix_new[j];
-      C.pix_y[j] = py;
     }
-    uint32_t run = C.run[j];
-    if (C.pix_now[j] == py) {
-      ++run;
-    } else {
-      C.pix_now[j] = py;
-      run = 0;
-    }
-    C.run[j] = run;
-    const double l = lum3(fy);
-    if (run < ERPT_MAX_STACK && l > 0.0) splat(C.img, py, C.dep / l, fy);
   }
   const uint64_t n_acc = __popcll(__ballot(acc));
   if (lane_id() == 0) ctr_add(ctr, CTR_MLT_ACCEPT, n_acc);

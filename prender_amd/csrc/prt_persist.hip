@@ -3,7 +3,7 @@
 //
 // It renders the samples of a batch of scenes (the batched renderer's
 // persistent form and frames without light sampling), of one small frame or
-// Metropolis step (a depth-synchronous batch would pay two traversal launches
+// batch of Metropolis proposals (a depth-synchronous batch would pay two traversal launches
 // per depth, each as long as its slowest ray), or the last rays of a
 // depth-synchronous batch, from their queue.
 //
@@ -31,7 +31,14 @@
 // other, and against depth-synchronous batches: spheres 32x24 x 8 spp 834 ->
 // 175 us, 320x240 x 16 spp 1636 -> 951 us; mesh box 128x128 x 8 spp 2707 -> 926
 // us; glass with light sampling 201x151 x 27 spp 5997 -> 3176 us; Metropolis
-// steps of 15,360 chains 2.5 -> 0.41 ms.
+// batches of 15,360 chains 2.5 -> 0.41 ms.
+//
+// Markov chains of scenes without glass run here whole: a lane keeps a chain,
+// accepts or rejects when its path has ended and goes on with the chain's next
+// proposal, while the wave's other chains are wherever they are; the words of the
+// proposals that are due are dealt over the lanes.  Chains in step cost the longest
+// path of all chains per step: 15,360 chains x 64 steps 31.3 ms, each at its own
+// pace 23.4 ms; 180,000 x 48 142.5 and 131.5 ms.
 //
 // A wave works on one scene at a time, so the scene's parameters are
 // wave-uniform scalar loads: a lane starts a sample of another scene only
@@ -47,6 +54,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "prt_chain.h"
 #include "prt_device.h"
 #include "prt_kernels.h"
 #include "prt_math.h"
@@ -142,7 +150,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   bool act = false;
   d3 o = mk(0.0, 0.0, 0.0), d = o;
   float tr[3] = {1.0f, 1.0f, 1.0f}, pw[3] = {0.0f, 0.0f, 0.0f}, nr[3] = {0.0f, 0.0f, 0.0f};
-  uint32_t meta = 0, slot = 0;  // slot: sample of the scene (frame, queue: of the batch)
+  uint32_t meta = 0, slot = 0;  // slot: sample of the scene (frame, queue: of the batch), or chain
+  // its chain: the step, that step's image element and Philox key; whether the
+  // next proposal is due, and whether the last one was accepted
+  uint32_t it = 0, element = 0, accepts = 0;
+  RngKey key = SRC == PATH_CHAIN ? RngKey{0u, 0u} : key_of(P0);
+  bool due = false, took = false;
 
   while (true) {
     // ---- idle lanes take the wave's waiting segments, then new samples
@@ -191,7 +204,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           const uint64_t first = (uint64_t)(cb - st.chunk_base[cs]) * 64u;
           const uint64_t n_s = st.sample_base[cs + 1] - st.sample_base[cs];
           cn = (uint32_t)__builtin_amdgcn_readfirstlane((int)(n_s - first < 64u ? n_s - first : 64u));
-        } else if (SRC == PATH_FRAME) {
+        } else if (SRC == PATH_FRAME || SRC == PATH_CHAIN) {
           cs = 0;
           cn = min(st.unit, st.n_samples - cb * st.unit);
         } else {
@@ -224,7 +237,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
         } else {
           if (SRC == PATH_BATCH) slot = (cb - st.chunk_base[scene]) * 64u + co + rank;
           else slot = cb * st.unit + co + rank;
-          if (SRC == PATH_FRAME && P.mlt_u != nullptr) {  // a Metropolis proposal's own camera ray
+          if (SRC == PATH_CHAIN) {
+            it = st.chain.it0;
+            due = true;
+          } else if (SRC == PATH_FRAME && P.mlt_u != nullptr) {  // a Metropolis proposal's own camera ray
             o = mk(st.q.ox[slot], st.q.oy[slot], st.q.oz[slot]);
             d = mk(st.q.dx[slot], st.q.dy[slot], st.q.dz[slot]);
           } else {
@@ -235,7 +251,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           tr[0] = tr[1] = tr[2] = 1.0f;
           pw[0] = pw[1] = pw[2] = 0.0f;
           meta = rng_c2(0, 1u);
-          ++n_prim;
+          if (SRC != PATH_CHAIN) ++n_prim;
         }
         act = true;
       }
@@ -253,8 +269,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
       continue;
     }
     const Params& P = SRC == PATH_BATCH ? scene_params(st.scenes, scene) : P1;
-    const uint32_t pixel = (uint32_t)(st.batch.pixel_base + (int64_t)(slot / (uint32_t)P.spp));
-    const uint32_t k = slot % (uint32_t)P.spp;
+    if (SRC == PATH_CHAIN) {
+      // ---- proposals that are due, their words dealt over the wave's lanes
+      const ChainRun& R = st.chain;
+      const uint64_t due_m = __ballot(due);
+      if (due_m) {
+        const uint32_t stride = (uint32_t)P.mlt_stride, blocks = stride / 4u;
+        const uint32_t n_items = blocks * (uint32_t)__popcll(due_m);
+        uint32_t* words = R.erpt_on ? R.erpt.cur : R.mlt.cur;
+        uint32_t* prop = R.erpt_on ? R.erpt.prop : R.mlt.prop;
+        if (due) s_map[wbase + (uint32_t)__popcll(due_m & below)] = (uint8_t)lane;
+        wave_fence();
+        for (uint32_t base = 0; base < n_items; base += 64u) {
+          const uint32_t item = base + lane, blk = item % blocks;
+          const int src = item < n_items ? (int)s_map[wbase + item / blocks] : (int)lane;
+          const uint32_t chain = (uint32_t)__shfl((int)slot, src, 64), step = (uint32_t)__shfl((int)it, src, 64);
+          const bool moved = __shfl((int)took, src, 64) != 0;
+          if (item < n_items) {
+            uint4* cur = reinterpret_cast<uint4*>(words + (size_t)chain * stride) + blk;
+            uint4* out = reinterpret_cast<uint4*>(prop + (size_t)chain * stride) + blk;
+            const uint4 v = moved ? *out : *cur;
+            if (moved) *cur = v;
+            if (step < R.it1)
+              *out = R.erpt_on ? erpt_propose(R.erpt, chain, step, blk, R.d, v)
+                               : mlt_propose(R.mlt, chain, step, blk, R.p_large, v);
+          }
+        }
+        wave_fence();
+        if (due) {
+          due = took = false;
+          if (it < R.it1) {
+            element = mlt_camera_ray(P, prop + (size_t)slot * stride, o, d);
+            key = chain_key(R.key0 + it);
+            tr[0] = tr[1] = tr[2] = 1.0f;
+            pw[0] = pw[1] = pw[2] = 0.0f;
+            meta = rng_c2(0, 1u);
+            ++n_prim;
+          } else {
+            act = false;
+          }
+        }
+        if (!__any(act)) continue;
+      }
+    }
+    const uint32_t pixel =
+        SRC == PATH_CHAIN ? slot : (uint32_t)(st.batch.pixel_base + (int64_t)(slot / (uint32_t)P.spp));
+    const uint32_t k = SRC == PATH_CHAIN ? 0u : slot % (uint32_t)P.spp;
+    if (SRC != PATH_CHAIN) key = key_of(P);
     // ---- light samples and closest hits
     double t = PS_INF;
     int32_t id = -1;
@@ -284,9 +345,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           const d3 ct = mk(__shfl(tr[0], src, 64), __shfl(tr[1], src, 64), __shfl(tr[2], src, 64));
           const uint32_t sp = (uint32_t)__shfl((int)pixel, src, 64), sk = (uint32_t)__shfl((int)k, src, 64);
           const uint32_t sm = (uint32_t)__shfl((int)meta, src, 64);
+          RngKey sample_key = key;
+          if (SRC == PATH_CHAIN)
+            sample_key = RngKey{(uint32_t)__shfl((int)key.k0, src, 64), (uint32_t)__shfl((int)key.k1, src, 64)};
           if (has) {
             uint32_t w[3];
-            nee_words_of(P, sp, sk, (int)(sm & 0xFFu) - 1, META_BRANCH(sm), (int)(item % 3u), w);
+            nee_words_of(sample_key, sp, sk, (int)(sm & 0xFFu) - 1, META_BRANCH(sm), (int)(item % 3u), w);
             int32_t l = -1;
             shadow = lights ? nee_one_slots(P, lights, w, 0, x, nrm, ct, sr, l) : nee_one(P, w, 0, x, nrm, ct, sr, l);
           }
@@ -325,8 +389,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
       C.truncated = C.n_ext = C.pickups = C.dropped = C.direct = 0;
       VertexAdj va;
       const int depth = (int)(meta & 0xFFu);
-      const d3 add = shade_vertex(P, lds_mats ? lds_mats : P.mats, C, o, d, t, id, mk(tr[0], tr[1], tr[2]), mk(pw[0], pw[1], pw[2]), pixel, k,
-                                  depth, META_BRANCH(meta), va);
+      const d3 add = shade_vertex(P, lds_mats ? lds_mats : P.mats, C, o, d, t, id, mk(tr[0], tr[1], tr[2]), mk(pw[0], pw[1], pw[2]), key, pixel,
+                                  k, depth, META_BRANCH(meta), va);
       uint64_t acc[3] = {fix_of(add.x), fix_of(add.y), fix_of(add.z)};
       truncated += C.truncated;
       n_ext += C.n_ext;
@@ -344,6 +408,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           nr[j] = C.n0[j];
         }
         meta = C.meta0;
+      } else if (SRC == PATH_CHAIN) {
+        double f[3];
+        for (int c = 0; c < 3; ++c) {
+          acc[c] += s_acc[c][threadIdx.x];
+          s_acc[c][threadIdx.x] = 0ull;
+          f[c] = accum_get(&acc[c]);
+        }
+        const ChainRun& R = st.chain;
+        took = R.erpt_on ? erpt_accept(R.erpt, slot, it, f, element)
+                         : mlt_accept(R.mlt, slot, it, R.p_large, R.b, R.weight, R.inv_m, f, element);
+        accepts += took ? 1u : 0u;
+        ++it;
+        due = true;
       } else {
         const uint64_t at = (SRC == PATH_BATCH ? st.sample_base[scene] : 0ull) + slot;
         for (int c = 0; c < 3; ++c) {
@@ -359,7 +436,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   flush_stats(st.ctr, CTR_SNODES, tsh);
   const uint64_t s_prim = wave_sum_u32(n_prim), s_tr = wave_sum_u32(n_traced), s_sh = wave_sum_u32(n_shadow);
   const uint64_t s_ext = wave_sum_u32(n_ext), s_pick = wave_sum_u32(pickups), s_trunc = wave_sum_u32(truncated);
-  const uint64_t s_drop = wave_sum_u32(dropped);
+  const uint64_t s_drop = wave_sum_u32(dropped), s_acc_n = SRC == PATH_CHAIN ? wave_sum_u32(accepts) : 0ull;
   if (lane == 0) {
     auto count = [&](int c, uint64_t v) { ctr_add(st.ctr, c, v); };
     count(CTR_QUEUED, s_prim + s_ext);
@@ -370,6 +447,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
     count(CTR_PICKUP, s_pick);
     count(CTR_TRUNC, s_trunc);
     count(CTR_DROP, s_drop);
+    if (SRC == PATH_CHAIN) count(CTR_MLT_ACCEPT, s_acc_n);
   }
 }
 // Every pixel of every scene of the batch: fold its samples' accumulators
@@ -419,6 +497,7 @@ template <class F>
 static hipError_t with_path_kernel(PathSource src, bool nee, int waves, F&& f) {
   if (src == PATH_BATCH) return nee ? with_path_waves<PATH_BATCH, true>(waves, f) : with_path_waves<PATH_BATCH, false>(waves, f);
   if (src == PATH_FRAME) return nee ? with_path_waves<PATH_FRAME, true>(waves, f) : with_path_waves<PATH_FRAME, false>(waves, f);
+  if (src == PATH_CHAIN) return with_path_waves<PATH_CHAIN, true>(waves, f);
   return with_path_waves<PATH_QUEUE, true>(waves, f);
 }
 

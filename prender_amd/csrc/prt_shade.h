@@ -39,6 +39,12 @@ __device__ __forceinline__ void camera_ray(const Params& P, int x, int y, int sx
   d = normalize(sp - o);
 }
 
+// Philox key of a path: the render's, or the Markov chain's step's.
+struct RngKey {
+  uint32_t k0, k1;
+};
+__device__ __forceinline__ RngKey key_of(const Params& P) { return RngKey{P.key0, P.key1}; }
+
 // Random words 0..3 of a path vertex: Russian roulette, BSDF choice, the two
 // direction numbers (counter (pixel, sample, depth | branch << 8, 0)).  In a
 // Metropolis render the first mlt_depths vertices read them from the chain's
@@ -46,7 +52,7 @@ __device__ __forceinline__ void camera_ray(const Params& P, int x, int y, int sx
 // primary samples are exactly these next01() draws (radiance.h:108, 517,
 // 534; brdf.h:511-512, 866), while light sampling draws Next01() from an
 // independent stream (directLight_radiance.h:343-359).
-__device__ __forceinline__ void vertex_words(const Params& P, uint32_t pixel, uint32_t sample, int depth,
+__device__ __forceinline__ void vertex_words(const Params& P, RngKey key, uint32_t pixel, uint32_t sample, int depth,
                                              uint32_t branch, uint32_t b[4]) {
   if (P.mlt_u != nullptr && depth < P.mlt_depths) {
     const uint4 v = *reinterpret_cast<const uint4*>(P.mlt_u + (size_t)pixel * (uint32_t)P.mlt_stride +
@@ -54,7 +60,7 @@ __device__ __forceinline__ void vertex_words(const Params& P, uint32_t pixel, ui
     b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
     return;
   }
-  philox(pixel, sample, rng_c2(depth, branch), 0u, P.key0, P.key1, b);
+  philox(pixel, sample, rng_c2(depth, branch), 0u, key.k0, key.k1, b);
 }
 
 // Children go to qout positions off + j, j < cap, with j from *count_out.
@@ -155,8 +161,8 @@ __device__ __forceinline__ void emit_child(LaneCtx& C, d3 o, d3 d, d3 ct, d3 pw,
 // mats: the material table (P.mats, or a block's LDS copy of it).
 template <class Ctx>
 __device__ __forceinline__ d3 shade_vertex(const Params& P, const DevMaterial* mats, Ctx& C, d3 o, d3 d,
-                                           double t, int32_t id, d3 T, d3 Pw, uint32_t pixel, uint32_t sample,
-                                           int depth, uint32_t branch, VertexAdj& va) {
+                                           double t, int32_t id, d3 T, d3 Pw, RngKey key, uint32_t pixel,
+                                           uint32_t sample, int depth, uint32_t branch, VertexAdj& va) {
   d3 add = mk(0.0, 0.0, 0.0);
   const d3 zero = mk(0.0, 0.0, 0.0);
   va.entity = -1;
@@ -231,7 +237,7 @@ __device__ __forceinline__ d3 shade_vertex(const Params& P, const DevMaterial* m
   if (depth > P.depth_limit) rr *= ldexp(1.0, -(depth - P.depth_limit));  // pow(0.5, k), exact
   uint32_t b0[4];
   const uint32_t c2 = rng_c2(depth, branch);
-  vertex_words(P, pixel, sample, depth, branch, b0);
+  vertex_words(P, key, pixel, sample, depth, branch, b0);
   if (depth > P.depth) {
     if (u01(b0[0]) >= rr) {  // terminate with the emission
       va.own = vmul(T, E);
@@ -318,7 +324,7 @@ __device__ __forceinline__ d3 shade_vertex(const Params& P, const DevMaterial* m
     uint32_t wg = b0[1];
     if (P.mlt_u == nullptr) {
       uint32_t b3[4];
-      philox(pixel, sample, c2, 3u, P.key0, P.key1, b3);
+      philox(pixel, sample, c2, 3u, key.k0, key.k1, b3);
       wg = b3[1];
     }
     const bool take_refl = u01(wg) < probability;
@@ -461,12 +467,12 @@ __device__ __forceinline__ void nee_words(const Params& P, uint32_t pixel, uint3
 
 // The three words of light sample m alone (w[3m .. 3m + 2] of nee_words), at
 // two Philox blocks instead of three.
-__device__ __forceinline__ void nee_words_of(const Params& P, uint32_t pixel, uint32_t sample, int depth,
+__device__ __forceinline__ void nee_words_of(RngKey key, uint32_t pixel, uint32_t sample, int depth,
                                              uint32_t branch, int m, uint32_t w[3]) {
   const uint32_t c2 = rng_c2(depth, branch), first = m == 2 ? 2u : 1u;
   uint32_t a[4], b[4];
-  philox(pixel, sample, c2, first, P.key0, P.key1, a);
-  philox(pixel, sample, c2, first + 1u, P.key0, P.key1, b);
+  philox(pixel, sample, c2, first, key.k0, key.k1, a);
+  philox(pixel, sample, c2, first + 1u, key.k0, key.k1, b);
   w[0] = m == 0 ? a[0] : m == 1 ? a[3] : a[2];
   w[1] = m == 0 ? a[1] : m == 1 ? b[0] : a[3];
   w[2] = m == 0 ? a[2] : m == 1 ? b[1] : b[0];

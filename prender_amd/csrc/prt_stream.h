@@ -50,6 +50,7 @@
 
 #include "prt_device.h"
 #include "prt_kernels.h"
+#include "prt_mlt.h"
 
 // One work item: pixels [pixel_base, pixel_base + n_pixels) (y*W + x order) of
 // scene `scene`, all spp samples of each.
@@ -176,13 +177,15 @@ struct Persist {
   Batch batch;                  // pixels of a frame or queue
   RayQ q;                       // a queue's rays; the camera rays of Metropolis proposals
   ChunkList cl;                 // a queue's chunks
+  ChainRun chain;               // steps of Markov chains
 };
 
 // Where a launch's segments come from.
 enum PathSource {
   PATH_BATCH = 0,  // the camera samples of n_scenes scenes, 64 per chunk
   PATH_FRAME = 1,  // the camera samples of one scene (or its Metropolis proposals), unit per chunk
-  PATH_QUEUE = 2   // the rays of a queue, whose vertices have had their light samples
+  PATH_QUEUE = 2,  // the rays of a queue, whose vertices have had their light samples
+  PATH_CHAIN = 3   // the proposals of n_samples Markov chains of a scene without glass, unit chains per chunk
 };
 // waves: waves per SIMD to budget its registers for (2, or 3 without light
 // sampling; launches with light sampling take 2).  P: the scene of a frame or

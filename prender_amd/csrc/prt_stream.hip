@@ -390,7 +390,7 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
       VertexAdj va;
       const d3 add = shade_vertex(P, P.mats, C, mk(qin.ox[ray], qin.oy[ray], qin.oz[ray]),
                                   mk(qin.dx[ray], qin.dy[ray], qin.dz[ray]), hit_t[ray], hit_id[ray], T, Pw,
-                                  (uint32_t)pixel, k, depth, branch, va);
+                                  key_of(P), (uint32_t)pixel, k, depth, branch, va);
       delta = (int)(C.n_ext - e0) - 1;
       accum_add(&st.accum[3 * (size_t)slot + 0], add.x);
       accum_add(&st.accum[3 * (size_t)slot + 1], add.y);
