@@ -408,7 +408,8 @@ int prt_set_emission(prt_scene* scene, int entity, const double emission[3]);
  * primal decisions, for finite-difference checks under common random
  * numbers); hold = 0: they follow the current albedo again. */
 int prt_hold_rr_albedo(prt_scene* scene, int hold);
-/* Path-replay adjoint: given dL/dimage (W*H*3 device floats), accumulate
+/* Adjoint of the render with the same options: given dL/dimage (W*H*3 device
+ * floats), accumulate
  * dL/dalbedo into d_albedo_grad (n_faces*3 device floats of `entity`) and
  * dL/demission (3 doubles, host) for light `light`. */
 int prt_adjoint_device(prt_scene* scene, const prt_render_opts* opts,

@@ -88,7 +88,8 @@ struct Workspace {
   DevBuf desc[4];             // chunk descriptors (uint2) of q[0], q[1], the shadow queue, the second one
   DevBuf slabs;               // uint2 [3][PRT_SLAB_WAVES] slab (start, count) of q[0], q[1], the NEE output
   DevBuf accum, accum2;       // fixed-point sample radiance (accum2: adjoint primal)
-  DevBuf counts;              // uint32 [16]: chunks of q0, q1, sq, sq2 at 0..3, entries at 4..7
+  DevBuf recs[5];             // adjoint records (AdjointRecs: id, slot, before)
+  DevBuf counts;              // uint32 [16]: chunks of q0, q1, sq, sq2 at 0..3, entries at 4..7, adjoint records at 8, 9
   DevBuf fetch;               // uint32 claim counters, PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE per launch
   DevBuf ctr;                 // uint64 [CTR_WORDS]
   DevBuf pool;                // path kernel: waiting glass segments, PoolRec [waves][PRT_PATH_POOL]
@@ -270,8 +271,9 @@ int ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass);
 enum BatchForm { FORM_WAVEFRONT = 0, FORM_AUTO = 1, FORM_PATH = 2 };
 // One batch of camera samples (or Metropolis proposals, when P.mlt_u is set);
 // sample radiance accumulates into accum (fixed point).
+// n_records: entries a recording pass's vertices take.
 int run_batch(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, const Adjoint& A, BatchForm form,
-              Timer& tm, CallTotals& tot);
+              Timer& tm, CallTotals& tot, uint32_t* n_records = nullptr);
 // Whether n Markov chains of the scene run each at their own pace (run_chains),
 // not step by step as batches; steps steps of them.  P.mlt_u: their proposals.
 bool chains_async(const prt_scene* s, uint32_t n);

@@ -100,8 +100,23 @@ struct ShadowQ {
 // derivative of the sample radiance with respect to the face albedo is the
 // radiance the path still gathers from there on, minus the vertex's own
 // emission, divided by the albedo.
+enum AdjointPass {
+  ADJ_NONE = 0,
+  ADJ_REPLAY = 1,  // the samples' radiance is known (ltot): albedo gradients at once
+  ADJ_RECORD = 2   // albedo vertices are recorded until it is
+};
+// Albedo vertices of a recording pass, 64 entries per input chunk of a shade
+// launch.
+struct AdjointRecs {
+  int32_t* id;        // triangle, or -1: none
+  uint32_t* slot;     // sample of the batch
+  double* before[3];  // its radiance up to the vertex, with the vertex's own emission
+  const uint32_t* first;  // entry of the launch's first chunk
+  uint32_t* next;         // the next launch's
+  uint32_t cap;       // entries beyond it are not written
+};
 struct Adjoint {
-  int32_t on;
+  int32_t on;  // AdjointPass
   int32_t entity;             // POLYGON entity whose per-face albedo is differentiated
   int32_t light;              // light entity whose emission is differentiated
   int32_t pad_;
@@ -110,6 +125,7 @@ struct Adjoint {
   double* grad_alb;           // n_faces*3 of `entity`
   double* grad_e;             // 3
   double scale;               // d image / d sample radiance = sensor_response * smp
+  AdjointRecs recs;           // recording pass
 };
 
 // A batch: pixels [pixel_base, pixel_base + n_pixels) of the y*W + x order,
@@ -174,4 +190,6 @@ hipError_t launch_fill_u64(uint64_t* p, uint64_t v, int64_t n, hipStream_t s);
 hipError_t launch_scatter_albedo(float* tri_alb, const uint32_t* slot_of_tri, int64_t first, int64_t n_faces,
                                  const float* albedo, hipStream_t s);
 hipError_t launch_grad_to_f32(const double* g, float* out, int64_t n, hipStream_t s);
+// The albedo gradients of the n records of a batch whose samples' radiance is A.ltot.
+hipError_t launch_adjoint_resolve(const Params& P, const Batch& B, const Adjoint& A, uint32_t n, hipStream_t s);
 hipError_t launch_count_mismatch(const uint64_t* a, const uint64_t* b, int64_t n, uint64_t* ctr, hipStream_t s);

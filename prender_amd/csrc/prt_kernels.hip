@@ -180,13 +180,13 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADOW) void k_shadow
 
 // ------------------------------------------------------------ shade
 // Shade one queue (or, with primary = 1, every camera sample of the batch
-// against the hit of its sub-pixel's primary ray).  ADJ: with the adjoint
-// bookkeeping of a path replay (a separate instance, so forward renders
-// carry none of its registers).
+// against the hit of its sub-pixel's primary ray).  ADJ (AdjointPass): with the
+// adjoint bookkeeping of a path replay or a recording pass (separate
+// instances, so forward renders carry none of their registers).
 // MLDS: the scene's materials (at most PRT_LDS_MATERIALS) are copied into
 // the block's LDS and read from there.
 #define PRT_LDS_MATERIALS 64
-template <bool ADJ, bool MLDS>
+template <int ADJ, bool MLDS>
 __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
     Params P, Batch B, int primary, RayQ qin, ChunkList cl, const double* __restrict__ hit_t,
     const int32_t* __restrict__ hit_id, RayQ qout, uint32_t fan, uint2* slabs, uint64_t* __restrict__ accum,
@@ -214,11 +214,16 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
   C.cap = fan * 64u * (c_end - c);
   C.truncated = C.n_ext = C.pickups = C.dropped = 0;
   double ge[3] = {0.0, 0.0, 0.0};
-  // chunk descriptors are read two chunks ahead and (forward renders: the
-  // adjoint instance has no registers to spare) the hits (t, id) of a ray one
+  // chunk descriptors are read two chunks ahead and (not in a replay,
+  // whose instance has no registers to spare) the hits (t, id) of a ray one
   // chunk ahead, so that a chunk's triangle reads, which depend on the hit,
   // go out with its ray reads instead of after them
-  constexpr bool PF = !ADJ;
+  constexpr bool PF = ADJ != ADJ_REPLAY;
+  const uint32_t rec_first = ADJ == ADJ_RECORD ? *A.recs.first : 0u;
+  if (ADJ == ADJ_RECORD && blockIdx.x == 0 && threadIdx.x == 0) {
+    const uint32_t more = 64u * n_chunks;
+    *A.recs.next = rec_first > 0xFFFFFFFFu - more ? 0xFFFFFFFFu : rec_first + more;
+  }
   uint2 dn1 = make_uint2(0u, 0u), dn2 = make_uint2(0u, 0u);
   double hn_t = 0.0;
   int32_t hn_id = -1;
@@ -234,9 +239,15 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
     uint32_t i;
     double hc_t = 0.0;
     int32_t hc_id = -1;
+    // this lane's record; none until its vertex is known
+    const uint64_t rec = (uint64_t)rec_first + (c << 6) + lane_id();
+    const bool rec_fits = ADJ == ADJ_RECORD && rec < A.recs.cap;
     if (primary) {
       i = (c << 6) + lane_id();
-      if (i >= n_samples) continue;
+      if (i >= n_samples) {
+        if (rec_fits) A.recs.id[rec] = -1;
+        continue;
+      }
     } else {
       const uint2 dc = dn1;
       if (PF) {
@@ -251,7 +262,10 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
       } else if (c + 1 < c_end) {
         dn1 = cl.desc[c + 1];
       }
-      if (lane_id() >= dc.y) continue;
+      if (lane_id() >= dc.y) {
+        if (rec_fits) A.recs.id[rec] = -1;
+        continue;
+      }
       i = dc.x + lane_id();
     }
     d3 o, d, T, Pw;
@@ -296,10 +310,23 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
     const d3 add = shade_vertex(P, mats, C, o, d, t, id, T, Pw, key_of(P), (uint32_t)(B.pixel_base + pl), k, depth, branch,
                                 va);
     if (primary && P.mlt_flags != nullptr) P.mlt_flags[slot] = C.direct;
-    if (ADJ && A.on) {
+    if (ADJ == ADJ_RECORD) {
+      const bool keep = va.albedo && va.entity == A.entity && va.face >= 0;
+      if (rec_fits) {
+        A.recs.id[rec] = keep ? id : -1;
+        if (keep) {
+          const uint64_t* lb = accum + 3 * (size_t)slot;
+          A.recs.slot[rec] = slot;
+          A.recs.before[0][rec] = accum_get(lb) + va.pre.x + va.own.x;
+          A.recs.before[1][rec] = accum_get(lb + 1) + va.pre.y + va.own.y;
+          A.recs.before[2][rec] = accum_get(lb + 2) + va.pre.z + va.own.z;
+        }
+      }
+    }
+    if (ADJ) {
       const size_t px = sample_image_index(P, B, slot);
       const d3 g = mk(A.dimage[3 * px] * A.scale, A.dimage[3 * px + 1] * A.scale, A.dimage[3 * px + 2] * A.scale);
-      if (va.albedo && va.entity == A.entity && va.face >= 0) {
+      if (ADJ == ADJ_REPLAY && va.albedo && va.entity == A.entity && va.face >= 0) {
         // radiance still to come from this vertex on (no glass splits: one
         // path per sample), without the vertex's own emission
         const uint64_t* lt = A.ltot + 3 * (size_t)slot;
@@ -322,7 +349,7 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
     accum_add(&accum[3 * (size_t)slot + 1], add.y);
     accum_add(&accum[3 * (size_t)slot + 2], add.z);
   }
-  if (ADJ && A.on) {
+  if (ADJ) {
     for (int c = 0; c < 3; ++c) {
       const double w = wave_sum_f64(ge[c]);
       if (lane_id() == 0 && w != 0.0) atomicAdd(&A.grad_e[c], w);
@@ -440,10 +467,16 @@ __global__ __launch_bounds__(256) void k_slab_index(const uint2* __restrict__ sl
   const bool totals = blockIdx.x == 0;
   const uint32_t lim = totals ? n_slabs : s0;
   uint32_t ch = 0, ent = 0;
-  for (uint32_t s = tid; s < lim; s += 256u) {
-    const uint32_t c = slabs[s].y;
-    ch += (c + 63u) >> 6;
-    ent += c;
+  for (uint32_t s = tid; s < lim; s += 256u * 8u) {  // eight reads in flight
+    uint32_t c[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k) c[k] = slabs[min(s + 256u * k, n_slabs - 1u)].y;
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k) {
+      const uint32_t v = s + 256u * k < lim ? c[k] : 0u;
+      ch += (v + 63u) >> 6;
+      ent += v;
+    }
   }
   ch = (uint32_t)wave_sum_u32(ch);
   ent = (uint32_t)wave_sum_u32(ent);
@@ -529,6 +562,26 @@ __global__ void k_grad_to_f32(const double* g, float* out, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     out[i] = (float)g[i];
 }
+// A sample's radiance after a recorded vertex is its sum less what it had
+// before; the vertex scaled all of that by its albedo (no glass splits: one path
+// per sample).  A stream of 32 bytes per record beside one gather of the
+// sample's sum and of the pixel's gradient.
+__global__ __launch_bounds__(256) void k_adjoint_resolve(Params P, Batch B, Adjoint A, uint32_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    const int32_t id = A.recs.id[i];
+    if (id < 0) continue;
+    const uint32_t slot = A.recs.slot[i];
+    const size_t px = sample_image_index(P, B, slot);
+    const int32_t face = __float_as_int(reinterpret_cast<const float4*>(P.tris)[(size_t)id * 3 + 1].w);
+    for (int c = 0; c < 3; ++c) {
+      const double rest = accum_get(A.ltot + 3 * (size_t)slot + c) - A.recs.before[c][i];
+      const double rho = P.tri_alb[3 * (size_t)id + c];
+      if (rho > 0.0 && rest != 0.0)
+        atomicAdd(&A.grad_alb[3 * (size_t)face + c], A.dimage[3 * px + c] * A.scale * rest / rho);
+    }
+  }
+}
+
 // The replay must rebuild the primal sample radiance bit for bit.
 __global__ void k_count_mismatch(const uint64_t* a, const uint64_t* b, int64_t n, uint64_t* ctr) {
   uint32_t bad = 0;
@@ -611,14 +664,17 @@ hipError_t launch_shade(const Params& P, const Batch& B, int primary, const RayQ
                         uint64_t* accum, const Adjoint& A, uint64_t* ctr, hipStream_t s) {
   const dim3 grid(PRT_SLAB_WAVES / 4);
   const bool mlds = P.n_materials <= PRT_LDS_MATERIALS;
-  if (A.on)
-    hipLaunchKernelGGL((k_shade<true, false>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id, qout, fan,
-                       slabs, accum, A, ctr);
+  if (A.on == ADJ_REPLAY)
+    hipLaunchKernelGGL((k_shade<ADJ_REPLAY, false>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id,
+                       qout, fan, slabs, accum, A, ctr);
+  else if (A.on == ADJ_RECORD)
+    hipLaunchKernelGGL((k_shade<ADJ_RECORD, false>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id,
+                       qout, fan, slabs, accum, A, ctr);
   else if (mlds)
-    hipLaunchKernelGGL((k_shade<false, true>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id, qout, fan,
+    hipLaunchKernelGGL((k_shade<ADJ_NONE, true>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id, qout, fan,
                        slabs, accum, A, ctr);
   else
-    hipLaunchKernelGGL((k_shade<false, false>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id, qout, fan,
+    hipLaunchKernelGGL((k_shade<ADJ_NONE, false>), grid, dim3(256), 0, s, P, B, primary, qin, cl, hit_t, hit_id, qout, fan,
                        slabs, accum, A, ctr);
   return hipGetLastError();
 }
@@ -664,6 +720,12 @@ hipError_t launch_scatter_albedo(float* tri_alb, const uint32_t* slot_of_tri, in
 }
 hipError_t launch_grad_to_f32(const double* g, float* out, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_grad_to_f32, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, g, out, n);
+  return hipGetLastError();
+}
+hipError_t launch_adjoint_resolve(const Params& P, const Batch& B, const Adjoint& A, uint32_t n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (n > A.recs.cap) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_adjoint_resolve, dim3(grid_for(n, 256, 8192)), dim3(256), 0, s, P, B, A, n);
   return hipGetLastError();
 }
 hipError_t launch_count_mismatch(const uint64_t* a, const uint64_t* b, int64_t n, uint64_t* ctr, hipStream_t s) {
