@@ -80,8 +80,8 @@ __device__ __forceinline__ double flip_sign(double v, uint32_t sign) {
 // the signs of det, u and v together, which rounds nothing; the bounds are
 // tested without branches, whose sides the lanes of a wave would all take
 // anyway.
-__device__ __forceinline__ bool mt_test(const float4 a, const float4 b, const float4 c, d3 o, d3 d, double& t,
-                                        double& u, double& v) {
+template <class F4>  // float4, or the four floats of a native vector
+__device__ __forceinline__ bool mt_test(const F4 a, const F4 b, const F4 c, d3 o, d3 d, double& t, double& u, double& v) {
   const d3 v0 = mk(a.x, a.y, a.z);
   const d3 edge1 = mk(b.x, b.y, b.z) - v0;
   const d3 edge2 = mk(c.x, c.y, c.z) - v0;

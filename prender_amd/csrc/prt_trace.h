@@ -21,9 +21,19 @@ struct TravStats {
 // the scene's BVH depth), thread interleaved as well: entry k of every
 // thread of a region lies together (k * ovf_threads + thread), so the lanes
 // of a wave that spill at the same depth write 512 contiguous bytes instead
-// of 64 lines.  The overflow accesses are volatile so that the compiler keeps
-// them apart from the LDS ones: merged, both would become flat-address loads
-// and stores, which wait on every outstanding memory operation.
+// of 64 lines.
+//
+// An entry is a 64-bit key, t in the high word and the node in the low one, as
+// node_keys sorts them.  The levels of all lanes of a wave are usually in LDS,
+// which a wave-uniform branch finds out: entries are then written without a
+// branch per child (a miss is overwritten by the next entry), and read two at a
+// time.
+//
+// The overflow area, the nodes and the triangles lie in device memory, which
+// their pointers' type says: a pointer that a kernel reads from memory (the
+// scenes of a batch) is a flat one otherwise, whose loads wait for LDS accesses
+// as well and take no scalar base.
+#define PRT_GLOBAL __attribute__((address_space(1)))
 // four floats as a native vector (copyable out of an address-space-qualified
 // object, unlike float4)
 typedef float prt_f4 __attribute__((ext_vector_type(4)));
@@ -31,34 +41,20 @@ typedef float prt_f4 __attribute__((ext_vector_type(4)));
 template <int NL>
 struct StackN {
   static constexpr int stride = 256;  // threads per block of every traversal kernel
-  uint2* lds;                         // [NL][256]
-  uint2* ovf;                         // this thread's first overflow entry
+  static constexpr int levels = NL;
+  uint64_t* lds;                      // [NL][256]
+  PRT_GLOBAL uint64_t* ovf;           // this thread's first overflow entry
   size_t ostride;                     // entries between its consecutive overflow entries
   // (3 * BVH depth + 1 - NL overflow entries used at most)
   // the block's LDS copy of BVH nodes 0..n_top-1 (PRT_TOP_CACHE)
   const __attribute__((address_space(3))) prt_f4* top = nullptr;
   int n_top = 0;
-  __device__ __forceinline__ void push(int sp, int32_t node, float t) {
-    const uint2 e = make_uint2((uint32_t)node, __float_as_uint(t));
-    if (sp < NL) {
-      lds[sp * stride] = e;
-    } else {
-      volatile uint32_t* g = reinterpret_cast<volatile uint32_t*>(ovf + (size_t)(sp - NL) * ostride);
-      g[0] = e.x;
-      g[1] = e.y;
-    }
+  __device__ __forceinline__ void put(int k, uint64_t key) {
+    if (k < NL) lds[k * stride] = key;
+    else ovf[(size_t)(k - NL) * ostride] = key;
   }
-  __device__ __forceinline__ void pop(int sp, int32_t& node, float& t) {
-    uint2 e;
-    if (sp < NL) {
-      e = lds[sp * stride];
-    } else {
-      const volatile uint32_t* g = reinterpret_cast<const volatile uint32_t*>(ovf + (size_t)(sp - NL) * ostride);
-      e.x = g[0];
-      e.y = g[1];
-    }
-    node = (int32_t)e.x;
-    t = __uint_as_float(e.y);
+  __device__ __forceinline__ uint64_t get(int k) const {
+    return k < NL ? lds[k * stride] : ovf[(size_t)(k - NL) * ostride];
   }
 };
 typedef StackN<PRT_STACK_LDS> Stack;
@@ -69,10 +65,10 @@ typedef StackN<PRT_STACK_LDS> Stack;
 // shadow kernels region 1, because the two run at the same time on two
 // streams.
 #define PRT_DECLARE_STACK_N(S, P, NL, REGION)                                                             \
-  __shared__ uint2 s_stack_[(NL) * 256];                                                                  \
+  __shared__ uint64_t s_stack_[(NL) * 256];                                                               \
   StackN<NL> S{s_stack_ + threadIdx.x,                                                                    \
-               reinterpret_cast<uint2*>((P).stack_ovf +                                                   \
-                                        (size_t)(REGION) * (size_t)(P).ovf_threads * (size_t)(P).ovf_words) + \
+               (PRT_GLOBAL uint64_t*)((P).stack_ovf +                                                     \
+                                      (size_t)(REGION) * (size_t)(P).ovf_threads * (size_t)(P).ovf_words) + \
                    (size_t)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) % (P).ovf_threads),          \
                (size_t)(P).ovf_threads}
 #define PRT_DECLARE_STACK(S, P, REGION) PRT_DECLARE_STACK_N(S, P, PRT_STACK_LDS, REGION)
@@ -116,79 +112,125 @@ __device__ __forceinline__ float ray_inverse(double d) {
   return fabsf(i) < __builtin_inff() ? i : __builtin_copysignf(1.0e30f, (float)d);
 }
 
-// Slab test of the 4 children of node `cur` against the ray's float slabs:
-// entry distances sorted ascending with their child references (+inf: miss).
+// Smaller of two keys into a, larger into b.  A key's high word is a float in
+// [0, +inf], so as a double it is positive and finite (0x7F800000 is no
+// double's infinity) and its order is the keys' order as integers; the 64-bit
+// minimum leaves its operand's bits alone, denormals included.
+__device__ __forceinline__ void key_order(uint64_t& a, uint64_t& b) {
+  const double x = __longlong_as_double((long long)a), y = __longlong_as_double((long long)b);
+  double lo, hi;
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(x), "v"(y));
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(x), "v"(y));
+  a = (uint64_t)__double_as_longlong(lo);
+  b = (uint64_t)__double_as_longlong(hi);
+}
+#define PRT_KEY_MISS 0x7F800000u
+__device__ __forceinline__ bool key_hit(uint64_t key) { return (uint32_t)(key >> 32) != PRT_KEY_MISS; }
+
+// Slab test of the 4 children of node `cur` against the ray's float slabs: a key
+// per child, entry distance (+inf: miss) over child reference, ascending.
 // Each axis reads its entry and exit planes from the rows entry_rows picks:
 // fma(c, i, -oi) is monotonic in the plane coordinate c and every child has
 // lo <= hi (an empty slot lo = hi = +inf), so the entry plane's distance is
 // exactly the smaller of the two, without a min / max per axis.
-// The sort exchanges (distance, child) pairs by selects: 25 instructions,
-// where sorting 32-bit keys that carry the slot and picking the children by
-// slot afterwards took 45 (field of 2.1 M triangles 62.4 -> 61.0 ms a frame,
-// 2^20 rays 429 -> 407 us).
-// Nodes of the top levels come from the block's LDS copy.
+// The keys' sort is ten 64-bit minima and maxima (25 instructions as exchanges
+// by selects, 45 as 32-bit keys whose children are picked afterwards).
+// Nodes of the top levels come from the block's LDS copy (without it the
+// 82k-triangle box took 34.0 instead of 33.3 ms a frame), others at a 32-bit
+// offset from a scalar base while that reaches all nodes (2^25 of them).
 template <class Stk>
-__device__ __forceinline__ void node_children(const Stk& S, const DevNode* nodes, int32_t cur, uint32_t rows,
-                                              float ix, float iy, float iz, float oix, float oiy, float oiz, float tb,
-                                              float tn[4], int32_t cc[4]) {
+__device__ __forceinline__ void node_keys(const Stk& S, const DevNode* nodes, int32_t n_nodes, int32_t cur, uint32_t rows,
+                                          float ix, float iy, float iz, float oix, float oiy, float oiz, float tb,
+                                          uint64_t key[4]) {
   const uint32_t nx = rows & 0xFFu, ny = (rows >> 8) & 0xFFu, nz = rows >> 16;
-  const uint32_t fx = nx ^ 48u, fy = ny ^ 80u, fz = nz ^ 112u;
-  float4 nd[7];  // entry x, y, z rows, exit x, y, z rows, children
+  // entry x, y, z rows, exit x, y, z rows, children
+  const uint32_t off[7] = {nx, ny, nz, nx ^ 48u, ny ^ 80u, nz ^ 112u, 96u};
+  prt_f4 nd[7];
   if (cur < S.n_top) {
     typedef const __attribute__((address_space(3))) char lds_c;
     typedef const __attribute__((address_space(3))) prt_f4 lds_f4;
-    lds_c* t = reinterpret_cast<lds_c*>(S.top + (size_t)cur * 8);
-    const uint32_t off[7] = {nx, ny, nz, fx, fy, fz, 96u};
+    lds_c* t = reinterpret_cast<lds_c*>(S.top);
 #pragma unroll
-    for (int k = 0; k < 7; ++k) {
-      const prt_f4 v = *reinterpret_cast<lds_f4*>(t + off[k]);
-      nd[k] = make_float4(v.x, v.y, v.z, v.w);
-    }
+    for (int k = 0; k < 7; ++k) nd[k] = *reinterpret_cast<lds_f4*>(t + (((uint32_t)cur << 7) + off[k]));
   } else {
-    const char* g = reinterpret_cast<const char*>(nodes + cur);
-    const uint32_t off[7] = {nx, ny, nz, fx, fy, fz, 96u};
+    typedef const PRT_GLOBAL char glb_c;
+    typedef const PRT_GLOBAL prt_f4 glb_f4;
+    glb_c* g = (glb_c*)nodes;
+    if (n_nodes <= (1 << 25)) {
 #pragma unroll
-    for (int k = 0; k < 7; ++k) nd[k] = *reinterpret_cast<const float4*>(g + off[k]);
+      for (int k = 0; k < 7; ++k) nd[k] = *reinterpret_cast<glb_f4*>(g + (((uint32_t)cur << 7) | off[k]));
+    } else {
+      g += (size_t)cur << 7;
+#pragma unroll
+      for (int k = 0; k < 7; ++k) nd[k] = *reinterpret_cast<glb_f4*>(g + off[k]);
+    }
   }
-  const float4 ex = nd[0], ey = nd[1], ez = nd[2], xx = nd[3], xy = nd[4], xz = nd[5];
-  const int4 ch = make_int4(__float_as_int(nd[6].x), __float_as_int(nd[6].y), __float_as_int(nd[6].z),
-                            __float_as_int(nd[6].w));
-  const float exa[4] = {ex.x, ex.y, ex.z, ex.w}, eya[4] = {ey.x, ey.y, ey.z, ey.w}, eza[4] = {ez.x, ez.y, ez.z, ez.w};
-  const float xxa[4] = {xx.x, xx.y, xx.z, xx.w}, xya[4] = {xy.x, xy.y, xy.z, xy.w}, xza[4] = {xz.x, xz.y, xz.z, xz.w};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float x0 = __builtin_fmaf(exa[k], ix, -oix), x1 = __builtin_fmaf(xxa[k], ix, -oix);
-    const float y0 = __builtin_fmaf(eya[k], iy, -oiy), y1 = __builtin_fmaf(xya[k], iy, -oiy);
-    const float z0 = __builtin_fmaf(eza[k], iz, -oiz), z1 = __builtin_fmaf(xza[k], iz, -oiz);
+    const float x0 = __builtin_fmaf(nd[0][k], ix, -oix), x1 = __builtin_fmaf(nd[3][k], ix, -oix);
+    const float y0 = __builtin_fmaf(nd[1][k], iy, -oiy), y1 = __builtin_fmaf(nd[4][k], iy, -oiy);
+    const float z0 = __builtin_fmaf(nd[2][k], iz, -oiz), z1 = __builtin_fmaf(nd[5][k], iz, -oiz);
     const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, 0.0f));
     const float tfar = fminf(fminf(x1, y1), fminf(z1, tb));
-    tn[k] = (tnear <= tfar) ? tnear : __builtin_inff();
+    const uint32_t t = (tnear <= tfar) ? __float_as_uint(tnear) : PRT_KEY_MISS;
+    key[k] = ((uint64_t)t << 32) | __float_as_uint(nd[6][k]);
   }
-  cc[0] = ch.x; cc[1] = ch.y; cc[2] = ch.z; cc[3] = ch.w;
-#define PRT_KSORT(a, b)                           \
-  {                                               \
-    const bool sw_ = tn[b] < tn[a];               \
-    const float t_ = sw_ ? tn[b] : tn[a];         \
-    tn[b] = sw_ ? tn[a] : tn[b];                  \
-    tn[a] = t_;                                   \
-    const int32_t c_ = sw_ ? cc[b] : cc[a];       \
-    cc[b] = sw_ ? cc[a] : cc[b];                  \
-    cc[a] = c_;                                   \
-  }
-  PRT_KSORT(0, 1) PRT_KSORT(2, 3) PRT_KSORT(0, 2) PRT_KSORT(1, 3)
-#if !defined(PRT_SORT4)
-  PRT_KSORT(1, 2)
-#endif
-#undef PRT_KSORT
+  key_order(key[0], key[1]);
+  key_order(key[2], key[3]);
+  key_order(key[0], key[2]);
+  key_order(key[1], key[3]);
+  key_order(key[1], key[2]);
 }
 
-// Pushes children 3, 2, 1 of a sorted node test (farthest first) that were
-// hit.
+// Pushes keys 3, 2, 1 of a node (farthest first) that are hits.
 template <class Stk>
-__device__ __forceinline__ void push_children(Stk& S, int& sp, const float tn[4], const int32_t cc[4]) {
+__device__ __forceinline__ void push_keys(Stk& S, int& sp, const uint64_t key[4]) {
+  if (!__any(sp > Stk::levels - 3)) {
 #pragma unroll
-  for (int j = 3; j >= 1; --j)
-    if (tn[j] != __builtin_inff()) S.push(sp++, cc[j], tn[j]);
+    for (int j = 3; j >= 1; --j) {
+      S.lds[sp * Stk::stride] = key[j];
+      sp += key_hit(key[j]) ? 1 : 0;
+    }
+  } else {
+#pragma unroll
+    for (int j = 3; j >= 1; --j)
+      if (key_hit(key[j])) S.put(sp++, key[j]);
+  }
+}
+
+// A lane's place in the tree: an internal node (0 <= cur < PRT_TRAV_POP), a leaf
+// code (< 0), PRT_TRAV_POP (its next node is on the stack, which is not empty) or
+// PRT_TRAV_DONE.
+#define PRT_TRAV_DONE 0x7FFFFFFF
+#define PRT_TRAV_POP 0x7FFFFFFE
+__device__ __forceinline__ int32_t next_entry(int sp) { return sp > 0 ? PRT_TRAV_POP : PRT_TRAV_DONE; }
+
+// Takes the top two entries of a lane at PRT_TRAV_POP, as far as it needs them:
+// an entry beyond tb is dropped, a first leaf is parked in lf (>= 0: none).  A lane
+// that finds nothing stays at PRT_TRAV_POP.  A loop until every lane of the wave
+// has its node ran as often as the lane with the most stale entries: after a hit
+// that is most of the stack, at some 25 instructions an entry for one lane.
+template <class Stk>
+__device__ __forceinline__ void pop_two(const Stk& S, int& sp, float tb, int32_t& cur, int32_t& lf) {
+  uint64_t e[2];
+  const int k1 = max(sp - 2, 0);
+  if (!__any(sp > Stk::levels)) {
+    e[0] = S.lds[(sp - 1) * Stk::stride];
+    e[1] = S.lds[k1 * Stk::stride];
+  } else {
+    e[0] = S.get(sp - 1);
+    e[1] = S.get(k1);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (cur == PRT_TRAV_POP) {
+      const int32_t node = (int32_t)(uint32_t)e[k];
+      const bool open = __uint_as_float((uint32_t)(e[k] >> 32)) <= tb, park = open && node < 0 && lf >= 0;
+      --sp;
+      lf = park ? node : lf;
+      cur = open && !park ? node : next_entry(sp);
+    }
+  }
 }
 
 // While-while traversal with speculative leaf postponement (Aila & Laine,
@@ -210,7 +252,7 @@ __device__ __forceinline__ bool nearer_hit(double t, int32_t ent, double t_best,
 }
 // Entity of a hit id (>= 0 triangle slot, <= -2 analytic entity, -1 none:
 // above every entity).
-__device__ __forceinline__ int32_t hit_entity(const float4* tris4, int32_t id) {
+__device__ __forceinline__ int32_t hit_entity(const PRT_GLOBAL prt_f4* tris4, int32_t id) {
   return id >= 0 ? __float_as_int(tris4[(size_t)id * 3].w) : (id <= -2 ? -2 - id : 0x7FFFFFFF);
 }
 
@@ -316,7 +358,6 @@ __device__ __forceinline__ bool analytic_hits(const Params& P, const AnalyticSlo
 // leaves open (a box whose entry equals the best t stays open), so the
 // closest hit is the one over all triangles, with the tie rule of
 // nearer_hit.
-#define PRT_TRAV_DONE 0x7FFFFFFF
 // any (the same for every ray of a launch, or a lane's own): stop at the first
 // hit below t_best instead.
 template <class Stk>
@@ -330,32 +371,22 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 
   float tb = t_best < 1.0e30 ? fup(t_best) : __builtin_inff();
   bool found = false;
   int sp = 0;
-  const float4* tris4 = reinterpret_cast<const float4*>(P.tris);
+  const PRT_GLOBAL prt_f4* tris4 = (const PRT_GLOBAL prt_f4*)P.tris;
   int32_t e_best = any ? 0 : hit_entity(tris4, id_best);
-  // cur: internal node (0 <= cur < PRT_TRAV_DONE), leaf code (< 0) or
-  // PRT_TRAV_DONE; lf: parked leaf (< 0) or none (>= 0)
-  int32_t cur = 0, lf = 0;
-  // the nearest pending entry that can still hold a closer hit
-  auto pop_next = [&]() -> int32_t {
-    while (sp > 0) {
-      int32_t node;
-      float t;
-      S.pop(--sp, node, t);
-      if (t <= tb) return node;
-    }
-    return PRT_TRAV_DONE;
-  };
+  int32_t cur = 0, lf = 0;  // lf: parked leaf (< 0) or none (>= 0)
   while (true) {
     while ((uint32_t)cur < (uint32_t)PRT_TRAV_DONE) {
-      float tn[4];
-      int32_t cc[4];
-      node_children(S, P.nodes, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, tn, cc);
-      ts.nodes++;
-      push_children(S, sp, tn, cc);
-      cur = (tn[0] != __builtin_inff()) ? cc[0] : pop_next();
-      if (cur < 0 && lf >= 0) {  // park the first leaf and keep walking
-        lf = cur;
-        cur = pop_next();
+      if (cur == PRT_TRAV_POP) pop_two(S, sp, tb, cur, lf);
+      if ((uint32_t)cur < (uint32_t)PRT_TRAV_POP) {
+        uint64_t key[4];
+        node_keys(S, P.nodes, P.n_nodes, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, key);
+        ts.nodes++;
+        push_keys(S, sp, key);
+        cur = key_hit(key[0]) ? (int32_t)(uint32_t)key[0] : next_entry(sp);
+        if (cur < 0 && lf >= 0) {  // park the first leaf and keep walking
+          lf = cur;
+          cur = next_entry(sp);
+        }
       }
       if (!__any(lf >= 0)) break;  // every lane still walking holds a leaf
     }
@@ -364,12 +395,12 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 
       const uint32_t first = code & 0x07FFFFFFu;
       const uint32_t count = (code >> 27) + 1u;
       // triangle k + 1 is loaded before triangle k is tested
-      const float4* tr0 = tris4 + (size_t)first * 3;
-      float4 na = tr0[0], nb = tr0[1], nc = tr0[2];
+      const PRT_GLOBAL prt_f4* tr0 = tris4 + (size_t)first * 3;
+      prt_f4 na = tr0[0], nb = tr0[1], nc = tr0[2];
       for (uint32_t k = 0; k < count; ++k) {
-        const float4 a = na, b = nb, c = nc;
+        const prt_f4 a = na, b = nb, c = nc;
         if (k + 1 < count) {
-          const float4* tr = tris4 + (size_t)(first + k + 1) * 3;
+          const PRT_GLOBAL prt_f4* tr = tris4 + (size_t)(first + k + 1) * 3;
           na = tr[0];
           nb = tr[1];
           nc = tr[2];
@@ -392,7 +423,7 @@ __device__ __forceinline__ bool traverse_ww(const Params& P, bool any, d3 o, d3 
         }
       }
       lf = cur;  // a second leaf met while walking is tested next
-      if (cur < 0) cur = pop_next();
+      if (cur < 0) cur = next_entry(sp);
     }
     if (cur == PRT_TRAV_DONE) break;
   }
@@ -494,7 +525,9 @@ __device__ __forceinline__ bool claim(const ClaimRange& r, uint32_t k, uint32_t&
 // wave, and a hit's entity, needed only for equal distances, is read again.
 // Frame of that box 41.5 -> 34.7 ms, with the analytic entities in LDS and the
 // shorter tests; the field of 2.1 M triangles 72.8 -> 60.1 ms and the batch of
-// eight scenes 54.4 -> 42.3 ms, whose tile queue had no refill.
+// eight scenes 54.4 -> 42.3 ms, whose tile queue had no refill.  Steps without a
+// loop or a branch per child (pop_two, push_keys), keys sorted by 64-bit minima
+// and scalar node bases: 34.4 -> 33.2, 59.6 -> 55.8 and 42.4 -> 41.1 ms.
 //
 // Source: next(base, n, idle) gives the wave's next rays base .. base + n - 1
 // (n > 0; idle: no lane of the wave holds a ray), false when there are none
@@ -576,15 +609,6 @@ __device__ __forceinline__ void traverse_pool(Source& src, const AnalyticSlot* s
   bool act = false, blocked = false;
   uint32_t base = 0, left = 0;  // wave-uniform: rays handed out and not yet started
   uint32_t n_nodes = 0, n_tris = 0, n_rays = 0;  // wave-uniform counts
-  auto pop_next = [&]() -> int32_t {
-    while (sp > 0) {
-      int32_t node;
-      float t;
-      S.pop(--sp, node, t);
-      if (t <= tb) return node;
-    }
-    return PRT_TRAV_DONE;
-  };
   while (true) {
     // ---- idle lanes take new rays
     const uint64_t idle = __ballot(!act);
@@ -630,23 +654,26 @@ __device__ __forceinline__ void traverse_pool(Source& src, const AnalyticSlot* s
       }
     }
     const Params& P = src.params();
-    const float4* tris4 = reinterpret_cast<const float4*>(P.tris);
+    const PRT_GLOBAL prt_f4* tris4 = (const PRT_GLOBAL prt_f4*)P.tris;
+    const DevNode* nodes = P.nodes;
+    const int32_t count = P.n_nodes;
     // ---- node and triangle steps until enough rays have finished
     while (true) {
       const bool walk = (uint32_t)cur < (uint32_t)PRT_TRAV_DONE;
       const uint32_t nw = (uint32_t)__popcll(__ballot(walk)), nl = (uint32_t)__popcll(__ballot(lf < 0));
       if (nw + nl == 0u) break;
       if (nw * (uint32_t)PRT_VOTE_NODE >= nl) {
-        n_nodes += nw;
-        if (walk) {
-          float tn[4];
-          int32_t cc[4];
-          node_children(S, P.nodes, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, tn, cc);
-          push_children(S, sp, tn, cc);
-          cur = (tn[0] != __builtin_inff()) ? cc[0] : pop_next();
+        if (cur == PRT_TRAV_POP) pop_two(S, sp, tb, cur, lf);
+        const bool visit = (uint32_t)cur < (uint32_t)PRT_TRAV_POP;
+        n_nodes += (uint32_t)__popcll(__ballot(visit));
+        if (visit) {
+          uint64_t key[4];
+          node_keys(S, nodes, count, cur, rows, ix, iy, iz, oix, oiy, oiz, tb, key);
+          push_keys(S, sp, key);
+          cur = key_hit(key[0]) ? (int32_t)(uint32_t)key[0] : next_entry(sp);
           if (cur < 0 && lf >= 0) {  // park the first leaf and keep walking
             lf = cur;
-            cur = pop_next();
+            cur = next_entry(sp);
           }
         }
       } else {
@@ -654,8 +681,8 @@ __device__ __forceinline__ void traverse_pool(Source& src, const AnalyticSlot* s
         if (lf < 0) {
           const uint32_t code = ~(uint32_t)lf;
           const uint32_t tri = code & 0x07FFFFFFu;
-          const float4* tr = tris4 + (size_t)tri * 3;
-          const float4 a = tr[0], b = tr[1], c = tr[2];
+          const PRT_GLOBAL prt_f4* tr = tris4 + (size_t)tri * 3;
+          const prt_f4 a = tr[0], b = tr[1], c = tr[2];
           double t, u, v;
           if (mt_test(a, b, c, o, d, t, u, v) &&
               (ANY ? t < t_best
@@ -675,7 +702,7 @@ __device__ __forceinline__ void traverse_pool(Source& src, const AnalyticSlot* s
             lf = (int32_t)~(code + 1u - (1u << 27));  // the leaf's next triangle
           } else {
             lf = cur < 0 ? cur : 0;  // a second leaf met while walking
-            if (cur < 0) cur = pop_next();
+            if (cur < 0) cur = next_entry(sp);
           }
         }
       }
