@@ -126,8 +126,8 @@ void Workspace::release() {
   batch_samples = queue_cap = shadow_cap = 0;
 }
 
-static const size_t kRayColBytes[RAYQ_COLS] = {8, 8, 8, 8, 8, 8, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4, 4};
-static const size_t kShadowColBytes[SHADOWQ_COLS] = {8, 8, 8, 8, 8, 8, 8, 4, 4, 4, 4, 4};
+static const size_t kRayColBytes[RAYQ_COLS] = {16, 16, 16, 16, 16, 16};
+static const size_t kShadowColBytes[SHADOWQ_COLS] = {16, 16, 16, 8, 16, 4};
 size_t ray_entry_bytes() {
   size_t b = 0;
   for (size_t v : kRayColBytes) b += v;
@@ -159,25 +159,20 @@ int alloc_shadow_queue(DevBuf* cols, int64_t cap) {
 
 RayQ ray_queue(DevBuf* b, int64_t cap) {
   RayQ q;
-  q.ox = (double*)b[0].p; q.oy = (double*)b[1].p; q.oz = (double*)b[2].p;
-  q.dx = (double*)b[3].p; q.dy = (double*)b[4].p; q.dz = (double*)b[5].p;
-  q.tr = (float*)b[6].p; q.tg = (float*)b[7].p; q.tb = (float*)b[8].p;
-  q.pr = (float*)b[9].p; q.pg = (float*)b[10].p; q.pb = (float*)b[11].p;
-  q.slot = (uint32_t*)b[12].p;
-  q.meta = (uint32_t*)b[13].p;
-  q.nx = (float*)b[14].p; q.ny = (float*)b[15].p; q.nz = (float*)b[16].p;
+  q.a = (double2*)b[0].p; q.b = (double2*)b[1].p; q.c = (double2*)b[2].p;
+  q.t = (float4*)b[3].p;
+  q.n = (float4*)b[4].p;
+  q.p = (float4*)b[5].p;
   q.cap = (uint32_t)cap;
   return q;
 }
 
 ShadowQ shadow_queue(DevBuf* b, int64_t cap) {
   ShadowQ q;
-  q.ox = (double*)b[0].p; q.oy = (double*)b[1].p; q.oz = (double*)b[2].p;
-  q.dx = (double*)b[3].p; q.dy = (double*)b[4].p; q.dz = (double*)b[5].p;
-  q.tmax = (double*)b[6].p;
-  q.cr = (float*)b[7].p; q.cg = (float*)b[8].p; q.cb = (float*)b[9].p;
-  q.slot = (uint32_t*)b[10].p;
-  q.light = (int32_t*)b[11].p;
+  q.a = (double2*)b[0].p; q.b = (double2*)b[1].p; q.c = (double2*)b[2].p;
+  q.tmax = (double*)b[3].p;
+  q.l = (float4*)b[4].p;
+  q.light = (int32_t*)b[5].p;
   q.cap = (uint32_t)cap;
   return q;
 }

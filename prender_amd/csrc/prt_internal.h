@@ -65,7 +65,7 @@ int dev_upload(DevBuf& b, const std::vector<T>& v, hipStream_t s) {
 }
 
 // Ray / shadow queues as 17 / 12 separately allocated SoA columns.
-enum { RAYQ_COLS = 17, SHADOWQ_COLS = 12 };
+enum { RAYQ_COLS = 6, SHADOWQ_COLS = 6 };
 int alloc_ray_queue(DevBuf* cols, int64_t cap);
 size_t ray_entry_bytes();     // device bytes per ray-queue entry
 size_t shadow_entry_bytes();  // device bytes per shadow-queue entry

@@ -96,8 +96,7 @@ __global__ __launch_bounds__(256) void k_gen_primary(Params P, Batch B, RayQ q) 
     const int sub = (int)(i % ss2);
     d3 o, d;
     camera_ray(P, (int)(pix % P.W), (int)(pix / P.W), sub % P.SS, sub / P.SS, o, d);
-    q.ox[i] = o.x; q.oy[i] = o.y; q.oz[i] = o.z;
-    q.dx[i] = d.x; q.dy[i] = d.y; q.dz[i] = d.z;
+    put_ray(q, i, o, d);
   }
 }
 
@@ -122,8 +121,7 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_TRAVERSE) void k_exte
   traverse_pool<false>(
       src, slots, S, ts,
       [&](uint32_t j, d3& o, d3& d, double& tmax) {
-        o = mk(q.ox[j], q.oy[j], q.oz[j]);
-        d = mk(q.dx[j], q.dy[j], q.dz[j]);
+        get_ray(q, j, o, d);
         tmax = PS_INF;
       },
       [&](uint32_t j, double t, int32_t id, bool, d3, d3) {
@@ -146,8 +144,9 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADOW) void k_shadow
   TravStats ts{0, 0, 0};
   double ge[3] = {0.0, 0.0, 0.0};
   auto lit = [&](uint32_t i) {
-    const uint32_t s = q.slot[i];
-    const float c[3] = {q.cr[i], q.cg[i], q.cb[i]};
+    const float4 l = q.l[i];
+    const uint32_t s = __float_as_uint(l.w);
+    const float c[3] = {l.x, l.y, l.z};
     accum_add(&accum[3 * (size_t)s + 0], c[0]);
     accum_add(&accum[3 * (size_t)s + 1], c[1]);
     accum_add(&accum[3 * (size_t)s + 2], c[2]);
@@ -162,8 +161,7 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADOW) void k_shadow
   traverse_pool<true>(
       src, slots, S, ts,
       [&](uint32_t j, d3& o, d3& d, double& tmax) {
-        o = mk(q.ox[j], q.oy[j], q.oz[j]);
-        d = mk(q.dx[j], q.dy[j], q.dz[j]);
+        get_ray(q, j, o, d);
         tmax = q.tmax[j];
       },
       [&](uint32_t j, double, int32_t, bool blocked, d3, d3) {
@@ -280,8 +278,7 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
       const int64_t pix = B.pixel_base + pl;
       const uint32_t hi = pl * ss2 + sub;
       if (P.mlt_u != nullptr) {  // a Metropolis proposal's own camera ray
-        o = mk(qin.ox[hi], qin.oy[hi], qin.oz[hi]);
-        d = mk(qin.dx[hi], qin.dy[hi], qin.dz[hi]);
+        get_ray(qin, hi, o, d);
       } else {
         camera_ray(P, (int)(pix % P.W), (int)(pix / P.W), sub % P.SS, sub / P.SS, o, d);
       }
@@ -292,12 +289,9 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_SHADE) void k_shade(
       depth = 0;
       branch = 1;
     } else {
-      slot = qin.slot[i];
-      o = mk(qin.ox[i], qin.oy[i], qin.oz[i]);
-      d = mk(qin.dx[i], qin.dy[i], qin.dz[i]);
-      T = mk(qin.tr[i], qin.tg[i], qin.tb[i]);
-      Pw = mk(qin.pr[i], qin.pg[i], qin.pb[i]);
-      const uint32_t meta = qin.meta[i];
+      uint32_t meta;
+      get_ray(qin, i, o, d);
+      get_segment(qin, i, T, Pw, meta, slot);
       depth = (int)(meta & 0xFFu);
       branch = META_BRANCH(meta);
       t = PF ? hc_t : hit_t[i];
@@ -405,11 +399,8 @@ __global__ __launch_bounds__(256) PRT_WAVES_ATTR(PRT_WAVES_NEE) void k_nee(
     d3 x, nrm, ct;
     if (lane_id() < dc.y) {
       const uint32_t i = dc.x + lane_id();
-      const uint32_t meta = q.meta[i];
-      slot = q.slot[i];
-      x = mk(q.ox[i], q.oy[i], q.oz[i]);
-      nrm = mk(q.nx[i], q.ny[i], q.nz[i]);
-      ct = mk(q.tr[i], q.tg[i], q.tb[i]);
+      uint32_t meta;
+      get_lit(q, i, x, nrm, ct, meta, slot);
       if (meta & META_NEE) {
         have = true;
         const uint32_t pl = slot / P.spp, k = slot % P.spp;

@@ -42,8 +42,7 @@ __global__ __launch_bounds__(256) void k_mlt_gen(Params P, uint32_t n, RayQ q) {
   const uint32_t* u = P.mlt_u + (size_t)i * (uint32_t)P.mlt_stride;
   d3 o, d;
   P.mlt_pix[i] = mlt_camera_ray(P, u, o, d);
-  q.ox[i] = o.x; q.oy[i] = o.y; q.oz[i] = o.z;
-  q.dx[i] = d.x; q.dy[i] = d.y; q.dz[i] = d.z;
+  put_ray(q, i, o, d);
 }
 
 __global__ __launch_bounds__(256) void k_mlt_seed_record(const uint64_t* __restrict__ accum,

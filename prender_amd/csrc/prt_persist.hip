@@ -228,12 +228,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
         const Params& P = SRC == PATH_BATCH ? scene_params(st.scenes, scene) : P1;
         if (SRC == PATH_QUEUE) {
           const uint32_t i = st.cl.desc[cb].x + co + rank;
-          o = mk(st.q.ox[i], st.q.oy[i], st.q.oz[i]);
-          d = mk(st.q.dx[i], st.q.dy[i], st.q.dz[i]);
-          tr[0] = st.q.tr[i]; tr[1] = st.q.tg[i]; tr[2] = st.q.tb[i];
-          pw[0] = st.q.pr[i]; pw[1] = st.q.pg[i]; pw[2] = st.q.pb[i];
-          meta = st.q.meta[i] & ~META_NEE;
-          slot = st.q.slot[i];
+          d3 T, Pw;
+          get_ray(st.q, i, o, d);
+          get_segment(st.q, i, T, Pw, meta, slot);
+          tr[0] = (float)T.x; tr[1] = (float)T.y; tr[2] = (float)T.z;
+          pw[0] = (float)Pw.x; pw[1] = (float)Pw.y; pw[2] = (float)Pw.z;
+          meta &= ~(META_NEE | META_PICK);
         } else {
           if (SRC == PATH_BATCH) slot = (cb - st.chunk_base[scene]) * 64u + co + rank;
           else slot = cb * st.unit + co + rank;
@@ -241,8 +241,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
             it = st.chain.it0;
             due = true;
           } else if (SRC == PATH_FRAME && P.mlt_u != nullptr) {  // a Metropolis proposal's own camera ray
-            o = mk(st.q.ox[slot], st.q.oy[slot], st.q.oz[slot]);
-            d = mk(st.q.dx[slot], st.q.dy[slot], st.q.dz[slot]);
+            get_ray(st.q, slot, o, d);
           } else {
             const int64_t pixel = st.batch.pixel_base + (int64_t)(slot / (uint32_t)P.spp);
             const int sub = (int)(slot % (uint32_t)P.spp % (uint32_t)(P.SS * P.SS));

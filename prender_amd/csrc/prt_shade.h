@@ -63,6 +63,43 @@ __device__ __forceinline__ void vertex_words(const Params& P, RngKey key, uint32
   philox(pixel, sample, rng_c2(depth, branch), 0u, key.k0, key.k1, b);
 }
 
+// Origin and direction of entry i of a ray or shadow queue.
+template <class Queue>
+__device__ __forceinline__ void put_ray(const Queue& q, size_t i, d3 o, d3 d) {
+  q.a[i] = make_double2(o.x, o.y);
+  q.b[i] = make_double2(o.z, d.x);
+  q.c[i] = make_double2(d.y, d.z);
+}
+template <class Queue>
+__device__ __forceinline__ void get_ray(const Queue& q, size_t i, d3& o, d3& d) {
+  const double2 a = q.a[i], b = q.b[i], c = q.c[i];
+  o = mk(a.x, a.y, b.x);
+  d = mk(b.y, c.x, c.y);
+}
+// The rest of entry i of a ray queue.
+__device__ __forceinline__ void get_segment(const RayQ& q, size_t i, d3& T, d3& Pw, uint32_t& meta, uint32_t& slot) {
+  const float4 t = q.t[i];
+  slot = __float_as_uint(q.n[i].w);
+  meta = __float_as_uint(t.w);
+  T = mk(t.x, t.y, t.z);
+  Pw = mk(0.0, 0.0, 0.0);
+  if (meta & META_PICK) {
+    const float4 p = q.p[i];
+    Pw = mk(p.x, p.y, p.z);
+  }
+}
+// What its light samples need of it.
+__device__ __forceinline__ void get_lit(const RayQ& q, size_t i, d3& x, d3& nrm, d3& ct, uint32_t& meta, uint32_t& slot) {
+  const double2 a = q.a[i];
+  const double oz = q.b[i].x;
+  const float4 n = q.n[i], t = q.t[i];
+  x = mk(a.x, a.y, oz);
+  nrm = mk(n.x, n.y, n.z);
+  ct = mk(t.x, t.y, t.z);
+  meta = __float_as_uint(t.w);
+  slot = __float_as_uint(n.w);
+}
+
 // Children go to qout positions off + j, j < cap, with j from *count_out.
 struct ShadeCtx {
   RayQ qout;
@@ -92,15 +129,11 @@ __device__ __forceinline__ void emit_child(ShadeCtx& C, d3 o, d3 d, d3 ct, d3 pw
     return;
   }
   j += C.off;
-  C.qout.ox[j] = o.x; C.qout.oy[j] = o.y; C.qout.oz[j] = o.z;
-  C.qout.dx[j] = d.x; C.qout.dy[j] = d.y; C.qout.dz[j] = d.z;
-  C.qout.tr[j] = (float)ct.x; C.qout.tg[j] = (float)ct.y; C.qout.tb[j] = (float)ct.z;
-  C.qout.pr[j] = (float)pw.x; C.qout.pg[j] = (float)pw.y; C.qout.pb[j] = (float)pw.z;
-  C.qout.slot[j] = C.slot;
-  C.qout.meta[j] = meta;
-  if (meta & META_NEE) {
-    C.qout.nx[j] = (float)nrm.x; C.qout.ny[j] = (float)nrm.y; C.qout.nz[j] = (float)nrm.z;
-  }
+  const bool pick = pw.x != 0.0 || pw.y != 0.0 || pw.z != 0.0;
+  put_ray(C.qout, j, o, d);
+  C.qout.t[j] = make_float4((float)ct.x, (float)ct.y, (float)ct.z, __uint_as_float(meta | (pick ? META_PICK : 0u)));
+  C.qout.n[j] = make_float4((float)nrm.x, (float)nrm.y, (float)nrm.z, __uint_as_float(C.slot));
+  if (pick) C.qout.p[j] = make_float4((float)pw.x, (float)pw.y, (float)pw.z, 0.0f);
   C.n_ext++;
 }
 
@@ -443,11 +476,9 @@ __device__ __forceinline__ UniformLight uniform_light(const Params& P, int li) {
 
 __device__ __forceinline__ void put_shadow(ShadowQ& q, uint32_t j, const ShadowRay& s, uint32_t slot, int32_t light) {
   q.light[j] = light;
-  q.ox[j] = s.o2.x; q.oy[j] = s.o2.y; q.oz[j] = s.o2.z;
-  q.dx[j] = s.dir.x; q.dy[j] = s.dir.y; q.dz[j] = s.dir.z;
+  put_ray(q, j, s.o2, s.dir);
   q.tmax[j] = s.tmax;
-  q.cr[j] = s.c[0]; q.cg[j] = s.c[1]; q.cb[j] = s.c[2];
-  q.slot[j] = slot;
+  q.l[j] = make_float4(s.c[0], s.c[1], s.c[2], __uint_as_float(slot));
 }
 
 // Random words of the three light samples of a diffuse vertex (dimensions

@@ -273,10 +273,7 @@ __global__ __launch_bounds__(256) void k_stream_gen(Stream st, RayQ q, int cur) 
       d3 o, d;
       camera_ray(P, (int)(pix % P.W), (int)(pix / P.W), sub % P.SS, sub / P.SS, o, d);
       const uint32_t i = st.prim_base + nt.ray_base + r;
-      q.ox[i] = o.x; q.oy[i] = o.y; q.oz[i] = o.z;
-      q.dx[i] = d.x; q.dy[i] = d.y; q.dz[i] = d.z;
-      q.slot[i] = nt.slot << st.tile_shift;
-      q.meta[i] = 0u;
+      put_ray(q, i, o, d);
     }
     if (lane_id() == 0) rays += nt.n_rays;
   }
@@ -303,8 +300,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PRT_STREAM_
   traverse_pool<false>(
       src, slots, S, ts,
       [&](uint32_t i, d3& o, d3& d, double& tmax) {
-        o = mk(q.ox[i], q.oy[i], q.oz[i]);
-        d = mk(q.dx[i], q.dy[i], q.dz[i]);
+        get_ray(q, i, o, d);
         tmax = PS_INF;
       },
       [&](uint32_t i, double t, int32_t id, bool, d3, d3) {
@@ -361,10 +357,8 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
       valid = lane_id() < dc.cnt;
       if (valid) {
         ray = dc.base + lane_id();
-        slot = qin.slot[ray];
-        T = mk(qin.tr[ray], qin.tg[ray], qin.tb[ray]);
-        Pw = mk(qin.pr[ray], qin.pg[ray], qin.pb[ray]);
-        const uint32_t meta = qin.meta[ray];
+        uint32_t meta;
+        get_segment(qin, ray, T, Pw, meta, slot);
         depth = (int)(meta & 0xFFu);
         branch = META_BRANCH(meta);
         const SlotInfo si = st.slot_info[slot >> shift];
@@ -388,9 +382,10 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
       C.slot = slot;
       const uint32_t e0 = C.n_ext;
       VertexAdj va;
-      const d3 add = shade_vertex(P, P.mats, C, mk(qin.ox[ray], qin.oy[ray], qin.oz[ray]),
-                                  mk(qin.dx[ray], qin.dy[ray], qin.dz[ray]), hit_t[ray], hit_id[ray], T, Pw,
-                                  key_of(P), (uint32_t)pixel, k, depth, branch, va);
+      d3 o, d;
+      get_ray(qin, ray, o, d);
+      const d3 add = shade_vertex(P, P.mats, C, o, d, hit_t[ray], hit_id[ray], T, Pw, key_of(P), (uint32_t)pixel, k,
+                                  depth, branch, va);
       delta = (int)(C.n_ext - e0) - 1;
       accum_add(&st.accum[3 * (size_t)slot + 0], add.x);
       accum_add(&st.accum[3 * (size_t)slot + 1], add.y);
@@ -543,11 +538,8 @@ __global__ __launch_bounds__(256) void k_stream_nee(Stream st, RayQ q, int nxt, 
     d3 x, nrm, ct;
     if (lane_id() < dc.cnt) {
       const uint32_t i = dc.base + lane_id();
-      const uint32_t meta = q.meta[i];
-      slot = q.slot[i];
-      x = mk(q.ox[i], q.oy[i], q.oz[i]);
-      nrm = mk(q.nx[i], q.ny[i], q.nz[i]);
-      ct = mk(q.tr[i], q.tg[i], q.tb[i]);
+      uint32_t meta;
+      get_lit(q, i, x, nrm, ct, meta, slot);
       if (meta & META_NEE) {
         have = true;
         const SlotInfo si = st.slot_info[slot >> shift];
@@ -605,16 +597,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PRT_STREAM_
   traverse_pool<true>(
       src, slots, S, ts,
       [&](uint32_t i, d3& o, d3& d, double& tmax) {
-        o = mk(sq.ox[i], sq.oy[i], sq.oz[i]);
-        d = mk(sq.dx[i], sq.dy[i], sq.dz[i]);
+        get_ray(sq, i, o, d);
         tmax = sq.tmax[i];
       },
       [&](uint32_t i, double, int32_t, bool blocked, d3, d3) {
         if (blocked) return;
-        const uint32_t slot = sq.slot[i];
-        accum_add(&st.accum[3 * (size_t)slot + 0], sq.cr[i]);
-        accum_add(&st.accum[3 * (size_t)slot + 1], sq.cg[i]);
-        accum_add(&st.accum[3 * (size_t)slot + 2], sq.cb[i]);
+        const float4 l = sq.l[i];
+        const uint32_t slot = __float_as_uint(l.w);
+        accum_add(&st.accum[3 * (size_t)slot + 0], l.x);
+        accum_add(&st.accum[3 * (size_t)slot + 1], l.y);
+        accum_add(&st.accum[3 * (size_t)slot + 2], l.z);
       });
   flush_stats(st.ctr, CTR_SNODES, ts);
 }
