@@ -402,7 +402,7 @@ static int scene_build(prt_scene* s, const prt_scene_desc* d) {
   s->n_top = bo.n_top;
   s->bvh_ms = bo.build_ms;
   std::vector<float> tri4((size_t)s->n_tris * 12);
-  std::vector<float> nrm((size_t)s->n_tris * 3), alb(any_albedo ? (size_t)s->n_tris * 3 : 0);
+  std::vector<float> nrm((size_t)s->n_tris * 4), alb(any_albedo ? (size_t)s->n_tris * 3 : 0);
   s->slot_of_tri.assign(s->n_tris, 0);
   for (int64_t slot = 0; slot < s->n_tris; ++slot) {
     const uint32_t t = bo.order[slot];
@@ -415,8 +415,9 @@ static int scene_build(prt_scene* s, const prt_scene_desc* d) {
                            (de.light ? TRI_SHADE_LIGHT : 0u) | (de.has_albedo ? TRI_SHADE_ALBEDO : 0u);
     r[0] = v[0]; r[1] = v[1]; r[2] = v[2]; std::memcpy(&r[3], &ent, 4);
     r[4] = v[3]; r[5] = v[4]; r[6] = v[5]; std::memcpy(&r[7], &face, 4);
-    r[8] = v[6]; r[9] = v[7]; r[10] = v[8]; std::memcpy(&r[11], &shade, 4);
-    for (int k = 0; k < 3; ++k) nrm[3 * slot + k] = t_nrm[3 * (size_t)t + k];
+    r[8] = v[6]; r[9] = v[7]; r[10] = v[8]; r[11] = 0.0f;
+    for (int k = 0; k < 3; ++k) nrm[4 * slot + k] = t_nrm[3 * (size_t)t + k];
+    std::memcpy(&nrm[4 * slot + 3], &shade, 4);
     if (any_albedo)
       for (int k = 0; k < 3; ++k) alb[3 * slot + k] = t_alb[3 * (size_t)t + k];
   }

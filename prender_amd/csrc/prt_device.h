@@ -8,7 +8,9 @@
 //   tris    : float4[3*n_tris], 48 B per triangle in leaf order:
 //             (v0.xyz, entity), (v1.xyz, face), (v2.xyz, unused) — the float32
 //             vertices of the reference's Obj storage (ObjLoader.h:39-75);
-//   tri_nrm : float[3*n_tris] f32 face normal (ObjLoader.cpp:577-700);
+//   tri_nrm : float4[n_tris] (f32 face normal (ObjLoader.cpp:577-700), shade
+//             word): all that shading a hit needs of its triangle, in one
+//             aligned 16-byte load;
 //   tri_alb : float[3*n_tris] per-face albedo or null;
 //   entities, materials, lights: small tables read through the scalar cache.
 #pragma once
@@ -73,8 +75,7 @@ struct DevEntity {
   double u_len, v_len, area;
 };
 
-// Fourth word of a triangle record's third float4: the entity's material
-// index and flags (the first two hold the entity and face indices).
+// A triangle's shade word: its entity's material index and flags.
 #define TRI_SHADE_MAT_MASK 0x00FFFFFFu
 #define TRI_SHADE_NINV 0x01000000u    // normal_vector_inverse < 0
 #define TRI_SHADE_LIGHT 0x02000000u   // material isLight()
@@ -105,7 +106,7 @@ struct Params {
   // scene arrays
   const DevNode* nodes;
   const float* tris;         // read as float4 on the device
-  const float* tri_nrm;
+  const float* tri_nrm;      // read as float4 on the device
   const float* tri_alb;
   const float* tri_alb_rr;   // albedo for Russian-roulette probabilities (null: tri_alb)
   const DevEntity* ents;

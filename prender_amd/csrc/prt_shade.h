@@ -211,22 +211,25 @@ __device__ __forceinline__ d3 shade_vertex(const Params& P, const DevMaterial* m
   const d3 o2 = o + d * 0.000001;
   d3 x, n;
   int ei;
-  // the hit entity's material and flags: a triangle carries them in its
-  // record (TRI_SHADE_*), so its material is read without the entity record
+  // the hit entity's material and flags: a triangle carries them beside its
+  // normal (TRI_SHADE_*), so its material is read without the entity record and
+  // a hit costs one 16-byte gather (the word in the vertex record, 48 bytes a
+  // triangle, was a second line)
   uint32_t mat;
   bool ninv_neg, is_light, has_alb, uvplane;
   if (id >= 0) {
     const float4* tr = reinterpret_cast<const float4*>(P.tris) + (size_t)id * 3;
     ei = __float_as_int(tr[0].w);
     va.face = __float_as_int(tr[1].w);
-    const uint32_t sw = __float_as_uint(tr[2].w);
+    const float4 ns = reinterpret_cast<const float4*>(P.tri_nrm)[id];
+    const uint32_t sw = __float_as_uint(ns.w);
     mat = sw & TRI_SHADE_MAT_MASK;
     ninv_neg = (sw & TRI_SHADE_NINV) != 0;
     is_light = (sw & TRI_SHADE_LIGHT) != 0;
     has_alb = (sw & TRI_SHADE_ALBEDO) != 0;
     uvplane = false;
     x = o2 + d * t;  // polygon.h:170
-    n = mk(P.tri_nrm[3 * (size_t)id], P.tri_nrm[3 * (size_t)id + 1], P.tri_nrm[3 * (size_t)id + 2]);
+    n = mk(ns.x, ns.y, ns.z);
   } else {
     ei = -2 - id;
     const DevEntity& e = P.ents[ei];
