@@ -117,13 +117,13 @@ def main():
     ms_ext, ms_sh, ms_shade = sum_("ms_extend"), sum_("ms_shadow"), sum_("ms_shade")
     launches = sum_("launches_extend")
     # engine 0's choice: scenes without light sampling render in one
-    # persistent launch (k_persist traces every ray of the frame), scenes
+    # persistent launch (k_path traces every ray of the frame), scenes
     # with glass through the streaming tile queue (k_stream_extend /
     # _shadow), the others depth by depth (k_extend / k_shadow)
     persistent = not (desc.sampling.next_event_estimation and sinfo["lights"] > 0)
     streamed = not persistent and any(m.reflection == "reflection" for m in desc.materials)
     if persistent:
-        kx = ks = "k_persist"
+        kx = ks = "k_path"
         kernels = {kx: (sum_("bytes_extend") + sum_("bytes_shadow"), ms_ext, launches)}
     else:
         kx, ks = ("k_stream_extend", "k_stream_shadow") if streamed else ("k_extend", "k_shadow")
@@ -184,7 +184,7 @@ def main():
     tu = out["traversal_union"]
     tu["frac"] = tu["achieved"] / HBM_PEAK_GBS
     if persistent:
-        out["roofline"]["note"] += ("; k_persist also shades and samples lights, so its launch time is the "
+        out["roofline"]["note"] += ("; k_path also shades and samples lights, so its launch time is the "
                                     "whole frame's and its bound is latency rather than HBM")
         out["traversal_union"]["note"] = "one launch traces, shades and resolves every path of the frame"
         out["mrays_per_s_by_class"].update(
@@ -426,14 +426,14 @@ def bench_batch(args, torch, G, prt, info):
             o1 = prt.PrtBatchOpts.from_buffer_copy(topts)
             o1.persistent, o1.persist_waves = 1, opts.persist_waves or 2
             s1 = prt.render_batch_device([scenes[i] for i in rest], [ptrs[i] for i in rest], opts=o1)
-            roof["k_persist"] = (s1["bytes_extend"] + s1["bytes_shadow"], s1["ms_extend"], 1)
+            roof["k_path"] = (s1["bytes_extend"] + s1["bytes_shadow"], s1["ms_extend"], 1)
         if nee:
             o0 = prt.PrtBatchOpts.from_buffer_copy(topts)
             o0.persistent = 0
             s0 = prt.render_batch_device([scenes[i] for i in nee], [ptrs[i] for i in nee], opts=o0)
             roof["k_stream_extend"] = (s0["bytes_extend"], s0["ms_extend"], s0["launches_extend"])
     elif opts.persistent == 1:
-        roof["k_persist"] = (tst["bytes_extend"] + tst["bytes_shadow"], tst["ms_extend"], 1)
+        roof["k_path"] = (tst["bytes_extend"] + tst["bytes_shadow"], tst["ms_extend"], 1)
     else:
         roof["k_stream_extend"] = (tst["bytes_extend"], tst["ms_extend"], tst["launches_extend"])
 
