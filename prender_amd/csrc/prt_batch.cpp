@@ -244,7 +244,7 @@ int ensure_stream_workspace(prt_scene* lead, const BatchConfig& c, const StreamG
   if ((rc = dev_alloc(w.tiles, (size_t)n_tiles * sizeof(TileDesc)))) return rc;
   if ((rc = dev_alloc(w.outs, (size_t)n_scenes * 2 * sizeof(float*)))) return rc;
   if ((rc = dev_alloc(w.runs, 2 * W * (size_t)g.max_runs * sizeof(RunRec)))) return rc;  // shade's, NEE's
-  if ((rc = dev_alloc(w.nruns, 2 * W * sizeof(uint32_t)))) return rc;
+  if ((rc = dev_alloc(w.nruns, 2 * W * sizeof(RunCount)))) return rc;
   for (int p = 0; p < 2; ++p)
     if ((rc = dev_alloc(w.desc[p], (size_t)g.max_desc * sizeof(ChunkDesc)))) return rc;
   if ((rc = dev_alloc(w.sh_desc, (size_t)g.max_sh_desc * sizeof(ChunkDesc)))) return rc;
@@ -334,7 +334,7 @@ int run_stream(prt_scene* const* scenes, int n, const BatchConfig& c, float* con
   S.new_tiles = (NewTile*)w.new_tiles.p;
   S.ray_runs = (RunRec*)w.runs.p;
   S.sh_runs = S.ray_runs + (size_t)PRT_SLAB_WAVES * geo.max_runs;
-  S.ray_nruns = (uint32_t*)w.nruns.p;
+  S.ray_nruns = (RunCount*)w.nruns.p;
   S.sh_nruns = S.ray_nruns + PRT_SLAB_WAVES;
   S.desc[0] = (ChunkDesc*)w.desc[0].p;
   S.desc[1] = (ChunkDesc*)w.desc[1].p;

