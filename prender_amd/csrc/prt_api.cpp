@@ -688,8 +688,13 @@ extern "C++" int prt::ensure_workspace(prt_scene* s, int64_t batch_samples, bool
 // The part of the workspace a frame of the path kernel needs.
 static int ensure_path_workspace(prt_scene* s, int64_t samples) {
   Workspace& w = s->pool->ws;
+  // the queued renders use the same accumulators: a failed allocation has
+  // released them, so they are not recorded until it has succeeded
+  const int64_t recorded = w.batch_samples;
+  w.batch_samples = 0;
   int rc;
   if ((rc = dev_alloc(w.accum, (size_t)samples * 3 * sizeof(uint64_t)))) return rc;
+  w.batch_samples = recorded;
   if ((rc = dev_alloc(w.counts, 16 * sizeof(uint32_t)))) return rc;
   return dev_alloc(w.ctr, CTR_WORDS * sizeof(uint64_t));
 }

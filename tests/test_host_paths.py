@@ -1,0 +1,80 @@
+"""The library's host side without a GPU: workspace sizes after failed allocations
+and the order of launches, with tests/native/host_hip.cpp in the place of the HIP
+runtime.  Kernels do nothing there but what the host reads back."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from prender_amd import prt
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, sys
+sys.modules["torch"] = None  # it would bring the real runtime
+host = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+host.hh_fail_above.argtypes = [C.c_size_t]
+from prender_amd import generators as G, prt
+
+def script(*children):
+    host.hh_script((C.c_uint32 * len(children))(*children), len(children))
+
+def launched():
+    out = C.create_string_buffer(1 << 20)
+    host.hh_launched(out, len(out))
+    return out.value.decode().split()
+
+def no_faults():
+    out = C.create_string_buffer(1 << 16)
+    assert host.hh_faults(out, len(out)) == 0, out.value.decode()
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("needs the HIP headers and compiler")
+    if not os.path.exists(prt.LIB_PATH):
+        pytest.skip("libprt.so is not built (python -m prender_amd.build)")
+    d = tmp_path_factory.mktemp("host_hip")
+    obj, lib = str(d / "host_hip.o"), str(d / "libhost_hip.so")
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "--offload-arch=gfx950", "-O1", "-std=c++17", "-fPIC",
+                    "-I", os.path.join(ROOT, "prender_amd", "csrc"), "-c",
+                    os.path.join(ROOT, "tests", "native", "host_hip.cpp"), "-o", obj], check=True)
+    subprocess.run(["g++", "-shared", "-o", lib, obj], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, lib], cwd=ROOT, stdout=subprocess.PIPE,
+                           stderr=subprocess.STDOUT, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout[-3000:]
+        return r.stdout
+
+    return run
+
+
+# A frame of the path kernel whose accumulators cannot be allocated has released
+# the ones that the queued renders had: the next render allocates its own.
+@pytest.mark.parametrize("after", ["box.render(engine=1)", "box.render(engine=1, samples=2)",
+                                   "box.render_mlt(chains=64, mutations_per_chain=2)"])
+def test_render_after_a_failed_allocation(host, after):
+    host(f"""
+box = prt.Scene(G.config2(width=32, height=24, samples=2, level=2))
+big = prt.Scene(G.cornell_spheres(width=1024, height=1024, samples=1))
+{after}
+host.hh_fail_above(90 << 20)  # the big frame's 96 MiB of accumulators are not to be had
+try:
+    big.render()
+    raise SystemExit("the allocation did not fail")
+except prt.PrtError as e:
+    assert "(-3)" in str(e), e
+{after}
+no_faults()
+host.hh_fail_above(1 << 40)
+big.render()
+{after}
+no_faults()
+""")
