@@ -864,8 +864,9 @@ extern "C++" int prt::run_chains(prt_scene* s, const Params& P, const ChainRun& 
 // ray count once per PRT_DEPTHS_PER_SYNC depths.  Without the adjoint (which
 // reads the partial sums of a sample in path order) a depth's shadow rays are
 // traced on the scene's second stream as PRT_OVERLAP_SHADOW selects; a NEE
-// that rewrites a shadow queue waits for the shadow launch that read it, and
-// the batch's end waits for every shadow launch.
+// that rewrites a shadow queue waits for the shadow launch that read it, a
+// shadow launch on the main stream for the one before it (they share the stack
+// area), and the batch's end for every shadow launch.
 static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t* accum, Adjoint A,
                         BatchForm form, Timer& tm, CallTotals& tot, uint32_t* n_records) {
   Workspace& w = s->pool->ws;
@@ -979,6 +980,8 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
     sh_pending = -1;
     if ((rc = next_fetch(&f))) return rc;  // a fill clearing its counters goes on st first
     hipStream_t on = side ? st_sh : st;
+    // never beside another shadow launch: they share a stack area
+    if (!side && sh_used[b ^ 1]) HIPCHK(hipStreamWaitEvent(on, s->ev_sh[b ^ 1], 0));
     if (side) {
       HIPCHK(hipEventRecord(s->ev_shade, st));
       HIPCHK(hipStreamWaitEvent(on, s->ev_shade, 0));
@@ -1031,7 +1034,8 @@ static int run_batch_on(prt_scene* s, const Params& P, const Batch& B, uint64_t*
       if (n_records) *n_records = w.h_counts[8 + (shades & 1)];
       if (rays == 0) break;
       if (form == FORM_AUTO && rays <= PRT_PATH_TAIL) {
-        // the rest of the batch in one launch
+        // the rest of the batch in one launch, alongside the shadow rays of q[cur]'s NEE
+        if (alt && (rc = shadow_alt(true))) return rc;
         const PathGrid g = path_grid(s->cu_count, 2, rays, true, true);
         if ((rc = ensure_path_pool(w.pool, g, s->has_glass))) return rc;
         if ((rc = run_path(s, PATH_QUEUE, P, B, cur, accum, g))) return rc;

@@ -61,9 +61,9 @@ typedef StackN<PRT_STACK_LDS> Stack;
 
 // Blocks of 256 threads; a thread's overflow area is picked by its global
 // index modulo ovf_threads (the host sizes the area for the largest grid)
-// within one of PRT_OVF_REGIONS regions: closest-hit kernels use region 0,
-// shadow kernels region 1, because the two run at the same time on two
-// streams.
+// within one of PRT_OVF_REGIONS regions: closest-hit and path kernels use region
+// 0, shadow kernels region 1, because the two run at the same time on two
+// streams.  Two launches that use one region must have an order between them.
 #define PRT_DECLARE_STACK_N(S, P, NL, REGION)                                                             \
   __shared__ uint64_t s_stack_[(NL) * 256];                                                               \
   StackN<NL> S{s_stack_ + threadIdx.x,                                                                    \

@@ -78,3 +78,39 @@ big.render()
 {after}
 no_faults()
 """)
+
+
+# Two launches of any-hit rays share one stack area, so one must end before the
+# other begins: also where the path kernel takes a batch's last rays while the
+# shadow rays of the depth before are on the second stream.  script: rays that the
+# shading of each depth leaves; the host looks at the first and every fourth.
+@pytest.mark.parametrize("children,tail", [((200000, 200000, 200000, 200000, 1000), True), ((60000,), True),
+                                           ((200000, 200000, 100, 0), False), ((0,), False)])
+def test_shadow_launches_are_ordered(host, children, tail):
+    host(f"""
+box = prt.Scene(G.config2(width=400, height=400, samples=1, level=2))
+script{tuple(children)!r}
+_, _, st = box.render(variance=False)
+assert any("k_pathILi2E" in k for k in launched()) == {tail}
+assert st["extension_rays"] == {sum(children)} and st["shadow_rays"] == {3 * sum(children)}, st
+no_faults()
+""")
+
+
+# the same over an adjoint's recording pass and its replay, and a batch
+def test_other_overlapping_launches_are_ordered(host):
+    host("""
+d = G.config5(width=64, height=48, samples=2)
+s = prt.Scene(d)
+dimg, grad = C.c_void_p(), C.c_void_p()
+host.hipMalloc(C.byref(dimg), C.c_size_t(64 * 48 * 12))
+host.hipMalloc(C.byref(grad), C.c_size_t(d.entities[1].indices.shape[0] * 12))
+script(*[3000] * 6)
+s.adjoint_device(dimg.value, 1, grad.value, 2)
+out = C.c_void_p()
+host.hipMalloc(C.byref(out), C.c_size_t(64 * 48 * 12))
+prt.render_batch_device([s], [out.value], None, prt.batch_opts())
+names = launched()
+assert sum("k_shadow" in k for k in names) >= 6 and any("k_stream_shadow" in k for k in names)
+no_faults()
+""")
