@@ -540,6 +540,19 @@ extern "C++" void prt::fill_stats(prt_stats* st, const uint64_t* c) {
   st->truncated_paths += c[CTR_TRUNC];
 }
 
+extern "C++" int prt::check_traced(const uint64_t* c, uint64_t primary_rays) {
+  if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
+  if (c[CTR_QUEUED] != primary_rays + c[CTR_EXT])
+    return fail(PRT_E_INTERNAL, std::to_string(c[CTR_QUEUED]) + " rays came from " + std::to_string(primary_rays) +
+                                    " camera rays and " + std::to_string(c[CTR_EXT]) + " children");
+  if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
+    return fail(PRT_E_INTERNAL, "traversal finished " + std::to_string(c[CTR_TRACED]) + " of " +
+                                    std::to_string(c[CTR_QUEUED]) + " rays and " +
+                                    std::to_string(c[CTR_STRACED]) + " of " + std::to_string(c[CTR_SHADOW]) +
+                                    " shadow rays");
+  return PRT_OK;
+}
+
 static int trace_device(prt_scene* s, const prt_ray* d_rays, int64_t n, prt_hit* d_hits, prt_stats* stats) {
   HIPCHK(hipSetDevice(s->device));
   std::lock_guard<std::recursive_mutex> pool_lock(s->pool->m);
@@ -1087,13 +1100,7 @@ static int finish_stats(prt_scene* s, const RenderSetup& R, Timer& tm, const Cal
   HIPCHK(hipMemcpyAsync(raw, s->pool->ws.ctr.p, sizeof(raw), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   sum_counters(raw, c);
-  if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
-  // every queued ray must have been traced exactly once
-  if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
-    return fail(PRT_E_INTERNAL, "traversal finished " + std::to_string(c[CTR_TRACED]) + " of " +
-                                    std::to_string(c[CTR_QUEUED]) + " rays and " +
-                                    std::to_string(c[CTR_STRACED]) + " of " + std::to_string(c[CTR_SHADOW]) +
-                                    " shadow rays");
+  if (const int rc = check_traced(c, tot.primary_rays)) return rc;
   double cat[T_NCAT] = {0, 0, 0, 0, 0, 0};
   double trav = 0.0;
   const double wall = tm.collect(cat, &trav, 1u << T_EXTEND | 1u << T_EXTEND0 | 1u << T_SHADOW);

@@ -255,6 +255,9 @@ struct CallTotals {
 
 // Adds the traversal / shading counters c[CTR_*] to *st.
 void fill_stats(prt_stats* st, const uint64_t* c);
+// An error unless every camera ray and every child of a vertex was queued and
+// traced exactly once, and every shadow ray traced.
+int check_traced(const uint64_t* c, uint64_t primary_rays);
 // Sizes the scene's workspace for batches of `batch_samples` camera samples.
 int ensure_workspace(prt_scene* s, int64_t batch_samples, bool two_accum);
 // Grid and claim sizes of a path-kernel launch over n samples (rays) cut into

@@ -169,10 +169,7 @@ static int render_mlt(prt_scene* s, const prt_mlt_opts* o, void* d_out, int as_f
   HIPCHK(hipStreamSynchronize(st));
   sum_counters(raw, c);
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
-  if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
-    return fail(PRT_E_INTERNAL, "traversal finished " + std::to_string(c[CTR_TRACED]) + " of " +
-                                    std::to_string(c[CTR_QUEUED]) + " rays");
+  if ((rc = check_traced(c, tot.primary_rays))) return rc;
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     fill_stats(stats, c);
@@ -336,10 +333,7 @@ static int render_erpt(prt_scene* s, const prt_erpt_opts* o, void* d_out, int as
   HIPCHK(hipStreamSynchronize(st));
   sum_counters(raw, c);
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  if (c[CTR_DROP] != 0) return fail(PRT_E_INVALID, "ray queue overflow (" + std::to_string(c[CTR_DROP]) + " rays)");
-  if (c[CTR_TRACED] != c[CTR_QUEUED] || c[CTR_STRACED] != c[CTR_SHADOW])
-    return fail(PRT_E_INTERNAL, "traversal finished " + std::to_string(c[CTR_TRACED]) + " of " +
-                                    std::to_string(c[CTR_QUEUED]) + " rays");
+  if ((rc = check_traced(c, tot.primary_rays))) return rc;
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     fill_stats(stats, c);

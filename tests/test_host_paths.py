@@ -114,3 +114,25 @@ names = launched()
 assert sum("k_shadow" in k for k in names) >= 6 and any("k_stream_shadow" in k for k in names)
 no_faults()
 """)
+
+
+# A render whose path kernel loses a sample fails its own check, as the batched
+# form's does.
+@pytest.mark.parametrize("call", ["box.render()", "spheres.render()", "box.render_mlt(chains=64, mutations_per_chain=3)",
+                                  "box.render_erpt(mutation=2.0)",
+                                  "prt.render_batch_device([spheres], [out.value], None, prt.batch_opts(persistent=1))"])
+def test_a_lost_sample_is_an_error(host, call):
+    host(f"""
+box = prt.Scene(G.config2(width=32, height=24, samples=2, level=2))
+spheres = prt.Scene(G.cornell_spheres(width=32, height=24, samples=2))
+out = C.c_void_p()
+host.hipMalloc(C.byref(out), C.c_size_t(32 * 24 * 12))
+{call}
+host.hh_lose(1)
+try:
+    {call}
+    raise SystemExit("the lost sample went unnoticed")
+except prt.PrtError as e:
+    assert "(-6)" in str(e), e
+no_faults()
+""")
