@@ -784,7 +784,13 @@ extern "C++" PathGrid prt::path_grid(int cu_count, int waves, uint64_t n, bool n
     g.unit = g.quota = (uint32_t)std::max<uint64_t>(1, per_wave);
     g.blocks = (int)std::max<uint64_t>(1, ((n + g.unit - 1) / g.unit + 3) / 4);
   }
-  if (per_wave >= 64 * 16) g.claim = 4;  // 256 samples per claim atomic
+  // 256 samples per claim atomic once that leaves every wave 64 claims to even
+  // out what samples cost.  From 4 claims a wave on, as it was, a field of 2.1 M
+  // triangles, 8 spp, light sampling took at 2^21, 2^22, 2^23, 2^24 samples 10.6,
+  // 14.6, 25.0, 44.5 ms against 7.0, 11.9, 22.1, 42.2 ms with one chunk per claim,
+  // the spheres 4.41, 8.94, 17.1, 33.6 against 4.41, 8.52, 16.7, 33.2; at 2^26
+  // samples without light sampling 62.3 and 64.1 ms, 41.2 and 41.0.
+  if (per_wave >= 64 * 256) g.claim = 4;
   return g;
 }
 

@@ -54,6 +54,8 @@ std::vector<Use> g_uses;
 std::vector<uint32_t> g_script;  // children of the coming shade launches
 size_t g_next = 0, g_limit = ~(size_t)0;
 uint32_t g_lost = 0;
+Persist g_path;  // of the last path kernel
+uint32_t g_path_waves = 0;
 float g_ms = 1000.0f;
 
 HostStream* stream_of(hipStream_t s) { return reinterpret_cast<HostStream*>(s); }
@@ -141,6 +143,7 @@ void emulate(const std::string& n, void** a, hipStream_t s) {
     arg<uint64_t*>(a, 6)[CTR_SHADOW] += out;
   } else if (is("k_path")) {
     const Persist& p = arg<Persist>(a, 0);
+    g_path = p;
     const bool batch = is("k_pathILi0E"), queue = is("k_pathILi2E"), chain = is("k_pathILi3E");
     traverses(n, s, region(batch ? p.scenes[0] : arg<Params>(a, 1), 0));
     if (queue) {
@@ -173,6 +176,12 @@ void hh_script(const uint32_t* children, int n) {
   g_next = 0;
 }
 void hh_lose(uint32_t samples) { g_lost = samples; }
+// chunks, chunks per claim and waves of the last path kernel
+void hh_path(uint32_t* out) {
+  out[0] = g_path.n_chunks;
+  out[1] = g_path.claim;
+  out[2] = g_path_waves;
+}
 int hh_faults(char* out, int size) {
   std::string all;
   for (auto& f : g_faults) all += f + "\n";
@@ -207,9 +216,10 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hi
   *s = g_call.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t s) {
   step(s);
   const std::string& name = g_names[f];
+  if (name.find("k_path") != std::string::npos) g_path_waves = grid.x * 4u;
   g_launched.push_back(name);
   emulate(name, args, s);
   return hipSuccess;

@@ -136,3 +136,21 @@ except prt.PrtError as e:
     assert "(-6)" in str(e), e
 no_faults()
 """)
+
+
+# What a sample costs differs over an image, so every wave of a path launch has
+# many claims to take, or claims single chunks.
+@pytest.mark.parametrize("nee", [0, 1])
+def test_path_claims_leave_work_to_share(host, nee):
+    host(f"""
+for height in (1023, 1024, 1025, 2048, 4096):
+    s = prt.Scene(G.cornell_spheres(width=1024, height=height, samples=2, supersamples=1, nee={nee}))
+    s.render(engine=3, variance=False)
+    got = (C.c_uint32 * 3)()
+    host.hh_path(got)
+    chunks, claim, waves = got
+    assert chunks >= 1024 * height * 2 // 64 and waves >= 2048
+    assert claim == 1 or chunks >= 64 * claim * waves, (height, chunks, claim, waves)
+    s.close()
+no_faults()
+""")
