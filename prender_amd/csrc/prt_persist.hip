@@ -478,9 +478,12 @@ __global__ __launch_bounds__(256) void k_persist_resolve(Persist st, int64_t n_p
 
 // ------------------------------------------------------------ launchers
 // Two register budgets, neither of which spills vector registers: 2 waves per
-// SIMD, and without light sampling 3 (166 VGPRs), for launches that fill them
+// SIMD, and without light sampling 3 (168 VGPRs), for launches that fill them
 // (spheres 320x240 x 16 spp 1033 -> 951 us).  A smaller launch gains nothing
-// from more waves and loses the LDS.
+// from more waves and loses the LDS.  An instance for 4 waves with light sampling
+// (128 VGPRs, 151 spilled to scratch memory) gave wrong sums for a reason not
+// found, so the build refuses an instance that spills vector registers
+// (build.py, check_spills).
 // LDS of the instances: at 2 waves (two blocks per CU) 12 stack entries and
 // five BVH levels, so that the tree's top costs an LDS access instead of an L2
 // one, or for a batch of scenes, which shares no tree, 32 entries; at 3 waves 14
