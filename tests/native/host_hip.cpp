@@ -136,6 +136,11 @@ void emulate(const std::string& n, void** a, hipStream_t s) {
     const uint32_t out = g_next < g_script.size() ? g_script[g_next++] : 0u;
     for (int i = 0; i < PRT_SLAB_WAVES; ++i) slabs[i] = make_uint2(0u, i ? 0u : out);
     arg<uint64_t*>(a, 12)[CTR_EXT] += out;
+    if (is("k_shadeILi2E")) {  // a recording pass: 64 entries per input chunk
+      const int64_t samples = arg<Batch>(a, 1).n_pixels * arg<Params>(a, 0).spp;
+      const AdjointRecs& r = arg<Adjoint>(a, 11).recs;
+      *r.next = *r.first + 64u * (arg<int>(a, 2) ? (uint32_t)((samples + 63) / 64) : *arg<ChunkList>(a, 4).n);
+    }
   } else if (is("k_nee")) {
     uint2* slabs = arg<uint2*>(a, 5);
     const uint32_t out = 3u * entries(arg<ChunkList>(a, 3));

@@ -154,3 +154,28 @@ for height in (1023, 1024, 1025, 2048, 4096):
     s.close()
 no_faults()
 """)
+
+
+# Records that cannot be allocated: the batch is replayed, its samples' radiance
+# being known; nothing else of the call depends on them.
+@pytest.mark.parametrize("limit,replayed", [(1 << 40, False), (3 << 20, True)])
+def test_adjoint_without_memory_for_records(host, limit, replayed):
+    host(f"""
+d = G.config5(width=64, height=48, samples=8)
+s = prt.Scene(d)
+dimg, grad = C.c_void_p(), C.c_void_p()
+host.hipMalloc(C.byref(dimg), C.c_size_t(64 * 48 * 12))
+host.hipMalloc(C.byref(grad), C.c_size_t(d.entities[1].indices.shape[0] * 12))
+script(*[2000] * 4)
+s.adjoint_device(dimg.value, 1, None, 2)
+host.hh_fail_above({limit})
+launched()
+script(*[2000] * 4, 0, *[2000] * 4)
+_, st = s.adjoint_device(dimg.value, 1, grad.value, 2)
+names = launched()
+assert any("k_shadeILi2E" in k for k in names)
+assert any("k_shadeILi1E" in k for k in names) == {replayed}
+assert any("k_adjoint_resolve" in k for k in names) != {replayed}
+assert st["primary_rays"] == 64 * 48 * 4 * {2 if replayed else 1}
+no_faults()
+""")
