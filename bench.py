@@ -424,7 +424,7 @@ def bench_batch(args, torch, G, prt, info):
         rest = [i for i in range(len(scenes)) if i not in nee]
         if rest:
             o1 = prt.PrtBatchOpts.from_buffer_copy(topts)
-            o1.persistent, o1.persist_waves = 1, opts.persist_waves or 2
+            o1.persistent, o1.trav_blocks_per_cu = 1, 0  # the same instance: persist_waves or the automatic one
             s1 = prt.render_batch_device([scenes[i] for i in rest], [ptrs[i] for i in rest], opts=o1)
             roof["k_path"] = (s1["bytes_extend"] + s1["bytes_shadow"], s1["ms_extend"], 1)
         if nee:
@@ -455,12 +455,14 @@ def bench_batch(args, torch, G, prt, info):
     pers = seq_s = max_diff = seq_diff = None
     if not args.no_trials:
         # the persistent engine: one launch over every sample of the batch; one
-        # trial per register budget (2, 3 or 4 waves per SIMD), the fastest timed
+        # trial per instance (2 waves per SIMD, without light sampling also 3), the
+        # fastest timed
         progress("persistent engine")
         pers = {}
         trials = {}
-        for wv in (2, 3, 4):
-            po = prt.batch_opts(seed=args.seed + args.steps - 1, persistent=True, trav_blocks_per_cu=wv)
+        lit = any(s.desc.sampling.next_event_estimation and s.info()["lights"] > 0 for s in scenes)
+        for wv in (2,) if lit else (2, 3):
+            po = prt.batch_opts(seed=args.seed + args.steps - 1, persistent=True, persist_waves=wv)
             trials[wv] = prt.render_batch_device(scenes, ptrs, opts=po)["ms_total"]
         best_w = min(trials, key=trials.get)
         torch.cuda.synchronize()
@@ -468,7 +470,7 @@ def bench_batch(args, torch, G, prt, info):
         pers_same = not pers_diff
         t0 = time.perf_counter()
         for i in range(args.steps):
-            po = prt.batch_opts(seed=args.seed + i, persistent=True, trav_blocks_per_cu=best_w)
+            po = prt.batch_opts(seed=args.seed + i, persistent=True, persist_waves=best_w)
             pst = prt.render_batch_device(scenes, ptrs, opts=po)
         torch.cuda.synchronize()
         pers_s = (time.perf_counter() - t0) / args.steps

@@ -367,17 +367,18 @@ typedef struct prt_batch_opts {
                                    waves claim 64-sample chunks from one shared counter and follow each
                                    sample's whole path (shading, NEE, shadow rays, glass branches) with
                                    no ray queues and no waits between waves; then one launch folds the
-                                   pixels.  trav_blocks_per_cu (2..4) sets its waves per SIMD;
-                                   tile_samples, inflight_tiles, use_graph and tile_stride do not
-                                   apply; at most 2^28 camera samples (a fixed-point accumulator each).
+                                   pixels.  tile_samples, inflight_tiles, stack_lds, use_graph and
+                                   tile_stride do not apply; at most 2^28 camera samples (a
+                                   fixed-point accumulator each).
                                    2 = split: the scenes without next-event estimation in one
                                    persistent launch, the others through the tile queue (with these
                                    options), one after the other.
                                    The images are the same bit for bit in every mode. */
-    int32_t persist_waves;      /* waves per SIMD the persistent kernel's registers are budgeted for
-                                   (2..4) in modes 1 and 2; 0 = mode 1: trav_blocks_per_cu if given, else 3
-                                   for batches that fill them (2 below that).  Launches with light sampling
-                                   run at 2, others at most at 3 */
+    int32_t persist_waves;      /* waves per SIMD of the persistent kernel in modes 1 and 2 (2..4 are
+                                   taken).  There are two instances: 2, which launches with light
+                                   sampling run whatever is asked, and 3 without, which 4 means too.
+                                   0 = mode 1: trav_blocks_per_cu if given (2 for less, 3 for more);
+                                   else 3 for launches that fill them, 2 for smaller ones */
 } prt_batch_opts;
 /* d_rgb[i] / d_var[i]: W_i*H_i*3 float device buffers of scene i (d_var or
  * its entries may be NULL).  All scenes must live on one device; the call
@@ -389,7 +390,8 @@ int prt_render_batch_device(prt_scene* const* scenes, int n_scenes,
  * traversal grids and the launch form (plain or graph replay) by coordinate
  * descent on a subsample of the batch's tiles (every k-th tile, k from
  * base->tile_stride or chosen for ~16M samples per trial), then the
- * persistent engine and the split form, each at 2, 3 and 4 waves per SIMD, on
+ * persistent engine and, where some scenes sample lights and some do not, the
+ * split form, once per instance of the persistent kernel (persist_waves), on
  * the whole batch (when it fits and base->tile_stride asks for no
  * subsample), and writes the fastest
  * options to *best (tile_stride copied from base; inflight_tiles from base,

@@ -774,7 +774,7 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 extern "C++" PathGrid prt::path_grid(int cu_count, int waves, uint64_t n, bool nee, bool whole_chunks) {
   PathGrid g;
   if (waves == 0) waves = n >= (uint64_t)std::max(1, cu_count) * 2 * 256 ? 3 : 2;
-  waves = nee ? 2 : std::min(3, std::max(2, waves));  // the instances there are
+  waves = path_waves(waves, nee);
   g.waves = waves;
   g.blocks = std::max(1, cu_count) * waves;  // one 256-thread block per CU puts one wave on each SIMD
   const uint64_t per_wave = (n + g.n_waves() - 1) / g.n_waves();

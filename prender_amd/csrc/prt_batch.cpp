@@ -823,7 +823,8 @@ int prt_render_batch_device(prt_scene* const* scenes, int n_scenes, const prt_ba
 // launch form (the samples in flight stay the caller's or the automatic
 // size), each trial rendering every k-th tile so that a trial costs about
 // 1/k of the whole batch; ranked by device time per camera sample.  Then
-// the persistent and split forms on the whole batch.
+// the persistent and split forms on the whole batch, once per instance of the
+// path kernel.
 int prt_tune_batch(prt_scene* const* scenes, int n_scenes, const prt_batch_opts* base, float* const* d_rgb,
                    float* const* d_var, prt_batch_opts* best, double* best_ns_per_sample) {
   int rc;
@@ -894,33 +895,27 @@ int prt_tune_batch(prt_scene* const* scenes, int n_scenes, const prt_batch_opts*
   }
   cur.inflight_tiles = inflight > 0 ? (int32_t)std::max<int64_t>(1, inflight / cur.tile_samples) : 0;
   cur.tile_stride = base ? base->tile_stride : 0;
-  // the persistent engine (every sample, one launch) at each register
-  // budget, when the batch fits it and no subsample was asked for
+  // the persistent engine (every sample, one launch), when the batch fits it and
+  // no subsample was asked for, at each register budget that it has an instance
+  // for; then the split, whose persistent half has no light sampling
   if (total <= kMaxPersistSamples && (!base || base->tile_stride <= 1)) {
     const prt_batch_opts queued = cur;
-    for (int wv = 2; wv <= 4; ++wv) {
-      prt_batch_opts o = queued;
-      o.persistent = 1;
-      o.trav_blocks_per_cu = wv;
-      BatchConfig c;
-      if ((rc = resolve_config(scenes, n_scenes, &o, c))) return rc;
-      BatchResult res;
-      if ((rc = run_persistent(scenes, n_scenes, c, d_rgb, d_var, nullptr, &res))) return rc;
-      const double ns = res.samples ? res.ms * 1e6 / (double)res.samples : 1e30;
-      if (ns < best_ns) { best_ns = ns; cur = o; }
-    }
-    // split: scenes without NEE persistent (at each register budget), the
-    // others through the tuned tile queue
-    for (int wv = 2; wv <= 4; ++wv) {
-      prt_batch_opts o = queued;
-      o.persistent = 2;
-      o.persist_waves = wv;
-      BatchConfig c;
-      if ((rc = resolve_config(scenes, n_scenes, &o, c))) return rc;
-      BatchResult res;
-      if ((rc = run_split(scenes, n_scenes, c, d_rgb, d_var, nullptr, &res))) return rc;
-      const double ns = res.samples ? res.ms * 1e6 / (double)res.samples : 1e30;
-      if (ns < best_ns) { best_ns = ns; cur = o; }
+    int n_nee = 0;
+    for (int i = 0; i < n_scenes; ++i) n_nee += scenes[i]->P.nee && scenes[i]->P.n_lights > 0;
+    for (int form = 1; form <= 2; ++form) {
+      if (form == 2 && (n_nee == 0 || n_nee == n_scenes)) continue;  // one of the other forms
+      for (int wv = 2; wv <= 3; ++wv) {
+        if (path_waves(wv, form == 1 && n_nee > 0) != wv) continue;
+        prt_batch_opts o = queued;
+        o.persistent = form;
+        o.persist_waves = wv;
+        BatchConfig c;
+        if ((rc = resolve_config(scenes, n_scenes, &o, c))) return rc;
+        BatchResult res;
+        if ((rc = (form == 1 ? run_persistent : run_split)(scenes, n_scenes, c, d_rgb, d_var, nullptr, &res))) return rc;
+        const double ns = res.samples ? res.ms * 1e6 / (double)res.samples : 1e30;
+        if (ns < best_ns) { best_ns = ns; cur = o; }
+      }
     }
   }
   *best = cur;

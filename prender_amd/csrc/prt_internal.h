@@ -267,6 +267,9 @@ struct PathGrid {
   uint32_t unit = 64, claim = 1, quota = 64;
   uint32_t n_waves() const { return (uint32_t)blocks * 4u; }
 };
+// Waves per SIMD of the instance that runs when `waves` are asked for: two with
+// light sampling, else two or three.
+inline int path_waves(int waves, bool nee) { return nee ? 2 : std::min(3, std::max(2, waves)); }
 PathGrid path_grid(int cu_count, int waves, uint64_t n, bool nee, bool whole_chunks);
 int ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass);
 // How run_batch may trace a batch: wavefront only, the path kernel where the

@@ -179,3 +179,27 @@ assert any("k_adjoint_resolve" in k for k in names) != {replayed}
 assert st["primary_rays"] == 64 * 48 * 4 * {2 if replayed else 1}
 no_faults()
 """)
+
+
+# The tuner times each form once per instance of the path kernel that there is
+# (light sampling: two waves per SIMD; without: two and three), and reports one of
+# them.  Every measured span here is shorter than the last, so the last trial wins.
+@pytest.mark.parametrize("nees,instances,form,waves", [((0, 1), 3, 2, 3), ((1, 1), 1, 1, 2), ((0, 0), 2, 1, 3)])
+def test_tuner_times_each_instance_once(host, nees, instances, form, waves):
+    host(f"""
+scenes = [prt.Scene(G.cornell_spheres(width=32 + 8 * i, height=24, samples=2, nee=n)) for i, n in enumerate({nees!r})]
+outs = []
+for s in scenes:
+    p = C.c_void_p()
+    host.hipMalloc(C.byref(p), C.c_size_t(s.width * s.height * 12))
+    outs.append(p.value)
+best, _ = prt.tune_batch(scenes, outs)
+tried = [k for k in launched() if "k_pathILi0E" in k]
+assert len(tried) == len(set(tried)) == {instances}, tried
+assert best.persistent == {form}
+assert (best.persist_waves or best.trav_blocks_per_cu) == {waves}, (best.persist_waves, best.trav_blocks_per_cu)
+prt.render_batch_device(scenes, outs, None, best)
+ran = [k for k in launched() if "k_pathILi0E" in k]
+assert len(ran) == 1 and ran[0] == tried[-1] and ran[0].endswith("Li{waves}EEv7Persist6Params"), ran
+no_faults()
+""")
