@@ -158,7 +158,8 @@ typedef struct prt_hit {
 /* Counters of one render / trace call. */
 typedef struct prt_stats {
     uint64_t camera_samples;   /* W*H*spp */
-    uint64_t primary_rays;     /* camera rays traversed (unique sub-pixel rays) */
+    uint64_t primary_rays;     /* camera rays traversed: one per sub-pixel in the queued engines, one per
+                                  camera sample in the one launch that follows whole paths */
     uint64_t extension_rays;   /* bounce rays traversed */
     uint64_t shadow_rays;      /* NEE shadow rays traversed */
     uint64_t pickup_hits;      /* specular-pickup contributions (no extra ray) */
@@ -167,7 +168,7 @@ typedef struct prt_stats {
     uint64_t truncated_paths;  /* paths stopped by the safety depth cap */
     uint64_t bytes_algorithmic;/* 128*nodes + 48*tris + 48*rays */
     double ms_total;           /* device time of the whole call */
-    double ms_extend;          /* closest-hit kernels */
+    double ms_extend;          /* closest-hit kernels; the one launch counts here with all it does */
     double ms_shade;           /* shading kernels */
     double ms_shadow;          /* shadow kernels */
     double ms_other;           /* generate / resolve / clears */

@@ -22,8 +22,6 @@ LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libprt.so")
 SOURCES = ["prt_kernels.hip", "prt_stream.hip", "prt_persist.hip", "prt_mlt.hip", "prt_api.cpp", "prt_batch.cpp", "prt_mlt.cpp", "bvh.cpp",
            "scene_file.cpp", "image_io.cpp"]
-HEADERS = ["prt_device.h", "prt_kernels.h", "prt_math.h", "prt_trace.h", "prt_shade.h", "prt_stream.h",
-           "prt_internal.h", "prt_mlt.h", "bvh.h"]
 ARCH = "gfx950"
 REMARK = "[-Rpass-analysis=kernel-resource-usage]"
 

@@ -756,11 +756,15 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 // batch's tail (rays).  A depth-synchronous depth or a tile-queue iteration
 // costs two traversal launches however few its rays; the path kernel pays no
 // launch per depth, but its waves wait for their slowest ray in every trip.
-// Measured (path kernel / queued engine, ms): mesh box, 0.13 M samples 0.90 /
-// 1.96, 0.15 M 0.93 / 2.04, 0.6 M 3.2 / 2.8, 1.05 M 5.1 / 3.7; with glass, where the
-// tile queue drains through long tails, spheres 2.1 M 4.0 / 6.3, spheres and 60k
-// triangles 2.6 M 8.8 / 11.5, 4.2 M 14.5 / 14.4, field of 200k triangles 1.6 M 3.1
-// / 3.4, of 400k 2.5 M 4.7 / 4.5.
+// Measured (path kernel / the queued engine of such scenes, ms):
+//   box, 104 triangles: 0.26 M samples 1.26 / 1.47, 0.39 M 1.73 / 1.68, 0.52 M 2.25 /
+//   1.92; 82k: 2.12 / 2.51, 2.85 / 2.87, 3.54 / 3.21; 1.3 M: 2.88 / 3.48, 3.87 / 4.11,
+//   4.62 / 4.62;
+//   with glass, where the tile queue drains through long tails, spheres 2.1 M samples
+//   4.41 / 6.27, 2.6 M 5.45 / 8.47; and 60k triangles 1.6 M 6.27 / 6.43, 2.1 M 8.21 /
+//   7.88, 2.6 M 10.2 / 10.8; field of 103k triangles 2.1 M 2.10 / 2.77, of 564k 1.0 M
+//   3.53 / 3.88, 1.6 M 4.33 / 4.26, 2.1 M 5.13 / 4.72, of 2.1 M 1.0 M 4.37 / 4.57, 1.6 M
+//   5.87 / 5.09, 2.1 M 6.93 / 5.61: for the largest meshes the line lies too high.
 #ifndef PRT_PATH_SAMPLES
 #define PRT_PATH_SAMPLES (3 << 17)
 #endif
@@ -880,9 +884,10 @@ extern "C++" int prt::run_chains(prt_scene* s, const Params& P, const ChainRun& 
 // into `accum` (fixed point, 3 per camera sample of the batch).  Each
 // slab-writing kernel is followed by k_slab_index, which lists the chunks
 // of the queue it wrote for the kernels that read it.  The host reads the
-// ray count once per PRT_DEPTHS_PER_SYNC depths.  Without the adjoint (which
-// reads the partial sums of a sample in path order) a depth's shadow rays are
-// traced on the scene's second stream as PRT_OVERLAP_SHADOW selects; a NEE
+// ray count once per PRT_DEPTHS_PER_SYNC depths.  A depth's shadow rays are
+// traced on the scene's second stream as PRT_OVERLAP_SHADOW selects (an
+// adjoint's replay, which reads the partial sums of a sample in path order, keeps
+// one stream; its recording pass waits for them before the next shade); a NEE
 // that rewrites a shadow queue waits for the shadow launch that read it, a
 // shadow launch on the main stream for the one before it (they share the stack
 // area), and the batch's end for every shadow launch.
@@ -1193,10 +1198,14 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
   if (dumping && (engine == 2 || engine == 3))
     return fail(PRT_E_INVALID, "progress images need the depth-synchronous engine");
   if (engine < 0 || engine > 3) return fail(PRT_E_INVALID, "engine must be 0..3");
-  // Scenes without next-event estimation render fastest in one persistent
-  // launch that follows each sample's whole path (cfg1: 1.64 against 2.71 ms
-  // per frame); with NEE its lanes trace their shadow rays one after another
-  // and the queued engines win.
+  // Scenes without next-event estimation take the path kernel at any size, others
+  // up to path_samples.  Measured without it (path kernel / the faster of the
+  // queued engines, ms, 16 spp): spheres 0.26 M samples 0.39 / 0.78, 16.8 M 10.4 / 12.7;
+  // and 60k triangles 1.0 M 1.68 / 2.57, 4.2 M 5.55 / 5.62, 16.8 M 21.2 / 18.8; box of 82k
+  // triangles 1.0 M 2.25 / 2.72, 4.2 M 7.56 / 5.88, 16.8 M 28.8 / 18.0, of 1.3 M 2.97 / 4.04,
+  // 10.2 / 7.59, 38.9 / 21.1; field of 2.1 M triangles 0.26 M 1.98 / 2.08, 16.8 M 17.1 /
+  // 14.5.  From some 3 M samples on, then, meshes are faster depth-synchronous
+  // (engine 1) at the price of its queues, 700 bytes a sample against 24.
   const bool nee_scene = s->P.nee && s->P.n_lights > 0;
   const bool persist_ok = stream_ok && (uint64_t)s->P.W * s->P.H * s->P.spp <= ((uint64_t)1 << 28);
   if (engine == 3 && !persist_ok)
@@ -1369,10 +1378,15 @@ int prt_set_emission(prt_scene* s, int entity, const double emission[3]) {
 
 // Adjoint, per batch: one pass renders the samples and records every vertex on
 // the differentiated entity with its sample's radiance up to it; then each
-// record's gradient is what the sample got after it.  A batch with more vertices
-// than records (PRT_ADJOINT_RECORDS per sample on average, or none where the
-// memory for them is not to be had) is replayed instead: the same paths again,
-// each vertex's gradient from the radiance that the first pass found.
+// record's gradient is what the sample got after it.  Records are slots, 64 per
+// chunk that a shade launch reads, also for lanes without a ray and vertices on
+// other entities.  A batch that needs more than PRT_ADJOINT_RECORDS per sample and
+// 64 * 64 (long paths, above all in batches below 2^19 samples: a slab writer has
+// one chunk there, which counts in full until its last ray has ended), or for
+// which the memory is not to be had, is replayed instead: the same paths again,
+// each vertex's gradient from the radiance that the first pass found.  A record
+// takes 32 bytes, up to 8.6 GB for a batch of 2^24 samples, kept in the device's
+// pool.
 // Measured with the forward render, box with 82k triangles: 256x256 x 32 spp 23.9
 // ms replayed, 16.5 ms recorded; 64x48 x 16 spp 4.9 and 3.3 ms.  With 2 records per
 // sample, so that every batch is replayed after all, 24.1 ms.

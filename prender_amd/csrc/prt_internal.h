@@ -64,7 +64,7 @@ int dev_upload(DevBuf& b, const std::vector<T>& v, hipStream_t s) {
   return PRT_OK;
 }
 
-// Ray / shadow queues as 17 / 12 separately allocated SoA columns.
+// Ray and shadow queues as separately allocated rows (RayQ, ShadowQ).
 enum { RAYQ_COLS = 6, SHADOWQ_COLS = 6 };
 int alloc_ray_queue(DevBuf* cols, int64_t cap);
 size_t ray_entry_bytes();     // device bytes per ray-queue entry
@@ -80,7 +80,7 @@ struct Workspace {
   int64_t batch_samples = 0;  // camera samples per batch
   int64_t queue_cap = 0;      // entries allocated per ray queue
   int64_t shadow_cap = 0;     // entries allocated in the shadow queue
-  DevBuf q[2][RAYQ_COLS];     // two ray queues (SoA)
+  DevBuf q[2][RAYQ_COLS];     // two ray queues
   DevBuf hit_t, hit_id;
   DevBuf sq[SHADOWQ_COLS];
   DevBuf sq2[SHADOWQ_COLS];   // second shadow queue (NEE scenes, when a depth's shadow rays are traced

@@ -26,7 +26,7 @@
 // chains in the vertices and 2,700 in 64 light samples.  So rays of one vertex
 // run side by side, few samples are spread over all waves, records that
 // every lane reads come from LDS, and scenes without light sampling have an
-// instance without it (173 instead of 213 VGPRs).  Measured against one lane
+// instance without it (173 instead of 215 VGPRs).  Measured against one lane
 // per sample that walks its glass tree and its light samples one after the
 // other, and against depth-synchronous batches: spheres 32x24 x 8 spp 834 ->
 // 175 us, 320x240 x 16 spp 1636 -> 951 us; mesh box 128x128 x 8 spp 2707 -> 926
