@@ -91,10 +91,10 @@ __device__ __forceinline__ int32_t scene_of_chunk(const Persist& st, uint32_t c)
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// SRC: PathSource.  NEE: some scene samples lights.  NL: LDS stack entries;
-// NTOP: BVH nodes kept in LDS; WAVES: waves per SIMD the registers are budgeted
-// for.
-template <int SRC, bool NEE, int NL, int NTOP, int WAVES>
+// SRC: PathSource.  NEE: some scene samples lights.  MANY: the analytic entities may
+// be more than a block keeps in LDS.  NL: LDS stack entries; NTOP: BVH nodes kept
+// in LDS; WAVES: waves per SIMD the registers are budgeted for.
+template <int SRC, bool NEE, bool MANY, int NL, int NTOP, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_path(Persist st,
                                                                                                  Params P1) {
   const Params& P0 = SRC == PATH_BATCH ? st.scenes[0] : P1;
@@ -116,6 +116,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   const DevMaterial* lds_mats = nullptr;
   if (kCache) {
     slots = load_analytic_slots(P1, s_ana);
+    if (!MANY) __builtin_assume(slots != nullptr);
     if (P1.n_materials <= PRT_PATH_MATERIALS) {
       if ((int)threadIdx.x < P1.n_materials) s_mats[threadIdx.x] = P1.mats[threadIdx.x];
       lds_mats = s_mats;
@@ -488,23 +489,28 @@ __global__ __launch_bounds__(256) void k_persist_resolve(Persist st, int64_t n_p
 // five BVH levels, so that the tree's top costs an LDS access instead of an L2
 // one, or for a batch of scenes, which shares no tree, 32 entries; at 3 waves 14
 // entries and four levels, or 20.
-template <int SRC, bool NEE, class F>
+// Frames without light sampling have an instance without the loop over more
+// analytic entities than the LDS copy holds: its scalars raised the three-wave
+// one's spills from 139 to 154 (spheres 320x240 x 16 spp 934 -> 955 us).
+template <int SRC, bool NEE, bool MANY, class F>
 static hipError_t with_path_waves(int waves, F&& f) {
   constexpr bool batch = SRC == PATH_BATCH;
   if constexpr (!NEE)
-    if (waves >= 3) return f(k_path<SRC, NEE, batch ? 20 : 14, batch ? PRT_TOP_NODES : 85, 3>);
-  return f(k_path<SRC, NEE, batch ? 32 : 12, batch ? PRT_TOP_NODES : PRT_WIDE_NODES, 2>);
+    if (waves >= 3) return f(k_path<SRC, NEE, MANY, batch ? 20 : 14, batch ? PRT_TOP_NODES : 85, 3>);
+  return f(k_path<SRC, NEE, MANY, batch ? 32 : 12, batch ? PRT_TOP_NODES : PRT_WIDE_NODES, 2>);
 }
 template <class F>
-static hipError_t with_path_kernel(PathSource src, bool nee, int waves, F&& f) {
-  if (src == PATH_BATCH) return nee ? with_path_waves<PATH_BATCH, true>(waves, f) : with_path_waves<PATH_BATCH, false>(waves, f);
-  if (src == PATH_FRAME) return nee ? with_path_waves<PATH_FRAME, true>(waves, f) : with_path_waves<PATH_FRAME, false>(waves, f);
-  if (src == PATH_CHAIN) return with_path_waves<PATH_CHAIN, true>(waves, f);
-  return with_path_waves<PATH_QUEUE, true>(waves, f);
+static hipError_t with_path_kernel(PathSource src, bool nee, bool many, int waves, F&& f) {
+  if (src == PATH_BATCH)
+    return nee ? with_path_waves<PATH_BATCH, true, true>(waves, f) : with_path_waves<PATH_BATCH, false, true>(waves, f);
+  if (src == PATH_CHAIN) return with_path_waves<PATH_CHAIN, true, true>(waves, f);
+  if (src == PATH_QUEUE) return with_path_waves<PATH_QUEUE, true, true>(waves, f);
+  if (nee) return with_path_waves<PATH_FRAME, true, true>(waves, f);
+  return many ? with_path_waves<PATH_FRAME, false, true>(waves, f) : with_path_waves<PATH_FRAME, false, false>(waves, f);
 }
 
 hipError_t launch_path(PathSource src, const Persist& p, const Params& P, int waves, int blocks, hipStream_t s) {
-  return with_path_kernel(src, p.nee != 0, waves, [&](void (*k)(Persist, Params)) {
+  return with_path_kernel(src, p.nee != 0, P.n_analytic > PRT_LDS_ANALYTIC, waves, [&](void (*k)(Persist, Params)) {
     hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, p, P);
     return hipGetLastError();
   });
