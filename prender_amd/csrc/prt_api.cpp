@@ -771,6 +771,17 @@ static int setup_render(prt_scene* s, const prt_render_opts* o, RenderSetup& R) 
 #ifndef PRT_PATH_SAMPLES_GLASS
 #define PRT_PATH_SAMPLES_GLASS (1 << 21)
 #endif
+// Every ray tests every analytic entity, in the path kernel two waves per SIMD
+// and at the lanes that have a ray then: with more entities than the LDS copy
+// holds it is the faster one for fewer samples, about as the number of the others.
+// Measured as above: spheres with glass, 40 entities, 0.61 M samples 2.69 / 3.19, 0.86 M
+// 3.65 / 3.87, 1.6 M 6.16 / 5.60; 100: 0.24 M 2.58 / 2.63, 0.38 M 3.10 / 2.98, 0.61 M 4.83
+// / 3.64; 400: 7 k 1.42 / 3.05, 55 k 4.04 / 3.20, 0.13 M 8.66 / 3.98; without glass, 100:
+// 0.13 M 1.46 / 1.57, 0.24 M 1.88 / 1.85, 0.38 M 2.77 / 2.16; 400: 55 k 1.98 / 2.88, 0.13 M
+// 5.43 / 3.18.
+#ifndef PRT_PATH_ENTITIES
+#define PRT_PATH_ENTITIES ((int64_t)1 << 25)
+#endif
 #ifndef PRT_PATH_TAIL
 #define PRT_PATH_TAIL (1 << 16)
 #endif
@@ -802,7 +813,11 @@ extern "C++" int prt::ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass)
   return dev_alloc(b, glass ? (size_t)g.n_waves() * PRT_PATH_POOL * sizeof(PoolRec) : 256);
 }
 
-static int64_t path_samples(const prt_scene* s) { return s->has_glass ? PRT_PATH_SAMPLES_GLASS : PRT_PATH_SAMPLES; }
+static int64_t path_samples(const prt_scene* s) {
+  const int64_t most = s->has_glass ? PRT_PATH_SAMPLES_GLASS : PRT_PATH_SAMPLES;
+  const int64_t more = s->P.n_analytic - PRT_LDS_ANALYTIC;
+  return more > 0 ? std::min(most, PRT_PATH_ENTITIES / more) : most;
+}
 
 // One batch's samples (src PATH_FRAME), or the rays of q[k] (PATH_QUEUE),
 // through the path kernel.
@@ -846,7 +861,7 @@ static int run_path(prt_scene* s, PathSource src, const Params& P, const Batch& 
 // when the proposal is complete: those scenes go step by step.
 // Measured (in step / own pace, ms): 15,360 chains 31.3 / 23.4, 65,536 64.3 / 53.9,
 // 180,000 142.5 / 131.5, 360,000 187.4 / 178.9.
-extern "C++" bool prt::chains_async(const prt_scene* s, uint32_t n) { return !s->has_glass && (int64_t)n <= path_samples(s); }
+extern "C++" bool prt::chains_async(const prt_scene* s, uint32_t n) { return !s->has_glass && n <= PRT_PATH_SAMPLES; }
 
 extern "C++" int prt::run_chains(prt_scene* s, const Params& P, const ChainRun& R, uint32_t n, uint32_t steps, Timer& tm,
                     CallTotals& tot) {

@@ -37,6 +37,8 @@ static_assert(PRT_MAX_LEAF >= 1 && PRT_MAX_LEAF <= 16, "leaf size must fit the 4
 // the path kernel keeps five levels (its two blocks per CU leave the LDS)
 #define PRT_WIDE_LEVELS 5
 #define PRT_WIDE_NODES 341  // 1 + 4 + 16 + 64 + 256
+// analytic entities of a scene that a block keeps in LDS; more are read one by one
+#define PRT_LDS_ANALYTIC 16
 // smallest LDS stack depth any kernel variant uses (sizes the overflow area)
 #define PRT_STACK_LDS_MIN 8
 #define PRT_STACK_TOTAL 128

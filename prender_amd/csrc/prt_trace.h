@@ -263,7 +263,6 @@ __device__ __forceinline__ int32_t hit_entity(const PRT_GLOBAL prt_f4* tris4, in
 
 // The analytic entities of a scene (at most PRT_LDS_ANALYTIC) as a block
 // keeps them in LDS, spheres first.
-#define PRT_LDS_ANALYTIC 16
 struct AnalyticSlot {
   double p0[3], radius;  // sphere; uvplane: p0
   double u_axis[3], v_axis[3], u_len, v_len, u_max, v_max;  // uvplane

@@ -203,3 +203,26 @@ ran = [k for k in launched() if "k_pathILi0E" in k]
 assert len(ran) == 1 and ran[0] == tried[-1] and ran[0].endswith("Li{waves}EEv7Persist6Params"), ran
 no_faults()
 """)
+
+
+# The more analytic entities there are beside a block's LDS copy, the smaller the
+# frames that the path kernel takes; the others go to the engine for their scene.
+@pytest.mark.parametrize("entities,glass,samples,path", [
+    (16, 1, 1 << 21, True), (17, 1, 1 << 21, True), (117, 1, 300000, True), (117, 1, 360000, False),
+    (1016, 1, 33000, True), (1016, 1, 34000, False), (16, 0, 3 << 17, True), (80, 0, 3 << 17, True),
+    (416, 0, 83000, True), (416, 0, 85000, False)])
+def test_path_frames_by_entities(host, entities, glass, samples, path):
+    host(f"""
+d = G.cornell_spheres(width={samples} // 8, height=8, samples=1, supersamples=1, nee=1)
+if not {glass}:
+    for m in d.materials:
+        m.reflection = "diffuse"
+while len(d.entities) < {entities}:
+    d.entities.append(G.Sphere((50.0, 40.0, 60.0 + 0.01 * len(d.entities)), 1.0, 2))
+prt.Scene(d).render(variance=False)
+names = launched()
+assert any("k_path" in k for k in names) == {path}, names
+assert any("k_stream" in k for k in names) == {bool(glass and not path)}
+assert any("k_extend" in k for k in names) == {not glass and not path}
+no_faults()
+""")
