@@ -199,8 +199,8 @@ typedef struct prt_render_opts {
     int32_t timing;            /* 1 = per-kernel device timing into prt_stats */
     int32_t image_f64;         /* 1 = out_rgb / out_var are double arrays (device entry points) */
     int32_t engine;            /* 0 = auto: scenes without next-event estimation and small
-                                  frames (up to 3 * 2^17 camera samples, 2^21 with glass)
-                                  render in one launch that follows each sample's whole
+                                  frames (up to 3 * 2^17 camera samples, 2^21 with glass,
+                                  fewer with many spheres and uvplanes) render in one launch that follows each sample's whole
                                   path, larger frames with glass stream through the
                                   batched renderer's tile queue, others run
                                   depth-synchronous batches; 1 = depth-synchronous

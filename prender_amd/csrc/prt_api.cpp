@@ -813,10 +813,10 @@ extern "C++" int prt::ensure_path_pool(DevBuf& b, const PathGrid& g, bool glass)
   return dev_alloc(b, glass ? (size_t)g.n_waves() * PRT_PATH_POOL * sizeof(PoolRec) : 256);
 }
 
+static int64_t path_samples_most(const prt_scene* s) { return s->has_glass ? PRT_PATH_SAMPLES_GLASS : PRT_PATH_SAMPLES; }
 static int64_t path_samples(const prt_scene* s) {
-  const int64_t most = s->has_glass ? PRT_PATH_SAMPLES_GLASS : PRT_PATH_SAMPLES;
   const int64_t more = s->P.n_analytic - PRT_LDS_ANALYTIC;
-  return more > 0 ? std::min(most, PRT_PATH_ENTITIES / more) : most;
+  return more > 0 ? std::min(path_samples_most(s), PRT_PATH_ENTITIES / more) : path_samples_most(s);
 }
 
 // One batch's samples (src PATH_FRAME), or the rays of q[k] (PATH_QUEUE),
@@ -1227,7 +1227,11 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
     return fail(PRT_E_INVALID, "the persistent engine writes float images of at most 2^28 samples, without "
                                "samples_override / batch_pixels");
   const int64_t frame = (int64_t)s->P.W * s->P.H * s->P.spp;
-  const bool path = engine == 3 || (engine == 0 && persist_ok && !dumping && (!nee_scene || frame <= path_samples(s)));
+  bool path = engine == 3 || (engine == 0 && persist_ok && !dumping && (!nee_scene || frame <= path_samples(s)));
+  // a frame that only its scene's entities keep from the path kernel takes it all
+  // the same where there is no memory for queues
+  const bool path_fits = engine == 0 && persist_ok && !dumping && frame <= path_samples_most(s);
+  int rc;
   if (engine == 2 || (engine == 0 && !path && s->has_glass && stream_ok && !dumping)) {
     prt_batch_opts b{};
     b.seed = o ? o->seed : 0;
@@ -1242,16 +1246,19 @@ static int render_device(prt_scene* s, const prt_render_opts* o, float* d_rgb, f
     prt_scene* const one[1] = {s};
     float* const rgb[1] = {d_rgb};
     float* const var[1] = {d_var};
-    return prt_render_batch_device(one, 1, &b, rgb, var, stats);
+    rc = prt_render_batch_device(one, 1, &b, rgb, var, stats);
+    if (rc != PRT_E_NOMEM || !path_fits) return rc;
+    path = true;
   }
   RenderSetup R;
-  int rc;
   if ((rc = setup_render(s, o, R))) return rc;
+  if (!path && (rc = ensure_workspace(s, R.bp * R.P.spp, false))) {
+    if (rc != PRT_E_NOMEM || !path_fits) return rc;
+    path = true;
+  }
   if (path) {
     R.bp = R.n_pix;  // one launch, which needs no queues
     if ((rc = ensure_path_workspace(s, R.n_pix * R.P.spp))) return rc;
-  } else if ((rc = ensure_workspace(s, R.bp * R.P.spp, false))) {
-    return rc;
   }
   hipStream_t st = s->stream;
   HIPCHK(launch_fill_u64((uint64_t*)s->pool->ws.ctr.p, 0ull, CTR_WORDS, st));

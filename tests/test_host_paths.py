@@ -226,3 +226,26 @@ assert any("k_stream" in k for k in names) == {bool(glass and not path)}
 assert any("k_extend" in k for k in names) == {not glass and not path}
 no_faults()
 """)
+
+
+# Without memory for queues those frames take the path kernel after all, as they did
+# before the limit depended on the entities; frames above its own limits fail.
+@pytest.mark.parametrize("glass,samples,ok", [(1, 1 << 20, True), (1, 3 << 20, False), (0, 3 << 17, True),
+                                              (0, 1 << 19, False)])
+def test_path_frames_without_memory_for_queues(host, glass, samples, ok):
+    host(f"""
+d = G.cornell_spheres(width={samples} // 8, height=8, samples=1, supersamples=1, nee=1)
+if not {glass}:
+    for m in d.materials:
+        m.reflection = "diffuse"
+while len(d.entities) < 1016:
+    d.entities.append(G.Sphere((50.0, 40.0, 60.0 + 0.01 * len(d.entities)), 1.0, 2))
+s = prt.Scene(d)
+host.hh_fail_above({80 if glass else 25} << 20)
+try:
+    s.render(variance=False)
+    assert {ok} and any("k_path" in k for k in launched())
+except prt.PrtError as e:
+    assert not {ok} and "(-3)" in str(e), e
+no_faults()
+""")
